@@ -1,5 +1,6 @@
 // C ABI of libchf: context life cycle, state exchange in the reference
 // layout, and the step sequence of the reference time loop (PF:220-532).
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -7,10 +8,12 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "chf_internal.h"
-#include "eig.h"
+#include "helmholtz.h"
 
 using namespace chf;
 
@@ -155,10 +158,11 @@ void free_all(Ctx* c) {
   f(c->costabf); f(c->twxf); f(c->twzf);
   for (auto& l : c->Lc) f(l);
   f(c->hvc); f(c->hgc);
-  f(c->rvT); f(c->roE); f(c->roO);
+  f(c->rvE); f(c->rvO); f(c->roE); f(c->roO);
   f(c->tsyn); f(c->tana); f(c->tpts); f(c->t0); f(c->t2); f(c->t4);
   f(c->inv); f(c->inv0); f(c->crep); f(c->bmat); f(c->bg0); f(c->bg1);
-  for (int i = 0; i < 2; ++i) { f(c->wL[i]); f(c->wR[i]); f(c->wlam[i]); }
+  for (int i = 0; i < 2; ++i) { f(c->hL[i]); f(c->hV[i]); f(c->hvec[i]); f(c->hwall[i]); }
+  f(c->tmean);
   f(c->phys_c); f(c->phys_r[0]); f(c->phys_r[1]); f(c->phys_r[2]); f(c->stats); f(c->twxu); f(c->twzu); f(c->twx); f(c->twz); f(c->twy); f(c->costab);
   f(c->gv); f(c->go); f(c->nonfinite);
   for (hipEvent_t e : c->event_pool) (void)hipEventDestroy(e);
@@ -169,110 +173,79 @@ void free_all(Ctx* c) {
   if (c->stream) (void)hipStreamDestroy(c->stream);
 }
 
-// Matrix-core A fragments of a rows x cols row-major matrix:
-// out[(rb * KB + kb) * 64 + lane] = A[16 rb + lane % 16][4 kb + lane / 16], zero outside.
-std::vector<double> pack_fragments(const std::vector<double>& a, int rows, int cols) {
-  const int MB = (rows + 15) / 16, KB = (cols + 3) / 4;
-  std::vector<double> out((size_t)MB * KB * 64, 0.0);
+// Matrix-core A fragments of an m x m row-major matrix, two k blocks of four
+// per entry: out[(rb * KP + kp) * 64 + lane] = A[16 rb + lane % 16][8 kp + lane / 16]
+// and the same four columns on, zero outside (KP = ceil(m / 8)).
+std::vector<double2> pack_pairs(const std::vector<double>& a, int m) {
+  const int MB = (m + 15) / 16, KP = (m + 7) / 8;
+  std::vector<double2> out((size_t)MB * KP * 64);
   for (int rb = 0; rb < MB; ++rb)
-    for (int kb = 0; kb < KB; ++kb)
+    for (int kp = 0; kp < KP; ++kp)
       for (int l = 0; l < 64; ++l) {
-        const int r = 16 * rb + l % 16, k = 4 * kb + l / 16;
-        if (r < rows && k < cols) out[((size_t)rb * KB + kb) * 64 + l] = a[(size_t)r * cols + k];
+        const int r = 16 * rb + l % 16, k = 8 * kp + l / 16;
+        auto at = [&](int kk) { return r < m && kk < m ? a[(size_t)r * m + kk] : 0.0; };
+        out[((size_t)rb * KP + kp) * 64 + l] = make_double2(at(k), at(k + 4));
       }
   return out;
 }
 
-// The omega_y half systems (get_coef_omegay, PF:3432-3455, folded by parity)
-// are [1^T ; c (sigma T0_I - T2_I)] x = [0 ; b] with c = dt/(2 re) and
-// sigma = 1/c + k^2: k^2 enters through sigma only.  On the null space of the
-// wall row, x = Q z with Q = [-1^T ; I], the interior rows read
-// c (sigma M0 - M2) z = b with M0 = T0_I Q, M2 = T2_I Q.  With
-// M0^-1 M2 = V diag(lam) V^-1 (lam: the Dirichlet second-derivative
-// eigenvalues, real and distinct),
-//     x = (Q V) diag(1 / (1 + c (k^2 - lam))) (V^-1 M0^-1) b,
-// so every mode shares two matrices and the per-mode work is a diagonal
-// scale.  The decomposition is accepted only if it reproduces direct solves
-// of the half system at k^2 = 0, 1 and the largest k^2 to 1e-12.
-int omega_diagonalise(Ctx* c, const std::vector<double>& t0, const std::vector<double>& t2,
-                      const std::vector<double>& al, const std::vector<double>& be) {
+// The decompositions of the half systems, which depend on the degree only: the
+// members of an ensemble that share one compute it once.
+using DegreeCache = std::map<int, std::array<la::HelmholtzHalf, 2>>;
+
+// Diagonalised v and omega_y operators (helmholtz.h), accepted only if they
+// reproduce direct solves of the half systems at k^2 = 0, the smallest and the
+// largest k^2 (the stored inverses are the fallback).
+int diagonalise(Ctx* c, const std::vector<double>& al, const std::vector<double>& be, DegreeCache& cache) {
   const Dims& d = c->d;
-  const int Ny = d.Ny;
   const double cc = c->prm.dt * 0.5 / c->prm.re;
-  double smax = 0.0;
+  double smin = 0.0, smax = 0.0;
   for (double a : al)
-    for (double b : be) smax = std::max(smax, a * a + b * b);
-  std::vector<double> Lh[2], Rh[2], lam[2];
-  for (int par = 0; par < 2; ++par) {
-    const int n = par ? d.no : d.ne, m = n - 1;
-    if (m < 1) return 0;
-    la::Mat M0((size_t)m * m), M2((size_t)m * m);
-    for (int r = 0; r < m; ++r) {
-      const int p = r + 1;  // interior point of row r
-      for (int k = 0; k < m; ++k) {
-        const int l0 = par, lk = 2 * (k + 1) + par;  // Q column k: -1 at x_0, +1 at x_{k+1}
-        M0[(size_t)r * m + k] = t0[(size_t)p * Ny + lk] - t0[(size_t)p * Ny + l0];
-        M2[(size_t)r * m + k] = t2[(size_t)p * Ny + lk] - t2[(size_t)p * Ny + l0];
-      }
+    for (double b : be) {
+      const double s = a * a + b * b;
+      smax = std::max(smax, s);
+      if (s > 0.0 && (smin == 0.0 || s < smin)) smin = s;
     }
-    la::Mat M0i, V, Vi;
-    if (!la::inverse(M0, m, M0i)) return 0;
-    const la::Mat G = la::matmul(M0i, M2, m, m, m);
-    std::vector<double> ev;
-    if (!la::eig_real(G, m, ev, V)) return 0;
-    if (!la::inverse(V, m, Vi)) return 0;
-    la::Mat L = la::matmul(Vi, M0i, m, m, m);
-    la::Mat R((size_t)n * m);
-    for (int k = 0; k < m; ++k) {
-      double s = 0.0;
-      for (int r = 0; r < m; ++r) s += V[(size_t)r * m + k];
-      R[k] = -s;
-      for (int r = 0; r < m; ++r) R[(size_t)(r + 1) * m + k] = V[(size_t)r * m + k];
+  const bool known = cache.count(d.N) != 0;
+  std::array<la::HelmholtzHalf, 2>& h = cache[d.N];
+  bool ok[2] = {false, false};
+  auto half = [&](int par) {
+    try {
+      ok[par] = known ? h[par].m > 0 : la::helmholtz_half(d.N, par, h[par]);
+      for (double s : {0.0, smin, smax}) ok[par] = ok[par] && la::helmholtz_verify(par, h[par], cc, s);
+    } catch (...) {
+      ok[par] = false;
     }
-    // verification against direct solves of the half system
-    for (double s : {0.0, 1.0, smax}) {
-      la::Mat A((size_t)n * n);
-      for (int j = 0; j < n; ++j) A[j] = 1.0;
-      for (int i = 1; i < n; ++i)
-        for (int j = 0; j < n; ++j) {
-          const size_t o = (size_t)i * Ny + 2 * j + par;
-          A[(size_t)i * n + j] = -cc * t2[o] + (1.0 + cc * s) * t0[o];
-        }
-      std::vector<double> b(m), x(n, 0.0), y(m, 0.0);
-      for (int r = 0; r < m; ++r) b[r] = std::sin(1.7 * r + 0.3) + 0.1 * r / m;
-      la::Mat rhs(n, 0.0);
-      for (int r = 0; r < m; ++r) rhs[r + 1] = b[r];
-      std::vector<int> piv;
-      if (!la::lu(A, piv, n)) return 0;
-      la::lu_solve(A, piv, n, rhs, 1);
-      for (int j = 0; j < m; ++j) {
-        double t = 0.0;
-        for (int r = 0; r < m; ++r) t += L[(size_t)j * m + r] * b[r];
-        y[j] = t / (1.0 + cc * (s - ev[j]));
-      }
-      double err = 0.0, ref = 0.0;
-      for (int i = 0; i < n; ++i) {
-        double t = 0.0;
-        for (int j = 0; j < m; ++j) t += R[(size_t)i * m + j] * y[j];
-        err = std::max(err, std::fabs(t - rhs[i]));
-        ref = std::max(ref, std::fabs(rhs[i]));
-      }
-      if (!(err <= 1e-12 * ref)) return 0;
-    }
-    Lh[par] = pack_fragments(L, m, m);
-    Rh[par] = pack_fragments(R, n, m);
-    lam[par] = ev;
-    lam[par].resize((size_t)((m + 15) / 16) * 16, 0.0);
+  };
+  std::thread other;
+  try {
+    other = std::thread(half, 1);
+  } catch (const std::system_error&) {
+    half(1);
   }
+  half(0);
+  if (other.joinable()) other.join();
+  if (!ok[0] || !ok[1]) return 0;
   for (int par = 0; par < 2; ++par) {
-    CHF_TRY(dalloc(c, &c->wL[par], Lh[par].size()));
-    CHF_TRY(dalloc(c, &c->wR[par], Rh[par].size()));
-    CHF_TRY(dalloc(c, &c->wlam[par], lam[par].size()));
-    CHF_TRY(hipMemcpy(c->wL[par], Lh[par].data(), Lh[par].size() * sizeof(double), hipMemcpyHostToDevice));
-    CHF_TRY(hipMemcpy(c->wR[par], Rh[par].data(), Rh[par].size() * sizeof(double), hipMemcpyHostToDevice));
-    CHF_TRY(hipMemcpy(c->wlam[par], lam[par].data(), lam[par].size() * sizeof(double), hipMemcpyHostToDevice));
+    const int m = h[par].m, R = 16 * ((m + 15) / 16);
+    const std::vector<double2> L = pack_pairs(h[par].L, m), V = pack_pairs(h[par].V, m);
+    std::vector<double> vec(5 * (size_t)R, 0.0);
+    for (int j = 0; j < R; ++j) vec[j] = j < m ? h[par].lam[j] : -1.0;  // padding rows: any finite scale of zero
+    for (int j = 0; j < m; ++j) {
+      vec[(size_t)R + j] = h[par].w1[j];
+      vec[2 * (size_t)R + j] = h[par].w2[j];
+      vec[3 * (size_t)R + j] = h[par].l1[j];
+      vec[4 * (size_t)R + j] = h[par].q[j];
+    }
+    CHF_TRY(dalloc(c, &c->hL[par], L.size()));
+    CHF_TRY(dalloc(c, &c->hV[par], V.size()));
+    CHF_TRY(dalloc(c, &c->hvec[par], vec.size()));
+    CHF_TRY(dalloc(c, &c->hwall[par], 4 * (size_t)d.ncol));
+    CHF_TRY(hipMemcpy(c->hL[par], L.data(), L.size() * sizeof(double2), hipMemcpyHostToDevice));
+    CHF_TRY(hipMemcpy(c->hV[par], V.data(), V.size() * sizeof(double2), hipMemcpyHostToDevice));
+    CHF_TRY(hipMemcpy(c->hvec[par], vec.data(), vec.size() * sizeof(double), hipMemcpyHostToDevice));
   }
-  c->wdiag = true;
+  c->diag = true;
   return 0;
 }
 
@@ -350,7 +323,7 @@ int autotune(Ctx* c) {
   return 0;
 }
 
-int build(Ctx* c) {
+int build(Ctx* c, DegreeCache& cache) {
   Dims& d = c->d;
   const chf_params& p = c->prm;
   d.Mx = p.nnx / 2;
@@ -388,7 +361,6 @@ int build(Ctx* c) {
   CHF_TRY(dalloc(c, &c->alpha, d.Mx));
   CHF_TRY(dalloc(c, &c->beta, d.Mz));
   CHF_TRY(dalloc(c, &c->v, fld));
-  CHF_TRY(dalloc(c, &c->vst, (size_t)d.ngroups * d.Ny * 2));
   CHF_TRY(dalloc(c, &c->oy, fld));
   CHF_TRY(dalloc(c, &c->u, fld));
   CHF_TRY(dalloc(c, &c->w, fld));
@@ -414,9 +386,7 @@ int build(Ctx* c) {
   for (auto& l : c->Lc) CHF_TRY(dalloc(c, &l, fld));
   CHF_TRY(dalloc(c, &c->hvc, fld));
   CHF_TRY(dalloc(c, &c->hgc, fld));
-  CHF_TRY(dalloc(c, &c->rvT, (size_t)(d.ne + d.no - 4) * d.ncol));
-  CHF_TRY(dalloc(c, &c->roE, (size_t)d.ne * d.ncol));
-  CHF_TRY(dalloc(c, &c->roO, (size_t)d.ne * d.ncol));
+  for (double2** q : {&c->rvE, &c->rvO, &c->roE, &c->roO}) CHF_TRY(dalloc(c, q, (size_t)d.ne * d.ncol));
   CHF_TRY(dalloc(c, &c->gv, fld));
   CHF_TRY(dalloc(c, &c->go, fld));
   CHF_TRY(dalloc(c, &c->nonfinite, 1));
@@ -428,11 +398,48 @@ int build(Ctx* c) {
   CHF_TRY(hipMemcpy(c->alpha, al.data(), d.Mx * sizeof(double), hipMemcpyHostToDevice));
   CHF_TRY(hipMemcpy(c->beta, be.data(), d.Mz * sizeof(double), hipMemcpyHostToDevice));
 
-  // operator classes: the collocation operators depend on k^2 only, so groups
-  // whose k^2 (computed as the set-up and solve kernels compute it) is bitwise
-  // equal share one set of inverses; solve blocks take up to two groups of a
-  // class, in order of their first group
-  {
+  // SCHEB operator matrices
+  std::vector<double> t0, t1, t2, t4;
+  scheb(d.N, t0, t1, t2, t4);
+  const size_t tt = (size_t)d.Ny * d.Ny;
+  CHF_TRY(dalloc(c, &c->t0, tt));
+  CHF_TRY(dalloc(c, &c->t2, tt));
+  CHF_TRY(dalloc(c, &c->t4, tt));
+  CHF_TRY(hipMemcpy(c->t0, t0.data(), tt * sizeof(double), hipMemcpyHostToDevice));
+  CHF_TRY(hipMemcpy(c->t2, t2.data(), tt * sizeof(double), hipMemcpyHostToDevice));
+  CHF_TRY(hipMemcpy(c->t4, t4.data(), tt * sizeof(double), hipMemcpyHostToDevice));
+
+  // operators: diagonalised when the decomposition verifies, else their
+  // half-system inverses are stored.  CHF_OMEGA_INVERSES=stored in the
+  // environment selects the stored inverses without trying.
+  const char* force = std::getenv("CHF_OMEGA_INVERSES");
+  if (!(force && std::strcmp(force, "stored") == 0)) {
+    const int rc = diagonalise(c, al, be, cache);
+    if (rc) return rc;
+  }
+  const long neP = d.ne + (d.ne & 1), noP = d.no + (d.no & 1);
+  if (c->diag) {
+    // class 0 is the mean mode's k^2 = 0 operator, the only stored inverse
+    d.nclass = 1;
+    d.inv_row = neP + noP;
+    CHF_TRY(dalloc(c, &c->crep, 1));
+    CHF_TRY(hipMemset(c->crep, 0, sizeof(int)));
+    CHF_TRY(dalloc(c, &c->inv0, (size_t)d.ne * (neP + noP)));
+    c->inv_w = c->inv0;
+    c->row_w = neP + noP;
+    const double cc = p.dt * 0.5 / p.re;
+    std::vector<double> tm(tt);
+    for (int j = 0; j < d.Ny; ++j)
+      for (int l = 0; l < d.Ny; ++l)
+        tm[(size_t)l * d.Ny + j] = t0[(size_t)j * d.Ny + l] + cc * t2[(size_t)j * d.Ny + l];
+    CHF_TRY(dalloc(c, &c->tmean, tt));
+    CHF_TRY(hipMemcpy(c->tmean, tm.data(), tt * sizeof(double), hipMemcpyHostToDevice));
+    CHF_TRY(launch_wall_setup(*c));
+  } else {
+    // operator classes: the collocation operators depend on k^2 only, so groups
+    // whose k^2 (computed as the set-up and solve kernels compute it) is bitwise
+    // equal share one set of inverses; solve blocks take up to two groups of a
+    // class, in order of their first group
     std::map<double, int> cls_of;
     std::vector<std::vector<int>> members;
     for (int g = 0; g < d.ngroups; ++g) {
@@ -465,44 +472,14 @@ int build(Ctx* c) {
     CHF_TRY(hipMemcpy(c->bmat, bmat.data(), bmat.size() * sizeof(int), hipMemcpyHostToDevice));
     CHF_TRY(hipMemcpy(c->bg0, bg0.data(), bg0.size() * sizeof(int), hipMemcpyHostToDevice));
     CHF_TRY(hipMemcpy(c->bg1, bg1.data(), bg1.size() * sizeof(int), hipMemcpyHostToDevice));
-  }
-
-  // SCHEB operator matrices
-  std::vector<double> t0, t1, t2, t4;
-  scheb(d.N, t0, t1, t2, t4);
-  const size_t tt = (size_t)d.Ny * d.Ny;
-  CHF_TRY(dalloc(c, &c->t0, tt));
-  CHF_TRY(dalloc(c, &c->t2, tt));
-  CHF_TRY(dalloc(c, &c->t4, tt));
-  CHF_TRY(hipMemcpy(c->t0, t0.data(), tt * sizeof(double), hipMemcpyHostToDevice));
-  CHF_TRY(hipMemcpy(c->t2, t2.data(), tt * sizeof(double), hipMemcpyHostToDevice));
-  CHF_TRY(hipMemcpy(c->t4, t4.data(), tt * sizeof(double), hipMemcpyHostToDevice));
-
-  // omega_y operator: diagonalised when the decomposition verifies, else its
-  // half-system inverses are stored next to the v ones.  CHF_OMEGA_INVERSES=stored
-  // in the environment selects the stored inverses without trying.
-  {
-    const char* force = std::getenv("CHF_OMEGA_INVERSES");
-    const bool stored = force && std::strcmp(force, "stored") == 0;
-    const int rc = stored ? 0 : omega_diagonalise(c, t0, t2, al, be);
-    if (rc) return rc;
-    const long neP = d.ne + (d.ne & 1), noP = d.no + (d.no & 1);
-    if (c->wdiag) {
-      d.inv_row = neP + noP;
-      d.inv_stride = (long)d.ne * d.inv_row;
-      CHF_TRY(dalloc(c, &c->inv, (size_t)d.nclass * d.inv_stride));
-      CHF_TRY(dalloc(c, &c->inv0, (size_t)d.ne * (neP + noP)));
-      c->inv_w = c->inv0;
-      c->stride_w = 0;
-      c->row_w = neP + noP;
-    } else {
-      d.inv_row = 2 * (neP + noP);
-      d.inv_stride = (long)d.ne * d.inv_row;
-      CHF_TRY(dalloc(c, &c->inv, (size_t)d.nclass * d.inv_stride));
-      c->inv_w = c->inv + (neP + noP);
-      c->stride_w = d.inv_stride;
-      c->row_w = d.inv_row;
-    }
+    d.inv_row = 2 * (neP + noP);
+    d.inv_stride = (long)d.ne * d.inv_row;
+    CHF_TRY(dalloc(c, &c->inv, (size_t)d.nclass * d.inv_stride));
+    c->inv_w = c->inv + (neP + noP);
+    c->stride_w = d.inv_stride;
+    c->row_w = d.inv_row;
+    CHF_TRY(dalloc(c, &c->vst, (size_t)d.ngroups * d.Ny * 2));
+    CHF_TRY(hipMemsetAsync(c->vst, 0, (size_t)d.ngroups * d.Ny * 2 * sizeof(double2), c->stream));
   }
 
   // transform matrices: synthesis on the 2N+1 grid (folded rows p = 0..N),
@@ -604,7 +581,6 @@ int build(Ctx* c) {
     CHF_TRY(hipMemsetAsync(q, 0, fld * sizeof(double2), c->stream));
   for (double2* q : {c->cl1[0], c->cl1[1], c->cl3[0], c->cl3[1], c->au0, c->w0})
     CHF_TRY(hipMemsetAsync(q, 0, d.Ny * sizeof(double2), c->stream));
-  CHF_TRY(hipMemsetAsync(c->vst, 0, (size_t)d.ngroups * d.Ny * 2 * sizeof(double2), c->stream));
   CHF_TRY(hipMemsetAsync(c->nonfinite, 0, sizeof(int), c->stream));
 
   // kernels that stage more than 64 KiB of LDS
@@ -763,57 +739,30 @@ int nonlinear(Ctx* c, bool defer = true) {
   return 0;
 }
 
-int solve(Ctx* c) {
-  if (c->wdiag && !c->timing && c->overlap) {
-    // the omega_y path (right-hand side, diagonalised solve) does not touch
-    // the v path's data until the kinematics: it runs on the side stream,
-    // the matrix-core-bound omega_y solve beside the HBM-bound v solve.
-    // (With timing on, every launch runs alone so that each time is its own.)
-    CHF_TRY(hipEventRecord(c->ev_fork, c->stream));
-    CHF_TRY(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-    hipStream_t main = c->stream;
-    c->stream = c->side;  // the launchers and timing marks use c->stream
-    hipError_t e = timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1); });
-    if (e == hipSuccess) e = timed(c, K_WSOLVE, [&] { return launch_wsolve(*c); });
-    if (e == hipSuccess) e = hipEventRecord(c->ev_join, c->side);
-    c->stream = main;
-    CHF_TRY(e);
-    CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0); }));
-    c->hdefer = false;  // both right-hand-side kernels have formed h^n's point values
-    CHF_TRY(timed(c, K_SOLVE, [&] { return launch_solve(*c); }));
-    CHF_TRY(hipStreamWaitEvent(c->stream, c->ev_join, 0));
-  } else {
+// f32: the kinematics writes u, w, omega_x, omega_z in FP32 only, as the next
+// nonlinear pass of the mixed form with the FFT transforms reads them
+int solve(Ctx* c, bool f32) {
+  if (!c->diag) {
     CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0); }));
     CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1); }));
-    c->hdefer = false;
     CHF_TRY(timed(c, K_SOLVE, [&] { return launch_solve(*c); }));
-    if (c->wdiag) CHF_TRY(timed(c, K_WSOLVE, [&] { return launch_wsolve(*c); }));
+  } else if (!c->timing && c->overlap) {
+    // the omega_y path (right-hand side, solve) does not touch the v path's
+    // data until the kinematics: it runs on the side stream.  (With timing on,
+    // every launch runs alone so that each time is its own.)
+    CHF_TRY(on_two_streams(
+        c, [&] { const hipError_t e = launch_rhs(*c, 0); return e ? e : launch_hsolve(*c, 0); },
+        [&] { const hipError_t e = launch_rhs(*c, 1); return e ? e : launch_hsolve(*c, 1); }));
+  } else {
+    CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0); }));
+    CHF_TRY(timed(c, K_SOLVE, [&] { return launch_hsolve(*c, 0); }));
+    CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1); }));
+    CHF_TRY(timed(c, K_WSOLVE, [&] { return launch_hsolve(*c, 1); }));
   }
-  // the mixed form with the FFT transforms keeps u, w, omega_x, omega_z in
-  // FP32 only, as the next nonlinear pass reads them
-  CHF_TRY(timed(c, K_KINEMATICS, [&] { return launch_kinematics(*c, c->f32_fields); }));
-  c->f32_current = c->f32_fields;
-  c->f64_stale = c->f32_fields;
-  return 0;
-}
-
-// solve() split around k_solve, for an ensemble, whose members' k_solve blocks
-// run as one launch: the right-hand sides and the diagonalised omega_y solve
-// before it (the omega_y path shares no data with k_solve), v's transpose and
-// the kinematics after it.  Each kernel computes what it computes in solve().
-int solve_before(Ctx* c) {
-  CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0); }));
-  CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1); }));
-  c->hdefer = false;
-  if (c->wdiag) CHF_TRY(timed(c, K_WSOLVE, [&] { return launch_wsolve(*c); }));
-  return 0;
-}
-
-int solve_after(Ctx* c) {
-  CHF_TRY(launch_vtranspose(*c));
-  CHF_TRY(timed(c, K_KINEMATICS, [&] { return launch_kinematics(*c); }));
-  c->f32_current = false;
-  c->f64_stale = false;
+  c->hdefer = false;  // both right-hand-side kernels have formed h^n's point values
+  CHF_TRY(timed(c, K_KINEMATICS, [&] { return launch_kinematics(*c, f32); }));
+  c->f32_current = f32;
+  c->f64_stale = f32;
   return 0;
 }
 
@@ -865,7 +814,8 @@ int chf_create(const chf_params* prm, void** out) {
   }
   Ctx* c = new Ctx();
   c->prm = *prm;
-  int rc = build(c);
+  DegreeCache cache;
+  int rc = build(c, cache);
   if (rc) {
     g_create_err = c->err;
     free_all(c);
@@ -966,7 +916,7 @@ int chf_nonlinear(void* ctx) {
 int chf_solve(void* ctx) {
   if (!ctx) return -1;
   Ctx* c = static_cast<Ctx*>(ctx);
-  const int rc = solve(c);
+  const int rc = solve(c, c->f32_fields);
   return rc ? rc : check_finite(c, "chf_solve");
 }
 
@@ -975,7 +925,7 @@ int chf_step(void* ctx, int n) {
   Ctx* c = static_cast<Ctx*>(ctx);
   if (n < 0) return fail(c, "chf_step: negative step count");
   for (int i = 0; i < n; ++i) {
-    int rc = solve(c);
+    int rc = solve(c, c->f32_fields);
     if (rc) return rc;
     rc = nonlinear(c);
     if (rc) return rc;
@@ -1156,29 +1106,24 @@ int chf_timing(void* ctx, int id, double* total_ms, int* launches) {
 // ------------------------------------------------------------------ ensemble
 //
 // Independent channels of any mix of sizes, Reynolds numbers and precisions
-// advanced together.  One step of all members is one hipGraph launch of three
-// stages: every member's right-hand sides and omega_y solve as parallel
-// branches (each member on its own stream, forked from and joined to the
-// ensemble stream); one k_solve_members launch that streams every member's
-// half-system inverses (PF:242-394 over all members); then every member's
-// kinematics and nonlinear terms as parallel branches again.  Small members
-// fill the GPU together.  The AB2 history buffers swap every step, so a graph
-// (with the solve arguments it names) is captured per combination of the
-// members' history phases (normally two) and cached.
+// advanced together.  One step of all members is one hipGraph launch whose
+// parallel branches are the members' steps (each member on its own stream,
+// forked from and joined to the ensemble stream).  Small members fill the GPU
+// together.  The AB2 history buffers swap every step, so a graph is captured per
+// combination of the members' history phases (normally two) and cached.
 
 namespace {
 
 struct EnsGraph {
   std::vector<int> phase;         // members' history phases the graph was captured at
   hipGraphExec_t exec = nullptr;
-  void* solve_args = nullptr;     // device: the members' k_solve arguments for that phase
 };
 
 struct Ens {
   std::vector<Ctx*> m;
   hipStream_t origin = nullptr;
-  hipEvent_t fork = nullptr, mid = nullptr;
-  std::vector<hipEvent_t> ready, join;
+  hipEvent_t fork = nullptr;
+  std::vector<hipEvent_t> join;
   std::vector<EnsGraph> graphs;
   std::string err;
 };
@@ -1195,10 +1140,8 @@ int ens_fail(Ens* e, const std::string& msg, int rc = -1) {
   } while (0)
 
 void ens_free(Ens* e) {
-  for (auto& g : e->graphs) {
+  for (auto& g : e->graphs)
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
-    if (g.solve_args) (void)hipFree(g.solve_args);
-  }
   e->graphs.clear();
   for (Ctx* c : e->m) {
     if (!c) continue;
@@ -1209,21 +1152,15 @@ void ens_free(Ens* e) {
   e->m.clear();
   for (hipEvent_t ev : e->join) (void)hipEventDestroy(ev);
   e->join.clear();
-  for (hipEvent_t ev : e->ready) (void)hipEventDestroy(ev);
-  e->ready.clear();
-  if (e->mid) (void)hipEventDestroy(e->mid);
   if (e->fork) (void)hipEventDestroy(e->fork);
   if (e->origin) (void)hipStreamDestroy(e->origin);
 }
 
-// Captures one step of every member into g (solve arguments written first,
-// outside the capture); member host state (history phase) is restored
-// afterwards, the caller advances it per launch.
+// Captures one step of every member into g; member host state (history phase)
+// is restored afterwards, the caller advances it per launch.
 int ens_capture(Ens* e, EnsGraph* g) {
   const int n = (int)e->m.size();
   for (Ctx* c : e->m) g->phase.push_back(c->hcur);
-  ENS_TRY(hipMalloc(&g->solve_args, solve_members_bytes(n)));
-  ENS_TRY(write_solve_members(e->m.data(), n, g->solve_args));
   ENS_TRY(hipStreamBeginCapture(e->origin, hipStreamCaptureModeRelaxed));
   int rc = 0;
   std::string what;
@@ -1232,21 +1169,7 @@ int ens_capture(Ens* e, EnsGraph* g) {
     Ctx* c = e->m[i];
     he = hipStreamWaitEvent(c->stream, e->fork, 0);
     if (he != hipSuccess) break;
-    rc = solve_before(c);
-    if (rc) {
-      what = c->err;
-      break;
-    }
-    he = hipEventRecord(e->ready[i], c->stream);
-    if (he == hipSuccess) he = hipStreamWaitEvent(e->origin, e->ready[i], 0);
-  }
-  if (he == hipSuccess && rc == 0) he = launch_solve_members(e->origin, e->m.data(), n, g->solve_args);
-  if (he == hipSuccess && rc == 0) he = hipEventRecord(e->mid, e->origin);
-  for (int i = 0; i < n && he == hipSuccess && rc == 0; ++i) {
-    Ctx* c = e->m[i];
-    he = hipStreamWaitEvent(c->stream, e->mid, 0);
-    if (he != hipSuccess) break;
-    rc = solve_after(c);
+    rc = solve(c, false);
     if (rc == 0) rc = nonlinear(c, false);
     if (rc) {
       what = c->err;
@@ -1294,11 +1217,12 @@ int chf_ensemble_create(const chf_params* members, int n, void** out) {
     }
   }
   Ens* e = new Ens();
+  DegreeCache cache;
   for (int i = 0; i < n; ++i) {
     Ctx* c = new Ctx();
     c->prm = members[i];
     c->overlap = false;
-    const int rc = build(c);
+    const int rc = build(c, cache);
     if (rc) {
       g_create_err = "member " + std::to_string(i) + ": " + c->err;
       free_all(c);
@@ -1311,10 +1235,7 @@ int chf_ensemble_create(const chf_params* members, int n, void** out) {
   }
   hipError_t he = hipStreamCreateWithFlags(&e->origin, hipStreamNonBlocking);
   if (he == hipSuccess) he = hipEventCreateWithFlags(&e->fork, hipEventDisableTiming);
-  if (he == hipSuccess) he = hipEventCreateWithFlags(&e->mid, hipEventDisableTiming);
-  e->ready.assign(n, nullptr);
   e->join.assign(n, nullptr);
-  for (int i = 0; i < n && he == hipSuccess; ++i) he = hipEventCreateWithFlags(&e->ready[i], hipEventDisableTiming);
   for (int i = 0; i < n && he == hipSuccess; ++i) he = hipEventCreateWithFlags(&e->join[i], hipEventDisableTiming);
   if (he != hipSuccess) {
     g_create_err = std::string("ensemble streams/events: ") + hipGetErrorString(he);
@@ -1375,7 +1296,6 @@ int chf_ensemble_step(void* ens, int n) {
       const int rc = ens_capture(e, &g);
       if (rc) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
-        if (g.solve_args) (void)hipFree(g.solve_args);
         return rc;
       }
       exec = g.exec;

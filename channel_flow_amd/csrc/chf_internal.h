@@ -39,8 +39,8 @@ struct Dims {
   int Pn;     // N+1-point grid folded by parity: N/2+1
   long ncol;  // complex columns per plane: Mz*Mx
   int ngroups;  // (kx,|kz|) groups: Mx*(Mz/2)
-  int nclass;   // operator classes (groups with bitwise-equal k^2 share an inverse)
-  int nblocks;  // solve blocks: up to two groups of one class each
+  int nclass;   // stored inverses: operator classes (groups with bitwise-equal k^2 share one); else 1
+  int nblocks;  // stored inverses: solve blocks, up to two groups of one class each
   long inv_row;     // doubles per inverse row j: 2 (neP + noP), the four half systems side by side
   long inv_stride;  // doubles per group: ne * inv_row
 };
@@ -86,7 +86,7 @@ struct Ctx {
   Dims d{};
   int device = 0;
   hipStream_t stream = nullptr;
-  // second stream of the context (default priority): with the omega_y operator
+  // second stream of the context (default priority): with the operators
   // diagonalised, the omega_y right-hand side and solve run on it while the v
   // path runs on `stream`; the pair of events forks and joins it
   hipStream_t side = nullptr;
@@ -99,7 +99,7 @@ struct Ctx {
   double* beta = nullptr;   // [Mz]
   // state (complex, [Ny][Mz][Mx] unless noted)
   double2 *v = nullptr, *oy = nullptr;              // coefficients
-  double2* vst = nullptr;  // v as the solve writes it: per (kx, |kz|) group, [Ny][2 sides]
+  double2* vst = nullptr;  // stored inverses: v as k_solve writes it, per (kx, |kz|) group, [Ny][2 sides]
   double2 *u = nullptr, *w = nullptr, *ox = nullptr, *oz = nullptr;  // derived
   // Mixed form with the FFT transforms: u, w, omega_x, omega_z also in FP32,
   // the values the padded synthesis rounds them to on load.  The per-step
@@ -128,11 +128,8 @@ struct Ctx {
   double2* Lc[3] = {};    // [Ny][Mz][Mx]   Lamb vector coefficients
   double2 *hvc = nullptr, *hgc = nullptr;  // h coefficients
   // solve work
-  // v right-hand sides per mode: [column][even rows (ne - 2), then odd rows
-  // (no - 2)], so a solve block reads each of its modes' rows contiguously;
-  // omega_y right-hand sides per parity: [row][column] (the omega_y solve
-  // reads 64 neighbouring columns at a time)
-  double2* rvT = nullptr;
+  // parity-folded right-hand sides, [row][column]
+  double2 *rvE = nullptr, *rvO = nullptr;
   double2 *roE = nullptr, *roO = nullptr;
   double2 *gv = nullptr, *go = nullptr;  // explicit-operator coefficient vectors
   // gv/go are written by the kinematics pass for the next solve (it runs after
@@ -154,20 +151,21 @@ struct Ctx {
   // so a solve block reads one contiguous row per step.  Group 0: mean mode
   // (omega_y-type operator at k^2 = 0), its v halves are zero.
   double* inv = nullptr;
-  // omega_y half systems: either their inverses sit beside the v ones in `inv`
-  // (inv_w = inv + neP + noP, same strides), or the operator is diagonalised
-  // (wdiag) and only the mean group's k^2 = 0 inverse is stored, in inv0.
-  bool wdiag = false;
+  // diag: the operators are diagonalised (helmholtz.h) and only the mean
+  // group's k^2 = 0 inverse is stored, in inv0; otherwise the omega_y inverses
+  // sit beside the v ones in `inv` (inv_w = inv + neP + noP, same strides)
+  bool diag = false;
   int* crep = nullptr;                               // [nclass] first group of each class
   int *bmat = nullptr, *bg0 = nullptr, *bg1 = nullptr;  // [nblocks] class, groups (-1: none)
   double* inv0 = nullptr;
   const double* inv_w = nullptr;
   long stride_w = 0, row_w = 0;
-  // diagonalised omega_y solve, per parity: packed matrix-core A fragments of
-  // L = V^-1 M0^-1 ((n-1) x (n-1)) and R = Q V (n x (n-1)), eigenvalues lam
-  double* wL[2] = {nullptr, nullptr};
-  double* wR[2] = {nullptr, nullptr};
-  double* wlam[2] = {nullptr, nullptr};
+  // diagonalised solves, per parity: packed matrix-core A fragments of L and V
+  // (m x m, m = n - 1), the vectors lam, w1, w2, l1, q ([16 MB] each, MB 16-row
+  // blocks) and the wall matrix of every column (4 values)
+  double2 *hL[2] = {nullptr, nullptr}, *hV[2] = {nullptr, nullptr};
+  double *hvec[2] = {nullptr, nullptr}, *hwall[2] = {nullptr, nullptr};
+  double* tmean = nullptr;  // [l][p]: T0 + c T2 transposed (mean mode)
   double2* twx = nullptr;  // exp(-2 pi i m/Lx), m < Lx
   double2* twz = nullptr;  // exp(-2 pi i m/Lz), m < Lz
   // FFT forms of the wall-normal transforms (null when 2N has no split or
@@ -236,7 +234,7 @@ hipError_t launch_yanalysis(Ctx& c, const double2* const* in, double2* const* ou
 // which: 0 = v, 1 = omega_y; hc != nullptr: h^n from its coefficients hc, its
 // point values written to hn; else hn holds them
 hipError_t launch_yrhs(Ctx& c, int which, const double2* g, const double2* hc, double2* hn, const double2* hp,
-                       double2* oE, double2* oO, double2* oT);
+                       double2* oE, double2* oO);
 hipError_t launch_ysynth32(Ctx& c, const double2* const* in, float2* const* out, int nf);
 hipError_t launch_ysynth32f(Ctx& c, const float2* const* in, float2* const* out, int nf);  // FP32 coefficients in
 hipError_t launch_yanalysis32f(Ctx& c, const float2* const* in, float2* const* out, int nf);  // FP32 coefficients out
@@ -248,15 +246,11 @@ hipError_t launch_stream_c2r_unpadded(Ctx& c, const double2* in, double* out);
 hipError_t launch_physical(Ctx& c, const double2* field, double2* work, double* out);
 hipError_t launch_plane_stats(Ctx& c, const double* u, const double* v, const double* w, double* out);
 hipError_t launch_rhs(Ctx& c, int which);  // 0 = v, 1 = omega_y
-hipError_t launch_solve(Ctx& c);       // v, omega_y and the mean mode (k_solve, then launch_vtranspose)
+hipError_t launch_solve(Ctx& c);       // stored inverses: v, omega_y and the mean mode (k_solve, then launch_vtranspose)
 hipError_t launch_vtranspose(Ctx& c);  // v from the solve's per-group records to [Ny][Mz][Mx]
-// The k_solve blocks of several channels in one launch: solve_members_bytes(n)
-// of device memory hold their arguments, written by write_solve_members
-// (synchronous; the arguments name the members' current AB2 history phase).
-size_t solve_members_bytes(int n);
-hipError_t write_solve_members(Ctx* const* m, int n, void* dev);
-hipError_t launch_solve_members(hipStream_t st, Ctx* const* m, int n, const void* dev);
-hipError_t launch_wsolve(Ctx& c);      // diagonalised omega_y solve (all modes but the mean)
+// hsolve.hip: the diagonalised solves; 0 = v and the mean mode, 1 = omega_y
+hipError_t launch_hsolve(Ctx& c, int which);
+hipError_t launch_wall_setup(Ctx& c);
 // u, w, omega_x, omega_z (and the next RHS brackets) from v, omega_y, U, W;
 // f32: u, w, omega_x, omega_z into uf, wf, oxf, ozf (rounded to FP32) instead
 hipError_t launch_kinematics(Ctx& c, bool f32 = false);

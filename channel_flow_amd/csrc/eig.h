@@ -49,11 +49,11 @@ inline void lu_solve(const Mat& lu_, const std::vector<int>& piv, int n, Mat& b,
     }
   for (int i = n - 1; i >= 0; --i) {
     const double d = 1.0 / lu_[(size_t)i * n + i];
-    for (int j = 0; j < m; ++j) {
-      double s = b[(size_t)i * m + j];
-      for (int k = i + 1; k < n; ++k) s -= lu_[(size_t)i * n + k] * b[(size_t)k * m + j];
-      b[(size_t)i * m + j] = s * d;
+    for (int k = i + 1; k < n; ++k) {
+      const double f = lu_[(size_t)i * n + k];
+      for (int j = 0; j < m; ++j) b[(size_t)i * m + j] -= f * b[(size_t)k * m + j];
     }
+    for (int j = 0; j < m; ++j) b[(size_t)i * m + j] *= d;
   }
 }
 

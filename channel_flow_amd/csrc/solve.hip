@@ -1,6 +1,8 @@
-// Per-(kx,|kz|) solves of the v and omega_y equations with kinematics
-// (PF:242-394, getvelocityandvorticity PF:2347-2407), the mean mode
-// (PF:401-474), and the GPU set-up of the operator inverses (PF:181-204).
+// Per-(kx,|kz|) solves of the v and omega_y equations with stored inverses
+// (PF:242-394; the path taken when the diagonalised operators of hsolve.hip do
+// not verify), with their mean mode (PF:401-474), the kinematics
+// (getvelocityandvorticity PF:2347-2407), and the GPU set-up of the operator
+// inverses (PF:181-204).
 //
 // The collocation operators of get_coef_v (PF:3348-3381) and get_coef_omegay
 // (PF:3432-3455) depend on (kx, kz) through k^2 only, so the modes +kz and
@@ -15,7 +17,6 @@
 // zgetri inverses with a_multiply_x (PF:4123-4139).
 #include "chf_internal.h"
 #include "fftreg.h"
-#include "mfma.h"
 
 namespace chf {
 
@@ -24,11 +25,10 @@ namespace chf {
 struct SetupArgs {
   const double *t0, *t2, *t4;
   const double *al, *be;
-  double* inv;      // v halves (and omega halves when not diagonalised)
+  double* inv;      // v halves (null: not stored)
   double* inv_w;    // omega halves
   int Mx, N, Ny, ne, no;
   long stride, row, stride_w, row_w;
-  int wdiag;        // omega operator diagonalised: only group 0's omega halves are stored
   const int* crep;  // representative group of each operator class
   double dt, re;
 };
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void k_setup(SetupArgs a) {
   const int n = par ? a.no : a.ne;
   const int nP = n + (n & 1);  // even width: 16-byte aligned row pairs
   const int neP = a.ne + (a.ne & 1);
-  if (eq == 1 && g > 0 && a.wdiag) return;
+  if (eq == 0 && !a.inv) return;
   const long orow = eq ? a.row_w : a.row;
   double* out = (eq ? a.inv_w + (long)cls * a.stride_w : a.inv + (long)cls * a.stride) + par * neP;
   if (eq == 0 && g == 0) {  // k^2 = 0 has no v system (PF:184, 247)
@@ -162,7 +162,6 @@ hipError_t launch_setup_inverses(Ctx& c) {
   a.row = d.inv_row;
   a.stride_w = c.stride_w;
   a.row_w = c.row_w;
-  a.wdiag = c.wdiag ? 1 : 0;
   a.crep = c.crep;
   a.dt = c.prm.dt;
   a.re = c.prm.re;
@@ -178,9 +177,8 @@ hipError_t launch_setup_inverses(Ctx& c) {
 // ------------------------------------------------------------------- solve
 
 struct SolveArgs {
-  const double2* rvT;              // v right-hand sides, [column][Rv rows] (even rows, then odd)
+  const double2 *rvE, *rvO;        // v right-hand sides, [row][column] per parity
   const double2 *roE, *roO;        // omega_y right-hand sides, [row][column] per parity
-  int Rv;                          // (ne - 2) + (no - 2)
   const double* inv;
   const double* inv_w;
   double2 *vst, *oy;  // v by group (record [l][side], see KinArgs), omega_y
@@ -189,7 +187,6 @@ struct SolveArgs {
   const double *t0, *t2;
   int Mx, Mz, N, Ny, ne, no;
   long stride, row, stride_w, row_w, ncol;
-  int wdiag;
   const int *bmat, *bg0, *bg1;  // per block: operator class, first and second group (-1: none)
   double dt, re;
 };
@@ -211,8 +208,7 @@ __device__ __forceinline__ double2 stream_load(const double* p) {
 // the modes m0 = (kz, kx) and m1 = (Mz - kz, kx); groups with the same k^2
 // share the operator, so the block streams the class's half-system inverses
 // once, multiplies each by the 4 real right-hand-side vectors (Re, Im of both
-// modes) of each of its groups, and writes v^{n+1} (and omega_y^{n+1} when that
-// operator is not diagonalised) (PF:242-394).  The block holding group 0 is
+// modes) of each of its groups, and writes v^{n+1} and omega_y^{n+1} (PF:242-394).  The block holding group 0 is
 // the mean mode (PF:401-474): U and W with the omega_y-type operator at k^2 = 0.
 // Matrix columns per load batch in the streaming loop of k_solve; two batches
 // alternate, so the next batch is in flight while the current one is used.
@@ -220,30 +216,15 @@ __device__ __forceinline__ double2 stream_load(const double* p) {
 // beats 4 (8 loads, 3 waves), 5 and 8.
 constexpr int kSolveSU = 6;
 
-// MEMBERS: the solve of several independent channels (an ensemble) in one
-// launch.  Channel m owns the solve blocks [first[m], first[m + 1]) of the
-// grid, in the same XCD-contiguous order as a launch of its own; the block
-// size and LDS are the largest any channel needs.  Each block runs its
-// channel's block exactly as a launch of that channel alone would, so the
-// results are bit-identical to separate launches.
-template <bool MEMBERS>
-__global__ __launch_bounds__(512) void k_solve(SolveArgs a1, const SolveArgs* __restrict__ args,
-                                               const int* __restrict__ first, int nm) {
+__global__ __launch_bounds__(512) void k_solve(SolveArgs a) {
   extern __shared__ double rb[];  // [slot][Ny][4 vec], slot = group * neq + eq
-  constexpr int SU = kSolveSU;
-  int b = xcd_group(blockIdx.x, gridDim.x);
-  int m = 0;
-  if constexpr (MEMBERS) {
-    while (m + 1 < nm && b >= first[m + 1]) ++m;
-    b -= first[m];
-  }
-  const SolveArgs& a = MEMBERS ? args[m] : a1;
+  constexpr int SU = kSolveSU, neq = 2;
+  const int b = xcd_group(blockIdx.x, gridDim.x);
   const int Ny = a.Ny, N = a.N, ne = a.ne, no = a.no;
   const int mat = a.bmat[b];
   const int gs0 = a.bg0[b], gs1 = a.bg1[b];
   const int ngr = gs1 >= 0 ? 2 : 1;
   const bool mean = (gs0 == 0);
-  const int neq = a.wdiag ? 1 : 2;  // equations this kernel solves for a non-mean group
   const double c = a.dt * 0.5 / a.re;
 
   // ---- this thread's task: one row pair (2i, 2i+1) of one half system of one
@@ -281,16 +262,9 @@ __global__ __launch_bounds__(512) void k_solve(SolveArgs a1, const SolveArgs* __
         double2 x0 = make_double2(0, 0), x1 = make_double2(0, 0);
         if (i >= nbc) {
           const int r = i - nbc;
-          if (eq) {
-            const double2* src = odd ? a.roO : a.roE;
-            x0 = src[(long)r * a.ncol + col0];
-            if (kzab > 0) x1 = src[(long)r * a.ncol + col1];
-          } else {
-            // consecutive rows are consecutive threads: one contiguous run per mode
-            const int k = odd ? (ne - 2) + r : r;
-            x0 = a.rvT[col0 * a.Rv + k];
-            if (kzab > 0) x1 = a.rvT[col1 * a.Rv + k];
-          }
+          const double2* src = eq ? (odd ? a.roO : a.roE) : (odd ? a.rvO : a.rvE);
+          x0 = src[(long)r * a.ncol + col0];
+          if (kzab > 0) x1 = src[(long)r * a.ncol + col1];
         }
         double* dst = rb + ((gi * neq + eq) * Ny + row) * 4;
         dst[0] = x0.x;
@@ -630,8 +604,8 @@ __global__ __launch_bounds__(256) void k_vtranspose(const double2* __restrict__ 
 static SolveArgs solve_args(const Ctx& c) {
   const Dims& d = c.d;
   SolveArgs a{};
-  a.rvT = c.rvT;
-  a.Rv = d.ne + d.no - 4;
+  a.rvE = c.rvE;
+  a.rvO = c.rvO;
   a.roE = c.roE;
   a.roO = c.roO;
   a.inv = c.inv;
@@ -656,7 +630,6 @@ static SolveArgs solve_args(const Ctx& c) {
   a.row = d.inv_row;
   a.stride_w = c.stride_w;
   a.row_w = c.row_w;
-  a.wdiag = c.wdiag ? 1 : 0;
   a.bmat = c.bmat;
   a.bg0 = c.bg0;
   a.bg1 = c.bg1;
@@ -666,15 +639,13 @@ static SolveArgs solve_args(const Ctx& c) {
   return a;
 }
 
-// LDS bytes (two groups per block, one or two equations each) and threads of
-// one channel's solve blocks: one thread per task; with the omega_y operator
-// diagonalised a block streams the two v half systems only (ne/2 + no/2 row
-// pairs, 128 threads at N = 192), otherwise the omega_y half systems as well.
+// LDS bytes (two groups per block, two equations each) and threads of the
+// solve blocks: one thread per task, a row pair of a half system.
 static void solve_shape(const Ctx& c, size_t* shm, int* threads) {
   const Dims& d = c.d;
-  *shm = sizeof(double) * 4ull * d.Ny * 2 * (c.wdiag ? 1 : 2);
+  *shm = sizeof(double) * 4ull * d.Ny * 2 * 2;
   const int pairs = (d.ne + (d.ne & 1)) / 2 + (d.no + (d.no & 1)) / 2;
-  *threads = ((c.wdiag ? 1 : 2) * pairs + 63) / 64 * 64;
+  *threads = (2 * pairs + 63) / 64 * 64;
 }
 
 static hipError_t allow_shm(const void* kernel, size_t shm) {
@@ -697,239 +668,12 @@ hipError_t launch_solve(Ctx& c) {
   int threads;
   solve_shape(c, &shm, &threads);
   if (threads > 512) return hipErrorInvalidValue;
-  hipError_t e = allow_shm((const void*)k_solve<false>, shm);
+  hipError_t e = allow_shm((const void*)k_solve, shm);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_solve<false>, dim3(c.d.nblocks), dim3(threads), shm, c.stream, a, nullptr, nullptr, 1);
+  hipLaunchKernelGGL(k_solve, dim3(c.d.nblocks), dim3(threads), shm, c.stream, a);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_vtranspose(c);
-}
-
-size_t solve_members_bytes(int n) { return sizeof(SolveArgs) * (size_t)n + sizeof(int) * (size_t)(n + 1); }
-
-hipError_t write_solve_members(Ctx* const* m, int n, void* dev) {
-  std::vector<char> h(solve_members_bytes(n));
-  SolveArgs* args = reinterpret_cast<SolveArgs*>(h.data());
-  int* first = reinterpret_cast<int*>(h.data() + sizeof(SolveArgs) * (size_t)n);
-  first[0] = 0;
-  for (int i = 0; i < n; ++i) {
-    args[i] = solve_args(*m[i]);
-    first[i + 1] = first[i] + m[i]->d.nblocks;
-  }
-  return hipMemcpy(dev, h.data(), h.size(), hipMemcpyHostToDevice);
-}
-
-hipError_t launch_solve_members(hipStream_t st, Ctx* const* m, int n, const void* dev) {
-  size_t shm = 0;
-  int threads = 0;
-  long blocks = 0;
-  for (int i = 0; i < n; ++i) {
-    size_t s;
-    int t;
-    solve_shape(*m[i], &s, &t);
-    shm = s > shm ? s : shm;
-    threads = t > threads ? t : threads;
-    blocks += m[i]->d.nblocks;
-  }
-  if (threads > 512 || blocks > 0x7fffffffL) return hipErrorInvalidValue;
-  hipError_t e = allow_shm((const void*)k_solve<true>, shm);
-  if (e != hipSuccess) return e;
-  const SolveArgs* args = static_cast<const SolveArgs*>(dev);
-  const int* first = reinterpret_cast<const int*>(static_cast<const char*>(dev) + sizeof(SolveArgs) * (size_t)n);
-  hipLaunchKernelGGL(k_solve<true>, dim3((unsigned)blocks), dim3(threads), shm, st, SolveArgs{}, args, first, n);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------- diagonalised omega_y solve
-//
-// For every mode but the mean, omega_y^{n+1} of parity p is
-//   x = R diag(1 / (1 + c (k^2 - lam))) L b
-// (L, R, lam from the set-up), i.e. two FP64 matrix-core products with
-// matrices shared by all modes.  Block = one parity and 64 real columns (32
-// complex modes, kx fastest): the right-hand sides b (the n-1 interior rows)
-// are staged in LDS, Y = L B runs on v_mfma_f64_16x16x4f64 with the A
-// fragments of L read from L2, Y is scaled per (row, mode) and written back
-// to LDS as the B operand of X = R Y, and X lands in omega_y at degrees 2i + p.
-// Eight wavefronts per block own the 16-row blocks, TPW each (wave w: row
-// blocks w, w + 8, ...).  TPW = 1 whenever at most 8 row blocks exist (N up to
-// 254): the kernel then needs 70 VGPRs, so three blocks fit per CU and its
-// waves also fit beside the v solve's (measured 0.164 -> 0.143 ms against
-// TPW = 2, which larger N take).
-struct WArgs {
-  const double *L0, *L1, *R0, *R1, *lam0, *lam1;
-  const double *ro0, *ro1;  // parity-folded right-hand sides, real view [rows][2 ncol]
-  double* oy;               // real view [Ny][2 ncol]
-  const double *al, *be;
-  int n0, n1, Mx, Mz;
-  long ncold;
-  double c;
-};
-
-template <int TPW>
-__global__ __launch_bounds__(512) void k_wsolve(WArgs a) {
-  using MF = Mf<double>;
-  constexpr int CT = 64, NW = 8;  // columns, waves (<= 8 TPW row blocks)
-  extern __shared__ double sB[];   // [rows][CT]
-  const int par = blockIdx.y;
-  const int n = par ? a.n1 : a.n0, m = n - 1;
-  const double* L = par ? a.L1 : a.L0;
-  const double* R = par ? a.R1 : a.R0;
-  const double* lam = par ? a.lam1 : a.lam0;
-  const double* ro = par ? a.ro1 : a.ro0;
-  const int MB1 = (m + 15) / 16, KB = (m + 3) / 4, MB2 = (n + 15) / 16;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const long col0 = (long)blockIdx.x * CT;
-  // stage B: rows r < m, zero rows up to 16 MB1.  Each thread issues eight
-  // loads before its first LDS store; the loads are unconditional (row and
-  // column clamped into the array, the value zeroed afterwards), so no branch
-  // splits them and they are in flight together.
-  constexpr int SL = 8;
-  const int nst = 16 * MB1 * CT;
-  for (int i0 = threadIdx.x; i0 < nst; i0 += SL * blockDim.x) {
-    double v[SL];
-#pragma unroll
-    for (int u = 0; u < SL; ++u) {
-      const int idx = i0 + u * blockDim.x;
-      const int r = idx / CT, cc = idx - r * CT;
-      const long col = col0 + cc;
-      const double x = ro[(long)min(r, m - 1) * a.ncold + min(col, a.ncold - 1)];
-      v[u] = (idx < nst && r < m && col < a.ncold) ? x : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < SL; ++u) {
-      const int idx = i0 + u * blockDim.x;
-      if (idx < nst) sB[idx] = v[u];
-    }
-  }
-  __syncthreads();
-  MF::acc acc[TPW][4];
-  // acc = A B over k blocks 0..KB-1 (A: packed fragments of L or R, MB row
-  // blocks; B: the LDS tile).  The A fragments come from L2 in batches of four
-  // k blocks, the next batch requested before the current one is used; the
-  // batch indices are clamped so the loads are unconditional and the number in
-  // flight is fixed.
-  auto product = [&](const double* A, int MB) {
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) acc[t][cb] = MF::acc{0, 0, 0, 0};
-    double fa[TPW][4], fb[TPW][4];
-    auto fetch = [&](double (&f)[TPW][4], int kb0) {
-#pragma unroll
-      for (int t = 0; t < TPW; ++t) {
-        const int rb = min(wave + NW * t, MB - 1);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) f[t][u] = A[((long)rb * KB + min(kb0 + u, KB - 1)) * 64 + lane];
-      }
-    };
-    auto use = [&](const double (&f)[TPW][4], int kb0) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int kb = kb0 + u;
-        if (kb >= KB) break;
-        double bf[4];
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) bf[cb] = sB[(4 * kb + (lane >> 4)) * CT + 16 * cb + (lane & 15)];
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          if (wave + NW * t < MB) {
-#pragma unroll
-            for (int cb = 0; cb < 4; ++cb) acc[t][cb] = MF::mma(f[t][u], bf[cb], acc[t][cb]);
-          }
-        }
-      }
-    };
-    fetch(fa, 0);
-    for (int kb0 = 0; kb0 < KB; kb0 += 8) {
-      fetch(fb, kb0 + 4);
-      use(fa, kb0);
-      if (kb0 + 4 >= KB) break;
-      fetch(fa, kb0 + 8);
-      use(fb, kb0 + 4);
-    }
-  };
-  product(L, MB1);
-  __syncthreads();
-  // scale rows by 1 / (1 + c (k^2 - lam)) and write Y back as the next B operand
-  double s[4];
-#pragma unroll
-  for (int cb = 0; cb < 4; ++cb) {
-    const long cm = (col0 + 16 * cb + (lane & 15)) >> 1;
-    const int kz = (int)((unsigned)cm / (unsigned)a.Mx), kx = (int)(cm - (long)kz * a.Mx);
-    const bool in = cm < (a.ncold >> 1);
-    const double alx = in ? a.al[kx] : 0.0, bez = in ? a.be[kz] : 0.0;
-    s[cb] = alx * alx + bez * bez;
-  }
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    const int rb = wave + NW * t;
-    if (rb >= MB1) continue;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int row = 16 * rb + MF::row(lane, e);
-      const double lr = lam[row];
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const double y = row < m ? acc[t][cb][e] / (1.0 + a.c * (s[cb] - lr)) : 0.0;
-        sB[row * CT + 16 * cb + (lane & 15)] = y;
-      }
-    }
-  }
-  __syncthreads();
-  product(R, MB2);
-  // store x_i -> omega_y at degree 2i + p; the mean mode and the span Nyquist
-  // column are not solved here (PF:247)
-#pragma unroll
-  for (int cb = 0; cb < 4; ++cb) {
-    const long col = col0 + 16 * cb + (lane & 15);
-    const long cm = col >> 1;
-    if (col >= a.ncold || cm == 0) continue;
-    const int kz = (int)((unsigned)cm / (unsigned)a.Mx);
-    if (kz == a.Mz / 2) continue;
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const int rb = wave + NW * t;
-      if (rb >= MB2) continue;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = 16 * rb + MF::row(lane, e);
-        if (i < n) a.oy[(long)(2 * i + par) * a.ncold + col] = acc[t][cb][e];
-      }
-    }
-  }
-}
-
-hipError_t launch_wsolve(Ctx& c) {
-  const Dims& d = c.d;
-  WArgs a{};
-  a.L0 = c.wL[0];
-  a.L1 = c.wL[1];
-  a.R0 = c.wR[0];
-  a.R1 = c.wR[1];
-  a.lam0 = c.wlam[0];
-  a.lam1 = c.wlam[1];
-  a.ro0 = reinterpret_cast<const double*>(c.roE);
-  a.ro1 = reinterpret_cast<const double*>(c.roO);
-  a.oy = reinterpret_cast<double*>(c.oy);
-  a.al = c.alpha;
-  a.be = c.beta;
-  a.n0 = d.ne;
-  a.n1 = d.no;
-  a.Mx = d.Mx;
-  a.Mz = d.Mz;
-  a.ncold = 2 * d.ncol;
-  a.c = c.prm.dt * 0.5 / c.prm.re;
-  const int m = d.ne - 1;
-  const size_t shm = sizeof(double) * 64 * 16 * ((m + 15) / 16);
-  if (shm > 65536) return hipErrorInvalidValue;
-  const int mb = (d.ne + 15) / 16;  // row blocks of the larger (even) half system
-  if (mb > 16) return hipErrorInvalidValue;
-  const unsigned tiles = (unsigned)((a.ncold + 63) / 64);
-  if (mb <= 8)
-    hipLaunchKernelGGL(k_wsolve<1>, dim3(tiles, 2), dim3(512), shm, c.stream, a);
-  else
-    hipLaunchKernelGGL(k_wsolve<2>, dim3(tiles, 2), dim3(512), shm, c.stream, a);
-  return hipGetLastError();
 }
 
 hipError_t launch_kinematics(Ctx& c, bool f32) {

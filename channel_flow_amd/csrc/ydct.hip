@@ -306,8 +306,7 @@ __global__ __launch_bounds__(YT<V>::TX* ymax(A1, A2)) void k_ycheb(YArgs a) {
 // DCT, FP64), plus the AB2 forcing F = 3 dt/2 h^n - dt/2 h^(n-1), folded by
 // parity at the point pairs p = r + POFF, q = N - p: even row r
 // ((f+F)_p + (f+F)_q)/2 (rows r < ne - POFF), odd row r ((f+F)_p - (f+F)_q)/2
-// (r < no - POFF).  v: each mode's rows as one record, [column][Rv: even rows,
-// then odd rows]; omega_y: [row][column] per parity.
+// (r < no - POFF), [row][column] per parity.
 //
 // FUSE: h^n arrives as coefficients (the h assembly's output) and this kernel
 // forms its point values, writes them (the next step's h^(n-1) and the state
@@ -322,9 +321,9 @@ struct YRhsArgs {
   const double2* hc;  // FUSE: h^n coefficients
   double2* hn;        // h^n point values (FUSE: written, else read)
   const double2* hp;  // h^(n-1) point values
-  double2 *outT, *outE, *outO;
+  double2 *outE, *outO;
   long ncol;
-  int Rv, ne, no;
+  int ne, no;
   double dt;
   const double2* twL;
 };
@@ -435,14 +434,8 @@ __global__ __launch_bounds__(YT<double2>::TX* ymax(N1, N2)) void k_yrhs(YRhsArgs
       ev = yscale(yadd(vp, vq), 0.5);
       od = yscale(ysub(vp, vq), 0.5);
     }
-    if constexpr (POFF == 2) {
-      double2* rec = a.outT + col * a.Rv;
-      rec[r] = ev;
-      if (r < Mo) rec[Me + r] = od;
-    } else {
-      a.outE[(long)r * nc + col] = ev;
-      if (r < Mo) a.outO[(long)r * nc + col] = od;
-    }
+    a.outE[(long)r * nc + col] = ev;
+    if (r < Mo) a.outO[(long)r * nc + col] = od;
   }
 }
 
@@ -534,17 +527,15 @@ static hipError_t run_yrhs(Ctx& c, int which, bool fuse, const YRhsArgs& a) {
 }
 
 hipError_t launch_yrhs(Ctx& c, int which, const double2* g, const double2* hc, double2* hn, const double2* hp,
-                       double2* oE, double2* oO, double2* oT) {
+                       double2* oE, double2* oO) {
   YRhsArgs a{};
   a.g = g;
   a.hc = hc;
   a.hn = hn;
   a.hp = hp;
-  a.outT = oT;
   a.outE = oE;
   a.outO = oO;
   a.ncol = c.d.ncol;
-  a.Rv = c.d.ne + c.d.no - 4;
   a.ne = c.d.ne;
   a.no = c.d.no;
   a.dt = c.prm.dt;

@@ -56,10 +56,10 @@ typedef struct chf_state {
   double *vnp1, *omegaynp1, *rhsvn, *rhsomegayn, *unp1, *wnp1;   /* record 2 */
 } chf_state;
 
-/* Builds the per-(kx,|kz|) operator inverses on the GPU (replaces SCHEB PF:156
- * and the get_coef_v/get_coef_omegay + zgetrf/zgetri set-up loop, PF:181-204).
- * The omega_y operator is diagonalised when the decomposition reproduces
- * direct solves to 1e-12, else its half-system inverses are stored;
+/* Sets up the v and omega_y operators (replaces SCHEB PF:156 and the
+ * get_coef_v/get_coef_omegay + zgetrf/zgetri set-up loop, PF:181-204).  Both are
+ * diagonalised when the decomposition reproduces direct solves to 1e-11, else
+ * the half-system inverses of every (kx,|kz|) are built on the GPU and stored;
  * CHF_OMEGA_INVERSES=stored in the environment selects the stored inverses.
  * The wall-normal transforms (padded synthesis, analysis, Gauss-Lobatto
  * point values, the solves' right-hand sides) run as FFTs along y, in the
