@@ -163,7 +163,8 @@ void free_all(Ctx* c) {
   f(c->inv); f(c->inv0); f(c->crep); f(c->bmat); f(c->bg0); f(c->bg1);
   for (int i = 0; i < 2; ++i) { f(c->hL[i]); f(c->hV[i]); f(c->hvec[i]); f(c->hwall[i]); }
   f(c->tmean);
-  f(c->phys_c); f(c->phys_r[0]); f(c->phys_r[1]); f(c->phys_r[2]); f(c->stats); f(c->twxu); f(c->twzu); f(c->twx); f(c->twz); f(c->twy); f(c->costab);
+  for (int i = 0; i < 3; ++i) { f(c->phys_c[i]); f(c->phys_r[i]); }
+  f(c->stats_part); f(c->stats); f(c->twxu); f(c->twzu); f(c->twx); f(c->twz); f(c->twy); f(c->costab);
   f(c->gv); f(c->go); f(c->nonfinite);
   for (hipEvent_t e : c->event_pool) (void)hipEventDestroy(e);
   c->event_pool.clear();
@@ -981,15 +982,26 @@ int chf_set_timing(void* ctx, int on) {
 
 namespace {
 
-// Buffers of the unpadded physical transform, allocated on first use (they
-// are not part of the timestep).
+// Buffers of the unpadded physical transform and of the statistics, allocated
+// on first use (they are not part of the timestep).
 int ensure_physical(Ctx* c) {
-  if (c->stats) return 0;
   const Dims& d = c->d;
-  const size_t plane = (size_t)d.Ny * d.Mz * 2 * d.Mx;
-  CHF_TRY(dalloc(c, &c->phys_c, (size_t)d.Ny * d.ncol));
-  for (auto& p : c->phys_r) CHF_TRY(dalloc(c, &p, plane));
-  CHF_TRY(dalloc(c, &c->stats, 12 * (size_t)d.Ny));
+  if (!c->phys_c[0]) CHF_TRY(dalloc(c, &c->phys_c[0], (size_t)d.Ny * d.ncol));
+  if (!c->phys_r[0]) CHF_TRY(dalloc(c, &c->phys_r[0], (size_t)d.Ny * d.Mz * 2 * d.Mx));
+  return 0;
+}
+
+int ensure_statistics(Ctx* c) {
+  const Dims& d = c->d;
+  for (auto& p : c->phys_c)
+    if (!p) CHF_TRY(dalloc(c, &p, (size_t)d.Ny * d.ncol));
+  if (stats_in_lines(*c)) {
+    if (!c->stats_part) CHF_TRY(dalloc(c, &c->stats_part, 12 * (size_t)d.Ny * stats_splits(*c)));
+  } else {
+    for (auto& p : c->phys_r)
+      if (!p) CHF_TRY(dalloc(c, &p, (size_t)d.Ny * d.Mz * 2 * d.Mx));
+  }
+  if (!c->stats) CHF_TRY(dalloc(c, &c->stats, 12 * (size_t)d.Ny));
   return 0;
 }
 
@@ -1018,7 +1030,7 @@ int chf_physical(void* ctx, int field, double* out) {
   const int rc = ensure_physical(c);
   if (rc) return rc;
   CHF_TRY(form_fields64(c));
-  CHF_TRY(launch_physical(*c, f, c->phys_c, c->phys_r[0]));
+  CHF_TRY(launch_physical(*c, f, c->phys_c[0], c->phys_r[0]));
   const size_t n = (size_t)c->d.Ny * c->d.Mz * 2 * c->d.Mx;
   CHF_TRY(hipMemcpyAsync(out, c->phys_r[0], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   CHF_TRY(hipStreamSynchronize(c->stream));
@@ -1045,11 +1057,11 @@ int chf_statistics(void* ctx, double* out) {
   if (!ctx) return -1;
   Ctx* c = static_cast<Ctx*>(ctx);
   if (!out) return fail(c, "chf_statistics: null output");
-  const int rc = ensure_physical(c);
+  const int rc = ensure_statistics(c);
   if (rc) return rc;
   CHF_TRY(form_fields64(c));
-  for (int q = 0; q < 3; ++q) CHF_TRY(launch_physical(*c, field_ptr(c, q), c->phys_c, c->phys_r[q]));
-  CHF_TRY(launch_plane_stats(*c, c->phys_r[0], c->phys_r[1], c->phys_r[2], c->stats));
+  const double2* f[3] = {c->u, c->v, c->w};
+  CHF_TRY(launch_statistics(*c, f, c->phys_c, c->phys_r, c->stats_part, c->stats));
   CHF_TRY(hipMemcpyAsync(out, c->stats, 12 * (size_t)c->d.Ny * sizeof(double), hipMemcpyDeviceToHost,
                          c->stream));
   CHF_TRY(hipStreamSynchronize(c->stream));

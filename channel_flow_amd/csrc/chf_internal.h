@@ -173,8 +173,9 @@ struct Ctx {
   // then exp(-2 pi i m/N) (m < N), then exp(i pi k/2N) (k < N), FP64
   double2* twy = nullptr;
   // unpadded physical output and plane statistics (allocated on first use)
-  double2* phys_c = nullptr;                          // [Ny][Mz][Mx] work
-  double* phys_r[3] = {nullptr, nullptr, nullptr};    // [Ny][Mz][2 Mx] physical u, v, w
+  double2* phys_c[3] = {nullptr, nullptr, nullptr};   // [Ny][Mz][Mx] work (chf_physical: the first)
+  double* phys_r[3] = {nullptr, nullptr, nullptr};    // [Ny][Mz][2 Mx] physical fields (chf_physical: the first)
+  double* stats_part = nullptr;                       // statistics' partial sums
   double* stats = nullptr;                            // [12][Ny]
   double2 *twxu = nullptr, *twzu = nullptr;           // unpadded twiddles (2 Mx, Mz), set up at creation
   double2* scratch = nullptr;  // this device's no-allocation work memory (shared by its contexts)
@@ -239,11 +240,17 @@ hipError_t launch_ysynth32f(Ctx& c, const float2* const* in, float2* const* out,
 hipError_t launch_yanalysis32f(Ctx& c, const float2* const* in, float2* const* out, int nf);  // FP32 coefficients out
 hipError_t launch_yanalysis32(Ctx& c, const float2* const* in, double2* const* out, int nf);
 hipError_t launch_synth_points_h(Ctx& c, const double2* const* in, double2* const* out, int nf);  // FP32 compute in the mixed form
-hipError_t launch_span_inverse_unpadded(Ctx& c, double2* inout);
-hipError_t launch_stream_c2r_unpadded(Ctx& c, const double2* in, double* out);
+hipError_t launch_span_inverse_unpadded(Ctx& c, double2* const* inout, int nf);
+hipError_t launch_stream_c2r_lds(Ctx& c, const double2* in, double* out);
 // unpadded physical field: work = complex [Ny][Mz][Mx], out = real [Ny][nny][nnx]
 hipError_t launch_physical(Ctx& c, const double2* field, double2* work, double* out);
-hipError_t launch_plane_stats(Ctx& c, const double* u, const double* v, const double* w, double* out);
+// plane statistics [12][Ny] of three fields: work as above, one per field;
+// part = stats_splits() x [Ny][12] when stats_in_lines(), else phys = three
+// physical fields
+int stats_splits(const Ctx& c);
+bool stats_in_lines(const Ctx& c);
+hipError_t launch_statistics(Ctx& c, const double2* const* fields, double2* const* work, double* const* phys,
+                             double* part, double* out);
 hipError_t launch_rhs(Ctx& c, int which);  // 0 = v, 1 = omega_y
 hipError_t launch_solve(Ctx& c);       // stored inverses: v, omega_y and the mean mode (k_solve, then launch_vtranspose)
 hipError_t launch_vtranspose(Ctx& c);  // v from the solve's per-group records to [Ny][Mz][Mx]

@@ -215,7 +215,8 @@ static hipError_t launch_z(Ctx& c, double2* const* in, double2* const* out, int 
 
 // ------------------------------------------------ unpadded physical output
 
-// Streamwise c2r of LPB (y point, span point) lines per block:
+// Streamwise c2r of LPB (y point, span point) lines per block, for the lengths
+// without a register split (stats.hip has those):
 // in [Ny][Mz][Mx] complex -> out [Ny][Mz][nnx] real.
 struct XPArgs {
   const double2* in;
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(256) void k_xphys(XPArgs a) {
 }
 
 
-hipError_t launch_stream_c2r_unpadded(Ctx& c, const double2* in, double* out) {
+hipError_t launch_stream_c2r_lds(Ctx& c, const double2* in, double* out) {
   const Dims& d = c.d;
   XPArgs a{};
   a.in = in;
@@ -272,27 +273,6 @@ hipError_t launch_stream_c2r_unpadded(Ctx& c, const double2* in, double* out) {
   a.tw = c.twxu;
   const size_t shm = 2ull * a.LPB * a.L * sizeof(double2);
   hipLaunchKernelGGL(k_xphys, dim3((unsigned)((a.nlines + a.LPB - 1) / a.LPB)), dim3(256), shm, c.stream, a);
-  return hipGetLastError();
-}
-
-// transform(1, .) span step (fourtrx_zcomp, PF:790-803): Mz span modes ->
-// Mz span points per (wall-normal point, kx), Nyquist slot zeroed, in place.
-hipError_t launch_span_inverse_unpadded(Ctx& c, double2* inout) {
-  const Dims& d = c.d;
-  ZArgs a{};
-  a.in[0] = inout;
-  a.out[0] = inout;
-  a.Mx = d.Mx;
-  a.Mz = d.Mz;
-  a.Lz = d.Mz;
-  a.TX = pick_tx(d.Mx, d.Mz);
-  a.in_plane = (long)d.Mz * d.Mx;
-  a.out_plane = a.in_plane;
-  a.pl = make_plan(d.Mz);
-  a.tw = c.twzu;
-  dim3 grid(d.Mx / a.TX, d.Ny, 1);
-  const size_t shm = 2ull * a.TX * d.Mz * sizeof(double2);
-  hipLaunchKernelGGL(k_zfft_inv, grid, dim3(256), shm, c.stream, a);
   return hipGetLastError();
 }
 
@@ -1182,6 +1162,70 @@ static hipError_t zfft_reg64(Ctx& c, double2* const* in, double2* const* out, in
 
 hipError_t launch_zfft32(Ctx& c, const float2* const* in, float2* const* out, int nf, bool inv) {
   return zfft_reg(c, regz_args<float2>(c, in, out, nf, inv, c.twzf), inv, nf);
+}
+
+// One instantiation of the span kernel at the unpadded length Lz = Mz: the same
+// mode placement then reads modes 0 .. Mz - 1 in order with the Nyquist slot zero.
+template <int N1, int N2>
+static hipError_t run_span_unpadded(Ctx& c, const RegZ<double2>& a, int nf) {
+  using Gm = Geo<N1, N2>;
+  constexpr int TX = (256 / Gm::G) >= 16 ? 16 : ((256 / Gm::G) >= 8 ? 8 : 4);
+  constexpr size_t shm = sizeof(double2) * (Gm::L + (size_t)TX * Gm::LINE_Z);
+  const void* fn = (const void*)k_zfft_reg<N1, N2, TX, true, double2>;
+  if (shm > 65536) {
+    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((k_zfft_reg<N1, N2, TX, true, double2>), dim3((c.d.Mx + TX - 1) / TX, c.d.Ny, nf),
+                     dim3(TX * Gm::G), shm, c.stream, a);
+  return hipGetLastError();
+}
+
+// transform(1, .) span step (fourtrx_zcomp, PF:790-803): Mz span modes ->
+// Mz span points per (wall-normal point, kx), Nyquist slot zeroed, in place
+// (a block reads all of its columns before it writes them).
+hipError_t launch_span_inverse_unpadded(Ctx& c, double2* const* inout, int nf) {
+  const Dims& d = c.d;
+  RegZ<double2> a{};
+  for (int f = 0; f < nf; ++f) a.in[f] = a.out[f] = inout[f];
+  a.Mx = d.Mx;
+  a.Mz = d.Mz;
+  a.in_plane = a.out_plane = (long)d.Mz * d.Mx;
+  a.tw = c.twzu;
+  switch (d.Mz) {  // 256x193x256: 0.081 -> 0.041 ms a field against the LDS kernel
+    case 8: return run_span_unpadded<2, 4>(c, a, nf);
+    case 12: return run_span_unpadded<3, 4>(c, a, nf);
+    case 16: return run_span_unpadded<4, 4>(c, a, nf);
+    case 24: return run_span_unpadded<4, 6>(c, a, nf);
+    case 32: return run_span_unpadded<4, 8>(c, a, nf);
+    case 36: return run_span_unpadded<6, 6>(c, a, nf);
+    case 48: return run_span_unpadded<6, 8>(c, a, nf);
+    case 64: return run_span_unpadded<8, 8>(c, a, nf);
+    case 72: return run_span_unpadded<8, 9>(c, a, nf);
+    case 96: return run_span_unpadded<8, 12>(c, a, nf);
+    case 108: return run_span_unpadded<9, 12>(c, a, nf);
+    case 128: return run_span_unpadded<8, 16>(c, a, nf);
+    case 144: return run_span_unpadded<12, 12>(c, a, nf);
+    case 192: return run_span_unpadded<12, 16>(c, a, nf);
+    case 216: return run_span_unpadded<12, 18>(c, a, nf);
+    case 256: return run_span_unpadded<16, 16>(c, a, nf);
+    case 288: return run_span_unpadded<16, 18>(c, a, nf);
+    case 384: return run_span_unpadded<16, 24>(c, a, nf);
+    case 512: return run_span_unpadded<16, 32>(c, a, nf);
+    default: break;
+  }
+  ZArgs z{};
+  for (int f = 0; f < nf; ++f) z.in[f] = z.out[f] = inout[f];
+  z.Mx = d.Mx;
+  z.Mz = d.Mz;
+  z.Lz = d.Mz;
+  z.TX = pick_tx(d.Mx, d.Mz);
+  z.in_plane = z.out_plane = a.in_plane;
+  z.pl = make_plan(d.Mz);
+  z.tw = c.twzu;
+  const size_t shm = 2ull * z.TX * d.Mz * sizeof(double2);
+  hipLaunchKernelGGL(k_zfft_inv, dim3(d.Mx / z.TX, d.Ny, nf), dim3(256), shm, c.stream, z);
+  return hipGetLastError();
 }
 
 hipError_t launch_xpass32(Ctx& c) {
