@@ -324,6 +324,15 @@ int autotune(Ctx* c) {
   return 0;
 }
 
+// Fields from this many values on run their independent launches on the
+// context's two streams: each cross-stream wait costs about 10 us on the
+// device, and the launches' tails that the overlap fills only outweigh that on
+// large grids.  Step times (us) on two streams / one: 24x22x16 143 / 60,
+// 32x33x32 142 / 68, 96x101x96 mixed 266 / 241, 128x129x128 590 / 579 (1.06 M
+// values), 192x161x192 1680 / 1723 (2.97 M), 256x193x256 FP64 2985 / 2965, mixed
+// 1868 / 1873, 512x257x512 FP64 20720 / 21270, mixed 11800 / 12075.
+constexpr size_t kOverlapValues = size_t(2) << 20;
+
 int build(Ctx* c, DegreeCache& cache) {
   Dims& d = c->d;
   const chf_params& p = c->prm;
@@ -359,6 +368,7 @@ int build(Ctx* c, DegreeCache& cache) {
   CHF_TRY(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
 
   const size_t fld = (size_t)d.Ny * d.ncol;
+  c->overlap = c->overlap && fld >= kOverlapValues;
   CHF_TRY(dalloc(c, &c->alpha, d.Mx));
   CHF_TRY(dalloc(c, &c->beta, d.Mz));
   CHF_TRY(dalloc(c, &c->v, fld));
