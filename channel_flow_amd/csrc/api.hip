@@ -142,6 +142,8 @@ int validate(const chf_params* p, std::string& msg) {
 }
 
 void free_all(Ctx* c) {
+  if (c->holds_pool) hostcopy_release();
+  c->holds_pool = false;
   auto f = [](void* p) {
     if (p) (void)hipFree(p);
   };
@@ -350,6 +352,8 @@ int build(Ctx* c, DegreeCache& cache) {
   d.ncol = (long)d.Mz * d.Mx;
   d.ngroups = d.Mx * (d.Mz / 2);
 
+  hostcopy_retain();
+  c->holds_pool = true;
   CHF_TRY(hipGetDevice(&c->device));
   CHF_TRY(resolve_scratch(c->device, &c->scratch));
   int max_lds = 0;
@@ -866,7 +870,9 @@ int chf_set_state(void* ctx, const chf_state* st) {
       {c->hv[pv], st->unp1, fb}, {c->hg[pv], st->wnp1, fb}};
   for (auto& e : m)
     if (!e.src) return fail(c, "chf_set_state: null array");
-  for (auto& e : m) CHF_TRY(hipMemcpyAsync(e.dst, e.src, e.bytes, hipMemcpyHostToDevice, c->stream));
+  std::vector<HostArray> arrays;
+  for (auto& e : m) arrays.push_back({e.dst, const_cast<double*>(e.src), e.bytes});
+  CHF_TRY(copy_arrays(*c, arrays, false));
   c->hdefer = false;  // h^n's point values are the record's
   // u, w, omega_x, omega_z and the brackets of the loaded v, omega_y, U, W
   CHF_TRY(load_kinematics(c));
@@ -889,8 +895,9 @@ int chf_get_state(void* ctx, const chf_state* st) {
   for (auto& e : m)
     if (!e.dst) return fail(c, "chf_get_state: null array");
   CHF_TRY(form_h_points(c));
-  for (auto& e : m) CHF_TRY(hipMemcpyAsync(e.dst, e.src, e.bytes, hipMemcpyDeviceToHost, c->stream));
-  CHF_TRY(hipStreamSynchronize(c->stream));
+  std::vector<HostArray> arrays;
+  for (auto& e : m) arrays.push_back({const_cast<double2*>(e.src), e.dst, e.bytes});
+  CHF_TRY(copy_arrays(*c, arrays, true));
   return 0;
 }
 
@@ -901,10 +908,10 @@ int chf_init_fields(void* ctx, const double* vnp1, const double* omegaynp1, cons
   if (!vnp1 || !omegaynp1 || !au0 || !w0) return fail(c, "chf_init_fields: null array");
   const Dims& d = c->d;
   const size_t fb = (size_t)d.Ny * d.ncol * sizeof(double2), mb = d.Ny * sizeof(double2);
-  CHF_TRY(hipMemcpyAsync(c->v, vnp1, fb, hipMemcpyHostToDevice, c->stream));
-  CHF_TRY(hipMemcpyAsync(c->oy, omegaynp1, fb, hipMemcpyHostToDevice, c->stream));
-  CHF_TRY(hipMemcpyAsync(c->au0, au0, mb, hipMemcpyHostToDevice, c->stream));
-  CHF_TRY(hipMemcpyAsync(c->w0, w0, mb, hipMemcpyHostToDevice, c->stream));
+  CHF_TRY(copy_arrays(*c,
+                      {{c->v, const_cast<double*>(vnp1), fb}, {c->oy, const_cast<double*>(omegaynp1), fb},
+                       {c->au0, const_cast<double*>(au0), mb}, {c->w0, const_cast<double*>(w0), mb}},
+                      false));
   // h^n = 0 and L^n = 0 so that the rotation in getnonlinear leaves h^{-1} = 0 (PF:2316)
   c->hdefer = false;
   for (double2* q : {c->hv[0], c->hv[1], c->hg[0], c->hg[1]})
@@ -958,9 +965,10 @@ int chf_get_fields(void* ctx, double* unp1, double* wnp1, double* omegaxnp1, dou
   CHF_TRY(form_fields64(c));
   struct { const double2* src; double* dst; } m[] = {
       {c->u, unp1}, {c->w, wnp1}, {c->ox, omegaxnp1}, {c->oz, omegaznp1}};
+  std::vector<HostArray> arrays;
   for (auto& e : m)
-    if (e.dst) CHF_TRY(hipMemcpyAsync(e.dst, e.src, fb, hipMemcpyDeviceToHost, c->stream));
-  CHF_TRY(hipStreamSynchronize(c->stream));
+    if (e.dst) arrays.push_back({const_cast<double2*>(e.src), e.dst, fb});
+  CHF_TRY(copy_arrays(*c, arrays, true));
   return 0;
 }
 
@@ -1042,8 +1050,7 @@ int chf_physical(void* ctx, int field, double* out) {
   CHF_TRY(form_fields64(c));
   CHF_TRY(launch_physical(*c, f, c->phys_c[0], c->phys_r[0]));
   const size_t n = (size_t)c->d.Ny * c->d.Mz * 2 * c->d.Mx;
-  CHF_TRY(hipMemcpyAsync(out, c->phys_r[0], n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CHF_TRY(hipStreamSynchronize(c->stream));
+  CHF_TRY(copy_arrays(*c, {{c->phys_r[0], out, n * sizeof(double)}}, true));
   return 0;
 }
 

@@ -85,6 +85,7 @@ struct Ctx {
   chf_params prm{};
   Dims d{};
   int device = 0;
+  bool holds_pool = false;  // counted among the staging pool's users
   hipStream_t stream = nullptr;
   // second stream of the context (default priority): with the operators
   // diagonalised, the omega_y right-hand side and solve run on it while the v
@@ -209,6 +210,17 @@ FftPlan make_plan(int L);
 bool fft_length_ok(int L);
 
 extern const char* const kKernelNames[K_COUNT];
+
+// hostcopy.hip: device arrays to or from the caller's pageable arrays; returns
+// when the copies are done.  The contexts alive hold the staging pool.
+struct HostArray {
+  void* dev;
+  void* host;
+  size_t bytes;
+};
+hipError_t copy_arrays(Ctx& c, const std::vector<HostArray>& arrays, bool to_host);
+void hostcopy_retain();
+void hostcopy_release();
 
 // ---- kernel launchers (each returns hipGetLastError()) ----
 bool reg_fft_length32(int L);  // padded lengths that the mixed form takes
