@@ -14,8 +14,6 @@
 //                  and omega_y equations (get_coef_rhs PF:3385-3425 with
 //                  PF:252-257; get_rhs_omegay PF:3458-3489 with PF:335-340),
 //                  emitted as the parity-folded right-hand sides
-//   hassemble    : h_v = k^2 L_y + i alpha D L_x + i beta D L_z,
-//                  h_g = i alpha L_z - i beta L_x (PF:1502-1540, dz PF:570-599)
 #include <type_traits>
 
 #include "chf_internal.h"
@@ -409,189 +407,5 @@ hipError_t launch_rhs(Ctx& c, int which) {
   if (which == 0) return rhs_syn<2>(c, c.gv, c.hv[nxt], c.hv[prv], c.rvE, c.rvO);
   return rhs_syn<1>(c, c.go, c.hg[nxt], c.hg[prv], c.roE, c.roO);
 }
-
-// ---------------------------------------------------------------- h assembly
-
-// L^n coefficients in FP64, or (mixed form with FFT transforms) in FP32: the
-// FP32 analysis's results, exact in either width
-struct LIn {
-  const double2* d;
-  const float2* f;
-  // the stored value (float2 or double2); widened where it is used, so that
-  // a batch of loads stays in flight
-  template <bool F32>
-  __device__ __forceinline__ auto raw(long i) const {
-    if constexpr (F32) return f[i];
-    else return d[i];
-  }
-  template <bool F32>
-  __device__ __forceinline__ double2 at(long i) const {
-    const auto v = raw<F32>(i);
-    return make_double2(v.x, v.y);
-  }
-};
-
-template <class V>
-__device__ __forceinline__ double2 widen(V v) {
-  return make_double2(v.x, v.y);
-}
-
-struct MArgs {
-  LIn lx, lz;
-  double2 *o1, *o3;
-  const double* tpts;  // [Pn][Ny]
-  int N, Ny, Pn;
-  long ncol;
-};
-
-template <bool F32>
-__device__ void mean_points_block(const MArgs& a) {
-  __shared__ double2 s1[260], s3[260];
-  for (int l = threadIdx.x; l <= a.N; l += blockDim.x) {
-    s1[l] = a.lx.at<F32>((long)l * a.ncol);
-    s3[l] = a.lz.at<F32>((long)l * a.ncol);
-  }
-  __syncthreads();
-  for (int jj = threadIdx.x; jj < a.Pn; jj += blockDim.x) {
-    double2 e1 = make_double2(0, 0), o1 = make_double2(0, 0);
-    double2 e3 = make_double2(0, 0), o3 = make_double2(0, 0);
-    for (int l = 0; l <= a.N; ++l) {
-      const double t = a.tpts[jj * a.Ny + l];
-      const double2 x1 = s1[l], x3 = s3[l];
-      if (l & 1) {
-        o1.x += t * x1.x; o1.y += t * x1.y;
-        o3.x += t * x3.x; o3.y += t * x3.y;
-      } else {
-        e1.x += t * x1.x; e1.y += t * x1.y;
-        e3.x += t * x3.x; e3.y += t * x3.y;
-      }
-    }
-    a.o1[jj] = make_double2(e1.x + o1.x, e1.y + o1.y);
-    a.o3[jj] = make_double2(e3.x + o3.x, e3.y + o3.y);
-    const int q = a.N - jj;
-    if (q != jj) {
-      a.o1[q] = make_double2(e1.x - o1.x, e1.y - o1.y);
-      a.o3[q] = make_double2(e3.x - o3.x, e3.y - o3.y);
-    }
-  }
-}
-
-
-struct HArgs {
-  LIn lx, ly, lz;
-  double2 *hv, *hg;
-  const double *al, *be;
-  int Mx, N;
-  long ncol;
-};
-
-// One thread per complex column; the derivative runs the backward recurrence
-// c_k b_k = b_{k+2} + 2 (k+1) a_{k+1}, which equals the reference's explicit
-// sum b_k = (2/c_k) sum_{j>k, j+k odd} j a_j.
-// The launch carries one extra block that computes the mean-mode Lamb point
-// values (mean_points_block) from the same coefficients.
-template <bool F32>
-__global__ __launch_bounds__(256) void k_hassemble(HArgs a, MArgs m) {
-  if (blockIdx.x == gridDim.x - 1) {
-    mean_points_block<F32>(m);
-    return;
-  }
-  const long cm = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cm >= a.ncol) return;
-  const int kz = (int)((unsigned)cm / (unsigned)a.Mx);
-  const int kx = (int)(cm - (long)kz * a.Mx);
-  const double al = a.al[kx], be = a.be[kz];
-  const double k2 = al * al + be * be;
-  const int N = a.N;
-  double2 bx2 = make_double2(0, 0), bx1 = make_double2(0, 0);
-  double2 bz2 = make_double2(0, 0), bz1 = make_double2(0, 0);
-  double2 lxn = make_double2(0, 0), lzn = make_double2(0, 0);  // a_{k+1}
-  for (int k0 = N; k0 >= 0; k0 -= 4) {
-    // loads issued four degrees ahead of the recurrence
-    decltype(a.lx.raw<F32>(0)) pl[4][3];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int k = k0 - t;
-      if (k >= 0) {
-        const long off = (long)k * a.ncol + cm;
-        pl[t][0] = a.lx.raw<F32>(off);
-        pl[t][1] = a.ly.raw<F32>(off);
-        pl[t][2] = a.lz.raw<F32>(off);
-      }
-    }
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int k = k0 - t;
-    if (k < 0) break;
-    const long off = (long)k * a.ncol + cm;
-    const double2 lx = widen(pl[t][0]), ly = widen(pl[t][1]), lz = widen(pl[t][2]);
-    double2 dx, dz;
-    if (k == N) {
-      dx = make_double2(0, 0);
-      dz = make_double2(0, 0);
-    } else {
-      const double f = 2.0 * (k + 1);
-      dx = make_double2(bx2.x + f * lxn.x, bx2.y + f * lxn.y);
-      dz = make_double2(bz2.x + f * lzn.x, bz2.y + f * lzn.y);
-    }
-    bx2 = bx1;
-    bx1 = dx;
-    bz2 = bz1;
-    bz1 = dz;
-    if (k == 0) {
-      dx.x *= 0.5;
-      dx.y *= 0.5;
-      dz.x *= 0.5;
-      dz.y *= 0.5;
-    }
-    // h_v = (k^2 L_y + i alpha D L_x) + i beta D L_z
-    double hvr = k2 * ly.x - al * dx.y;
-    double hvi = k2 * ly.y + al * dx.x;
-    hvr = hvr - be * dz.y;
-    hvi = hvi + be * dz.x;
-    // h_g = i alpha L_z - i beta L_x
-    const double hgr = -1.0 * al * lz.y + be * lx.y;
-    const double hgi = al * lz.x - be * lx.x;
-    a.hv[off] = make_double2(hvr, hvi);
-    a.hg[off] = make_double2(hgr, hgi);
-    lxn = lx;
-    lzn = lz;
-  }
-  }
-}
-
-hipError_t launch_hassemble(Ctx& c) {
-  HArgs a{};
-  const bool f32 = c.f32_fields;  // the analysis wrote L^n in FP32 (Lcf)
-  a.lx = LIn{c.Lc[0], f32 ? c.Lcf[0] : nullptr};
-  a.ly = LIn{c.Lc[1], f32 ? c.Lcf[1] : nullptr};
-  a.lz = LIn{c.Lc[2], f32 ? c.Lcf[2] : nullptr};
-  a.hv = c.hvc;
-  a.hg = c.hgc;
-  a.al = c.alpha;
-  a.be = c.beta;
-  a.Mx = c.d.Mx;
-  a.N = c.d.N;
-  a.ncol = c.d.ncol;
-  MArgs m{};
-  m.lx = a.lx;
-  m.lz = a.lz;
-  m.o1 = c.cl1[1 - c.hcur];
-  m.o3 = c.cl3[1 - c.hcur];
-  m.tpts = c.tpts;
-  m.N = c.d.N;
-  m.Ny = c.d.Ny;
-  m.Pn = c.d.Pn;
-  m.ncol = c.d.ncol;
-  const dim3 grid((unsigned)((a.ncol + kColumnThreads - 1) / kColumnThreads) + 1);
-  if (f32)
-    hipLaunchKernelGGL(k_hassemble<true>, grid, dim3(kColumnThreads), 0, c.stream, a, m);
-  else
-    hipLaunchKernelGGL(k_hassemble<false>, grid, dim3(kColumnThreads), 0, c.stream, a, m);
-  return hipGetLastError();
-}
-
-// Mean-mode Lamb (column (0,0) of L_x and L_z) -> values at the N+1 points
-// (PF:1592-1609), written into the "new" history slot.
 
 }  // namespace chf

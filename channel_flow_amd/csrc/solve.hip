@@ -1,8 +1,7 @@
 // Per-(kx,|kz|) solves of the v and omega_y equations with stored inverses
 // (PF:242-394; the path taken when the diagonalised operators of hsolve.hip do
-// not verify), with their mean mode (PF:401-474), the kinematics
-// (getvelocityandvorticity PF:2347-2407), and the GPU set-up of the operator
-// inverses (PF:181-204).
+// not verify), with their mean mode (PF:401-474), and the GPU set-up of the
+// operator inverses (PF:181-204).
 //
 // The collocation operators of get_coef_v (PF:3348-3381) and get_coef_omegay
 // (PF:3432-3455) depend on (kx, kz) through k^2 only, so the modes +kz and
@@ -402,176 +401,6 @@ __global__ __launch_bounds__(512) void k_solve(SolveArgs a) {
   }
 }
 
-// ------------------------------------------------------------- kinematics
-
-// getvelocityandvorticity (PF:2347-2407) for every mode with k^2 != 0:
-//   u = (i alpha Dv - i beta omega_y)/k^2,  w = (i beta Dv + i alpha omega_y)/k^2,
-//   omega_x = Dw - i beta v,                omega_z = -Du + i alpha v,
-// and for the mean mode (PF:435-438, 469-472) u = U, w = W, omega_z = -DU,
-// omega_x = DW.  D is the coefficient-space derivative of dz (PF:570-599),
-// b_k = b_{k+2} + 2(k+1) a_{k+1}, b_0 halved.
-//
-// The recurrences split into two independent chains by degree parity: chain q
-// reads v at degrees of parity q and omega_y at parity 1-q, and produces
-// Dv, u, w at parity 1-q and Du, Dw, omega_x, omega_z at parity q.  One thread
-// runs one chain of one mode, backwards over the degree, with its loads issued
-// eight degrees ahead.  Its outputs are stored non-temporally: the next
-// kernels read them, this one does not (the padded synthesis that reads u, w,
-// omega_x, omega_z runs 5% faster, this pass 3% slower).
-//
-// The same pass forms the explicit-operator brackets of the next solve's
-// right-hand sides (get_coef_rhs / get_rhs_omegay, PF:252-257, 335-340):
-//   g_v = c D^4 v + (1 - 2 c k^2) D^2 v - k^2 (1 - c k^2) v   (at parity q)
-//   g_w = c D^2 omega_y + (1 - c k^2) omega_y                  (at parity 1-q)
-// whose chains read the same v and omega_y degrees as chain q.
-struct KinArgs {
-  const double2 *v, *oy, *au0, *w0;
-  double2 *u, *w, *ox, *oz;
-  float2 *uf, *wf, *oxf, *ozf;  // F32: u, w, omega_x, omega_z rounded to FP32, written instead
-  double2 *gv, *go;  // brackets for the next solve
-  const double *al, *be;
-  int* nonfinite;    // set to 1 when v, omega_y, U or W hold a NaN or an infinity
-  int Mx, Mz, N, Ny;
-  long ncol;
-  double c;          // dt / (2 re)
-};
-
-// u, w, omega_x, omega_z at one offset: FP64, or (F32) rounded to FP32
-template <bool F32>
-__device__ __forceinline__ void kin_store(const KinArgs& a, int which, long off, double2 v) {
-  if constexpr (F32) {
-    float2* p = which == 0 ? a.uf : which == 1 ? a.wf : which == 2 ? a.oxf : a.ozf;
-    st_nt(p + off, make_float2((float)v.x, (float)v.y));
-  } else {
-    double2* p = which == 0 ? a.u : which == 1 ? a.w : which == 2 ? a.ox : a.oz;
-    st_nt(p + off, v);
-  }
-}
-
-template <bool F32>
-__global__ __launch_bounds__(256) void k_kinematics(KinArgs a) {
-  const int q = blockIdx.y;  // chain: parity of the v degrees it reads
-  const int N = a.N;
-  if (blockIdx.x == gridDim.x - 1) {
-    // mean mode, one block: U, W staged in LDS, derivatives by lanes 0..3
-    if (q != 0) return;
-    extern __shared__ double sm[];
-    double* x = sm;              // U.re U.im W.re W.im   [4][Ny]
-    double* d = sm + 4 * a.Ny;   // DU.re DU.im DW.re DW.im
-    bool finite = true;
-    for (int k = threadIdx.x; k < a.Ny; k += blockDim.x) {
-      const double2 U = a.au0[k], W = a.w0[k];
-      x[0 * a.Ny + k] = U.x; x[1 * a.Ny + k] = U.y; x[2 * a.Ny + k] = W.x; x[3 * a.Ny + k] = W.y;
-      finite = finite && isfinite(U.x) && isfinite(U.y) && isfinite(W.x) && isfinite(W.y);
-    }
-    if (!finite) a.nonfinite[0] = 1;
-    __syncthreads();
-    if (threadIdx.x < 4) {
-      const double* xa = x + threadIdx.x * a.Ny;
-      double* b = d + threadIdx.x * a.Ny;
-      double b2 = 0.0, b1 = 0.0;
-      b[N] = 0.0;
-      for (int k = N - 1; k >= 0; --k) {
-        const double bk = b2 + 2.0 * (k + 1) * xa[k + 1];
-        b2 = b1;
-        b1 = bk;
-        b[k] = (k == 0) ? 0.5 * bk : bk;
-      }
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < a.Ny; k += blockDim.x) {
-      const long off = (long)k * a.ncol;
-      kin_store<F32>(a, 0, off, make_double2(x[0 * a.Ny + k], x[1 * a.Ny + k]));
-      kin_store<F32>(a, 1, off, make_double2(x[2 * a.Ny + k], x[3 * a.Ny + k]));
-      kin_store<F32>(a, 3, off, make_double2(-1.0 * d[0 * a.Ny + k], -1.0 * d[1 * a.Ny + k]));
-      kin_store<F32>(a, 2, off, make_double2(d[2 * a.Ny + k], d[3 * a.Ny + k]));
-    }
-    return;
-  }
-  const long cm = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cm >= a.ncol || cm == 0) return;
-  const int kz = (int)((unsigned)cm / (unsigned)a.Mx);
-  const int kx = (int)(cm - (long)kz * a.Mx);
-  if (kz == a.Mz / 2) return;  // span Nyquist: never solved, stays zero (PF:247)
-  const double al = a.al[kx], be = a.be[kz];
-  const double k2 = al * al + be * be;
-  double2 vp = make_double2(0, 0);                    // v_{k+1}
-  double2 dv2 = make_double2(0, 0);                   // Dv_{k+2} (unhalved)
-  double2 up = make_double2(0, 0), wp = make_double2(0, 0);    // u_{k+1}, w_{k+1}
-  double2 du2 = make_double2(0, 0), dw2 = make_double2(0, 0);  // Du_{k+2}, Dw_{k+2}
-  // bracket chains: latest unhalved D^2 v, D^3 v, D^4 v, D omega, D^2 omega and omega_{k+1}
-  double2 d2s = make_double2(0, 0), d3s = make_double2(0, 0), d4s = make_double2(0, 0);
-  double2 e1s = make_double2(0, 0), e2s = make_double2(0, 0), wn = make_double2(0, 0);
-  const double cc = a.c, c2 = 1.0 - 2.0 * cc * k2, c0 = k2 * (1.0 - cc * k2), cw = 1.0 - cc * k2;
-  // x * 0 is 0 for every finite x and NaN for a NaN or an infinity: one
-  // multiply-add per value, no branch between the batched loads
-  double probe = 0.0;
-  for (int k0 = N; k0 >= 0; k0 -= 8) {
-    double2 in[8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int k = k0 - s;
-      if (k >= 0) in[s] = (((k & 1) == q) ? a.v : a.oy)[(long)k * a.ncol + cm];
-    }
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int k = k0 - s;
-      if (k < 0) break;
-      const long off = (long)k * a.ncol + cm;
-      const double f = 2.0 * (k + 1);
-      if ((k & 1) == q) {
-        // Du_k, Dw_k from u_{k+1}, w_{k+1}; omega_x, omega_z with v_k
-        double2 du = make_double2(du2.x + f * up.x, du2.y + f * up.y);
-        double2 dw = make_double2(dw2.x + f * wp.x, dw2.y + f * wp.y);
-        du2 = du;
-        dw2 = dw;
-        if (k == 0) {
-          du.x *= 0.5; du.y *= 0.5; dw.x *= 0.5; dw.y *= 0.5;
-        }
-        const double2 vk = in[s];
-        kin_store<F32>(a, 2, off, make_double2(dw.x + be * vk.y, dw.y - be * vk.x));
-        kin_store<F32>(a, 3, off, make_double2(-du.x - al * vk.y, -du.y + al * vk.x));
-        // brackets: D^2 v, D^4 v at k from D v, D^3 v at k+1; D omega at k from omega_{k+1}
-        double2 q2 = make_double2(d2s.x + f * dv2.x, d2s.y + f * dv2.y);
-        double2 q4 = make_double2(d4s.x + f * d3s.x, d4s.y + f * d3s.y);
-        e1s = make_double2(e1s.x + f * wn.x, e1s.y + f * wn.y);
-        d2s = q2;
-        d4s = q4;
-        if (k == 0) {
-          q2.x *= 0.5; q2.y *= 0.5; q4.x *= 0.5; q4.y *= 0.5;
-        }
-        st_nt(&a.gv[off], make_double2(cc * q4.x + c2 * q2.x - c0 * vk.x, cc * q4.y + c2 * q2.y - c0 * vk.y));
-        vp = vk;
-      } else {
-        // Dv_k from v_{k+1}; u_k, w_k with omega_y_k
-        double2 dv = make_double2(dv2.x + f * vp.x, dv2.y + f * vp.y);
-        dv2 = dv;
-        if (k == 0) {
-          dv.x *= 0.5; dv.y *= 0.5;
-        }
-        const double omr = in[s].x, omi = in[s].y;
-        const double2 uk = make_double2(-1.0 * al * dv.y / k2 + be * omi / k2, al * dv.x / k2 - be * omr / k2);
-        const double2 wk = make_double2(-1.0 * dv.y * be / k2 - 1.0 * omi * al / k2, be * dv.x / k2 + al * omr / k2);
-        kin_store<F32>(a, 0, off, uk);
-        kin_store<F32>(a, 1, off, wk);
-        up = uk;
-        wp = wk;
-        // brackets: D^3 v at k from D^2 v at k+1; D^2 omega at k from D omega at k+1
-        d3s = make_double2(d3s.x + f * d2s.x, d3s.y + f * d2s.y);
-        double2 r2 = make_double2(e2s.x + f * e1s.x, e2s.y + f * e1s.y);
-        e2s = r2;
-        if (k == 0) {
-          r2.x *= 0.5; r2.y *= 0.5;
-        }
-        st_nt(&a.go[off], make_double2(cc * r2.x + cw * omr, cc * r2.y + cw * omi));
-        wn = in[s];
-      }
-      probe = fma(in[s].x, 0.0, fma(in[s].y, 0.0, probe));
-    }
-  }
-  if (probe != probe) a.nonfinite[0] = 1;
-}
-
 // v from the solve's per-group records (record g = |kz| Mx + kx holds
 // [l][side], side 0 for kz = |kz|, 1 for kz = Mz - |kz|) into the field layout
 // [l][kz][kx].  Block = one |kz| and VL degrees: it reads the 256-byte record
@@ -674,47 +503,6 @@ hipError_t launch_solve(Ctx& c) {
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_vtranspose(c);
-}
-
-hipError_t launch_kinematics(Ctx& c, bool f32) {
-  if (f32 && !c.uf) return hipErrorInvalidValue;
-  const Dims& d = c.d;
-  KinArgs a{};
-  a.uf = c.uf;
-  a.wf = c.wf;
-  a.oxf = c.oxf;
-  a.ozf = c.ozf;
-  a.v = c.v;
-  a.oy = c.oy;
-  a.au0 = c.au0;
-  a.w0 = c.w0;
-  a.u = c.u;
-  a.w = c.w;
-  a.ox = c.ox;
-  a.oz = c.oz;
-  a.gv = c.gv;
-  a.go = c.go;
-  a.al = c.alpha;
-  a.be = c.beta;
-  a.nonfinite = c.nonfinite;
-  a.Mx = d.Mx;
-  a.Mz = d.Mz;
-  a.N = d.N;
-  a.Ny = d.Ny;
-  a.ncol = d.ncol;
-  a.c = c.prm.dt * 0.5 / c.prm.re;
-  const unsigned nb = (unsigned)((d.ncol + kColumnThreads - 1) / kColumnThreads) + 1;  // + the mean-mode block
-  const size_t shm = sizeof(double) * 8ull * d.Ny;
-  const void* k = f32 ? (const void*)k_kinematics<true> : (const void*)k_kinematics<false>;
-  if (shm > 65536) {
-    hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    if (e != hipSuccess) return e;
-  }
-  if (f32)
-    hipLaunchKernelGGL(k_kinematics<true>, dim3(nb, 2), dim3(kColumnThreads), shm, c.stream, a);
-  else
-    hipLaunchKernelGGL(k_kinematics<false>, dim3(nb, 2), dim3(kColumnThreads), shm, c.stream, a);
-  return hipGetLastError();
 }
 
 }  // namespace chf
