@@ -167,7 +167,8 @@ void free_all(Ctx* c) {
   f(c->tmean);
   for (int i = 0; i < 3; ++i) { f(c->phys_c[i]); f(c->phys_r[i]); }
   f(c->stats_part); f(c->stats); f(c->twxu); f(c->twzu); f(c->twx); f(c->twz); f(c->twy); f(c->costab);
-  f(c->gv); f(c->go); f(c->nonfinite);
+  f(c->gv); f(c->go);
+  if (c->nonfinite) (void)hipHostFree(c->nonfinite);
   for (hipEvent_t e : c->event_pool) (void)hipEventDestroy(e);
   c->event_pool.clear();
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
@@ -292,8 +293,8 @@ int autotune(Ctx* c) {
                     return launch_synth_points_h(*c, hc, ho, 2);
                   }});
   if (!c->twy) {
-    st.push_back({K_RHS_V, [c] { return launch_rhs(*c, 0); }});
-    st.push_back({K_RHS_O, [c] { return launch_rhs(*c, 1); }});
+    st.push_back({K_RHS_V, [c] { return launch_rhs(*c, 0, 1); }});
+    st.push_back({K_RHS_O, [c] { return launch_rhs(*c, 1, 1); }});
   }
   hipEvent_t e0 = nullptr, e1 = nullptr;
   CHF_TRY(hipEventCreate(&e0));
@@ -404,7 +405,8 @@ int build(Ctx* c, DegreeCache& cache) {
   for (double2** q : {&c->rvE, &c->rvO, &c->roE, &c->roO}) CHF_TRY(dalloc(c, q, (size_t)d.ne * d.ncol));
   CHF_TRY(dalloc(c, &c->gv, fld));
   CHF_TRY(dalloc(c, &c->go, fld));
-  CHF_TRY(dalloc(c, &c->nonfinite, 1));
+  CHF_TRY(hipHostMalloc((void**)&c->nonfinite, sizeof(int), hipHostMallocDefault));
+  *c->nonfinite = 0;
 
   // wavenumbers (PF:123-134, id = 0)
   std::vector<double> al(d.Mx), be(d.Mz);
@@ -596,7 +598,6 @@ int build(Ctx* c, DegreeCache& cache) {
     CHF_TRY(hipMemsetAsync(q, 0, fld * sizeof(double2), c->stream));
   for (double2* q : {c->cl1[0], c->cl1[1], c->cl3[0], c->cl3[1], c->au0, c->w0})
     CHF_TRY(hipMemsetAsync(q, 0, d.Ny * sizeof(double2), c->stream));
-  CHF_TRY(hipMemsetAsync(c->nonfinite, 0, sizeof(int), c->stream));
 
   // kernels that stage more than 64 KiB of LDS
   CHF_TRY(launch_setup_inverses(*c));
@@ -758,21 +759,19 @@ int nonlinear(Ctx* c, bool defer = true) {
 // nonlinear pass of the mixed form with the FFT transforms reads them
 int solve(Ctx* c, bool f32) {
   if (!c->diag) {
-    CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0); }));
-    CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1); }));
+    CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0, 1); }));
+    CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1, 1); }));
     CHF_TRY(timed(c, K_SOLVE, [&] { return launch_solve(*c); }));
-  } else if (!c->timing && c->overlap) {
-    // the omega_y path (right-hand side, solve) does not touch the v path's
-    // data until the kinematics: it runs on the side stream.  (With timing on,
-    // every launch runs alone so that each time is its own.)
-    CHF_TRY(on_two_streams(
-        c, [&] { const hipError_t e = launch_rhs(*c, 0); return e ? e : launch_hsolve(*c, 0); },
-        [&] { const hipError_t e = launch_rhs(*c, 1); return e ? e : launch_hsolve(*c, 1); }));
-  } else {
-    CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0); }));
-    CHF_TRY(timed(c, K_SOLVE, [&] { return launch_hsolve(*c, 0); }));
-    CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1); }));
-    CHF_TRY(timed(c, K_WSOLVE, [&] { return launch_hsolve(*c, 1); }));
+  } else if (!c->timing) {
+    // both equations in each launch (32x33x32 step 60 -> 51 us, 128x129x128 552 ->
+    // 540, 256x193x256 mixed 1866 -> 1844 against one launch each, on two streams there)
+    CHF_TRY(launch_rhs(*c, 0, 2));
+    CHF_TRY(launch_hsolve(*c, 0, 2));
+  } else {  // every launch alone, so that each time is its own
+    CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0, 1); }));
+    CHF_TRY(timed(c, K_SOLVE, [&] { return launch_hsolve(*c, 0, 1); }));
+    CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1, 1); }));
+    CHF_TRY(timed(c, K_WSOLVE, [&] { return launch_hsolve(*c, 1, 1); }));
   }
   c->hdefer = false;  // both right-hand-side kernels have formed h^n's point values
   CHF_TRY(timed(c, K_KINEMATICS, [&] { return launch_kinematics(*c, f32); }));
@@ -784,22 +783,20 @@ int solve(Ctx* c, bool f32) {
 // Waits for the context's work and reports a state that the last kinematics
 // pass found to hold a NaN or an infinity (v, omega_y, U or W).
 int check_finite(Ctx* c, const char* who) {
-  int flag = 0;
-  CHF_TRY(hipMemcpyAsync(&flag, c->nonfinite, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   CHF_TRY(hipStreamSynchronize(c->stream));
-  if (flag) {
+  if (*(volatile int*)c->nonfinite) {
     c->err = std::string(who) + ": the state is not finite (NaN or infinity in v, omega_y, U or W)";
     return CHF_NONFINITE;
   }
   return 0;
 }
 
-// A new v, omega_y, U, W: clear the non-finite flag, then derive u, w,
-// omega_x, omega_z and the next solve's right-hand-side brackets with the
-// kinematics pass that follows every solve.
+// A new v, omega_y, U, W: clear the non-finite flag (copy_arrays has waited for
+// the stream: no earlier pass still writes it), then derive u, w, omega_x,
+// omega_z and the next solve's right-hand-side brackets with the kinematics
+// pass that follows every solve.
 hipError_t load_kinematics(Ctx* c) {
-  hipError_t e = hipMemsetAsync(c->nonfinite, 0, sizeof(int), c->stream);
-  if (e != hipSuccess) return e;
+  *c->nonfinite = 0;
   c->f32_current = false;
   c->f64_stale = false;
   return launch_kinematics(*c);

@@ -396,16 +396,15 @@ static hipError_t rhs_syn(Ctx& c, const double2* g, const double2* hn, const dou
   return run_mfma_cos(c.stream, pb, 1, cb);
 }
 
-hipError_t launch_rhs(Ctx& c, int which) {
+hipError_t launch_rhs(Ctx& c, int first, int count) {
+  // FFT form (ydct.hip): the bracket's point values by the type-I DCT, and
+  // h^n's from its coefficients when they are not formed yet
+  if (c.twy) return launch_yrhs(c, first, count);
   const int nxt = c.hcur, prv = 1 - c.hcur;  // h^n, h^{n-1}
-  if (c.twy) {
-    // FFT form (ydct.hip): the bracket's point values by the type-I DCT, and
-    // h^n's from its coefficients when they are not formed yet
-    if (which == 0) return launch_yrhs(c, 0, c.gv, c.hdefer ? c.hvc : nullptr, c.hv[nxt], c.hv[prv], c.rvE, c.rvO);
-    return launch_yrhs(c, 1, c.go, c.hdefer ? c.hgc : nullptr, c.hg[nxt], c.hg[prv], c.roE, c.roO);
-  }
-  if (which == 0) return rhs_syn<2>(c, c.gv, c.hv[nxt], c.hv[prv], c.rvE, c.rvO);
-  return rhs_syn<1>(c, c.go, c.hg[nxt], c.hg[prv], c.roE, c.roO);
+  hipError_t e = hipSuccess;
+  if (first == 0) e = rhs_syn<2>(c, c.gv, c.hv[nxt], c.hv[prv], c.rvE, c.rvO);
+  if (e == hipSuccess && first + count == 2) e = rhs_syn<1>(c, c.go, c.hg[nxt], c.hg[prv], c.roE, c.roO);
+  return e;
 }
 
 }  // namespace chf

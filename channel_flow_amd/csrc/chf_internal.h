@@ -137,7 +137,8 @@ struct Ctx {
   // gv/go are written by the kinematics pass for the next solve (it runs after
   // every solve and whenever the state is replaced), so a resumed run forms
   // them with the same kernel as an uninterrupted one
-  // device flag: the last kinematics pass saw a NaN or an infinity in v,
+  // flag in pinned host memory, written by the device: a kinematics pass saw a
+  // NaN or an infinity in v,
   // omega_y, U or W (cleared when a new state is loaded)
   int* nonfinite = nullptr;
   // operators
@@ -244,10 +245,9 @@ int ydct_length_supported(int N);  // 1 when 2N has an FFT split
 hipError_t launch_ypoints(Ctx& c, const double2* const* in, double2* const* out, int nf);
 hipError_t launch_ysynth(Ctx& c, const double2* const* in, double2* const* out, int nf);
 hipError_t launch_yanalysis(Ctx& c, const double2* const* in, double2* const* out, int nf);
-// which: 0 = v, 1 = omega_y; hc != nullptr: h^n from its coefficients hc, its
-// point values written to hn; else hn holds them
-hipError_t launch_yrhs(Ctx& c, int which, const double2* g, const double2* hc, double2* hn, const double2* hp,
-                       double2* oE, double2* oO);
+// equations first .. first + count - 1 (0 = v, 1 = omega_y); h^n from its
+// coefficients, whose point values it writes, when they are pending (hdefer)
+hipError_t launch_yrhs(Ctx& c, int first, int count);
 hipError_t launch_ysynth32(Ctx& c, const double2* const* in, float2* const* out, int nf);
 hipError_t launch_ysynth32f(Ctx& c, const float2* const* in, float2* const* out, int nf);  // FP32 coefficients in
 hipError_t launch_yanalysis32f(Ctx& c, const float2* const* in, float2* const* out, int nf);  // FP32 coefficients out
@@ -264,11 +264,11 @@ int stats_splits(const Ctx& c);
 bool stats_in_lines(const Ctx& c);
 hipError_t launch_statistics(Ctx& c, const double2* const* fields, double2* const* work, double* const* phys,
                              double* part, double* out);
-hipError_t launch_rhs(Ctx& c, int which);  // 0 = v, 1 = omega_y
+hipError_t launch_rhs(Ctx& c, int first, int count);  // equations as launch_yrhs
 hipError_t launch_solve(Ctx& c);       // stored inverses: v, omega_y and the mean mode (k_solve, then launch_vtranspose)
 hipError_t launch_vtranspose(Ctx& c);  // v from the solve's per-group records to [Ny][Mz][Mx]
-// hsolve.hip: the diagonalised solves; 0 = v and the mean mode, 1 = omega_y
-hipError_t launch_hsolve(Ctx& c, int which);
+// hsolve.hip: the diagonalised solves; equation 0 = v and the mean mode, 1 = omega_y
+hipError_t launch_hsolve(Ctx& c, int first, int count);
 hipError_t launch_wall_setup(Ctx& c);
 // u, w, omega_x, omega_z (and the next RHS brackets) from v, omega_y, U, W;
 // f32: u, w, omega_x, omega_z into uf, wf, oxf, ozf (rounded to FP32) instead

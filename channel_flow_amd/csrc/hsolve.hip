@@ -26,8 +26,8 @@ struct HsArgs {
   const double2 *L[2], *V[2];  // per parity: packed A fragments (pack_pairs in api.hip)
   const double* vec[2];        // per parity: lam, w1, w2, l1, q, each [16 MB]
   const double* wall[2];       // per parity: [column][4], (d1, d2) -> (a, B)  (v)
-  const double2* rhs[2];       // per parity: folded right-hand sides [rows][ncol]
-  double* out;                 // v or omega_y, real view [Ny][2 ncol]
+  const double2* rhs[2][2];    // per equation (0 = v) and parity: folded right-hand sides [rows][ncol]
+  double* out[2];              // v, omega_y, real view [Ny][2 ncol]
   const double *al, *be;
   int m[2];
   int Mx, Mz;
@@ -109,18 +109,14 @@ constexpr int kHsThreads = 256;  // four wavefronts
 // equal work); below, one column block per wave and every row block, so no
 // wave idles.
 template <bool IS_V, int WR, int RB>
-__global__ __launch_bounds__(kHsThreads, RB == 4 ? 2 : 3) void k_hsolve(HsArgs a) {
+__device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
   using MF = Mf<double>;
   constexpr int CT = kHsCols, CB = WR;
-  extern __shared__ double sB[];  // [16 MB rows][CT], then the wall sums
   const int par = blockIdx.y;
-  int tile = blockIdx.x;
-  if constexpr (IS_V) {
-    if (tile == 0) {
-      if (par == 0) mean_mode_block(a, sB);
-      return;
-    }
-    --tile;
+  const int tile = (int)blockIdx.x - 1;
+  if (tile < 0) {
+    if (IS_V && par == 0) mean_mode_block(a, sB);
+    return;
   }
   const int m = par ? a.m[1] : a.m[0];
   const int MB = (m + 15) / 16, KP = (m + 7) / 8, R = 16 * MB;
@@ -134,7 +130,7 @@ __global__ __launch_bounds__(kHsThreads, RB == 4 ? 2 : 3) void k_hsolve(HsArgs a
   // stage B: matrix row r holds the right-hand side of point p = r + 1; rows
   // without one (v at p = 1, the padding) and columns past the end are zero
   {
-    const double2* ro = par ? a.rhs[1] : a.rhs[0];
+    const double2* ro = IS_V ? (par ? a.rhs[0][1] : a.rhs[0][0]) : (par ? a.rhs[1][1] : a.rhs[1][0]);
     constexpr int off = IS_V ? 1 : 0, SL = 6;
     const int nst = R * (CT / 2), last = m - 1 - off;
     for (int i0 = threadIdx.x; i0 < nst; i0 += SL * kHsThreads) {
@@ -297,7 +293,7 @@ __global__ __launch_bounds__(kHsThreads, RB == 4 ? 2 : 3) void k_hsolve(HsArgs a
   for (int cb = 0; cb < CB; ++cb) {
     const long col = 2 * col0 + cl + 16 * cb, cm = col >> 1;
     if (cm >= a.ncol || cm == 0 || (int)((unsigned)cm / (unsigned)a.Mx) == a.Mz / 2) continue;
-    double* o = a.out + (long)par * ncold + col;
+    double* o = (IS_V ? a.out[0] : a.out[1]) + (long)par * ncold + col;
     if (wr == 0 && lane < 16) {
       if constexpr (WR == 2) sum[cb] += red[2 * CT + cl + 16 * cb];
       o[0] = -sum[cb];
@@ -310,6 +306,14 @@ __global__ __launch_bounds__(kHsThreads, RB == 4 ? 2 : 3) void k_hsolve(HsArgs a
         if (row < m) o[2L * (row + 1) * ncold] = acc[t][cb][e];
       }
   }
+}
+
+// Both equations in one launch (first = 0, two layers), or one of them.
+template <int WR, int RB>
+__global__ __launch_bounds__(kHsThreads, RB == 4 ? 2 : 3) void k_hsolve(HsArgs a, int first) {
+  extern __shared__ double sB[];  // [16 MB rows][kHsCols], then the wall sums
+  if (first + blockIdx.z == 0) hsolve_block<true, WR, RB>(a, sB);
+  else hsolve_block<false, WR, RB>(a, sB);
 }
 
 // The wall matrices of every column and parity (wall_matrix of helmholtz.h).
@@ -370,44 +374,28 @@ hipError_t launch_wall_setup(Ctx& c) {
   return hipGetLastError();
 }
 
-template <bool IS_V, int WR, int RB>
-static hipError_t run_hsolve(Ctx& c, const HsArgs& a) {
+template <int WR, int RB>
+static hipError_t run_hsolve(Ctx& c, const HsArgs& a, int first, int count) {
   const size_t shm = sizeof(double) * ((size_t)kHsCols * 16 * ((a.m[0] + 15) / 16) + 5 * kHsCols);
-  const unsigned tiles = (unsigned)((2 * a.ncol + kHsCols - 1) / kHsCols) + (IS_V ? 1 : 0);  // + the mean-mode block
+  const unsigned tiles = (unsigned)((2 * a.ncol + kHsCols - 1) / kHsCols);
   if (sizeof(double) * 8ull * a.Ny > shm) return hipErrorInvalidValue;  // the mean-mode block's arrays
   if (shm > 65536) {
-    const hipError_t e = hipFuncSetAttribute((const void*)k_hsolve<IS_V, WR, RB>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+    const hipError_t e =
+        hipFuncSetAttribute((const void*)k_hsolve<WR, RB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_hsolve<IS_V, WR, RB>), dim3(tiles, 2), dim3(kHsThreads), shm, c.stream, a);
+  hipLaunchKernelGGL((k_hsolve<WR, RB>), dim3(tiles + 1, 2, count), dim3(kHsThreads), shm, c.stream, a, first);
   return hipGetLastError();
 }
 
-template <bool IS_V>
-static hipError_t launch_hs(Ctx& c, const HsArgs& a) {
-  switch ((a.m[0] + 15) / 16) {  // row blocks of the even half system (the odd one has as many or one less)
-    case 1: return run_hsolve<IS_V, 1, 1>(c, a);
-    case 2: return run_hsolve<IS_V, 1, 2>(c, a);
-    case 3: return run_hsolve<IS_V, 1, 3>(c, a);
-    case 4: return run_hsolve<IS_V, 2, 2>(c, a);
-    case 5: case 6: return run_hsolve<IS_V, 2, 3>(c, a);
-    case 7: case 8: return run_hsolve<IS_V, 2, 4>(c, a);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch_hsolve(Ctx& c, int which) {
+hipError_t launch_hsolve(Ctx& c, int first, int count) {
   HsArgs a = hs_args(c);
-  if (which == 1) {
-    a.rhs[0] = c.roE;
-    a.rhs[1] = c.roO;
-    a.out = reinterpret_cast<double*>(c.oy);
-    return launch_hs<false>(c, a);
-  }
-  a.rhs[0] = c.rvE;
-  a.rhs[1] = c.rvO;
-  a.out = reinterpret_cast<double*>(c.v);
+  a.rhs[0][0] = c.rvE;
+  a.rhs[0][1] = c.rvO;
+  a.rhs[1][0] = c.roE;
+  a.rhs[1][1] = c.roO;
+  a.out[0] = reinterpret_cast<double*>(c.v);
+  a.out[1] = reinterpret_cast<double*>(c.oy);
   a.au0 = c.au0;
   a.w0 = c.w0;
   a.c1n = c.cl1[c.hcur];
@@ -416,7 +404,15 @@ hipError_t launch_hsolve(Ctx& c, int which) {
   a.c3p = c.cl3[1 - c.hcur];
   a.tmean = c.tmean;
   a.inv0 = c.inv0;
-  return launch_hs<true>(c, a);
+  switch ((a.m[0] + 15) / 16) {  // row blocks of the even half system (the odd one has as many or one less)
+    case 1: return run_hsolve<1, 1>(c, a, first, count);
+    case 2: return run_hsolve<1, 2>(c, a, first, count);
+    case 3: return run_hsolve<1, 3>(c, a, first, count);
+    case 4: return run_hsolve<2, 2>(c, a, first, count);
+    case 5: case 6: return run_hsolve<2, 3>(c, a, first, count);
+    case 7: case 8: return run_hsolve<2, 4>(c, a, first, count);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace chf

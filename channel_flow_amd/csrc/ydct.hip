@@ -300,8 +300,8 @@ __global__ __launch_bounds__(YT<V>::TX* ymax(A1, A2)) void k_ycheb(YArgs a) {
   }
 }
 
-// Right-hand sides of the v (POFF = 2) and omega_y (POFF = 1) half systems
-// (PF:252-257, 335-340; the explicit operator as the bracket g formed by the
+// Right-hand sides of the v (equation 0, POFF = 2) and omega_y (1, POFF = 1) half
+// systems, both in one launch or one of them (PF:252-257, 335-340; the explicit operator as the bracket g formed by the
 // kinematics pass): f = sum_k g_k T_k at the Gauss-Lobatto points (the type-I
 // DCT, FP64), plus the AB2 forcing F = 3 dt/2 h^n - dt/2 h^(n-1), folded by
 // parity at the point pairs p = r + POFF, q = N - p: even row r
@@ -316,20 +316,27 @@ __global__ __launch_bounds__(YT<V>::TX* ymax(A1, A2)) void k_ycheb(YArgs a) {
 // end terms as k_ypoints, f + F in the step-B layout, the pairs from the LDS
 // tile), so a run that switches between them is bit-identical to one that
 // does not.
-struct YRhsArgs {
+struct YRhsEq {
   const double2* g;
   const double2* hc;  // FUSE: h^n coefficients
   double2* hn;        // h^n point values (FUSE: written, else read)
   const double2* hp;  // h^(n-1) point values
   double2 *outE, *outO;
+};
+struct YRhsArgs {
+  YRhsEq eq[2];
+  int first;  // equation of the launch's first layer
   long ncol;
   int ne, no;
   double dt;
   const double2* twL;
 };
 
-template <int N1, int N2, int POFF, bool FUSE>
-__global__ __launch_bounds__(YT<double2>::TX* ymax(N1, N2)) void k_yrhs(YRhsArgs a) {
+template <int N1, int N2, bool FUSE>
+__global__ __launch_bounds__(YT<double2>::TX* ymax(N1, N2)) void k_yrhs(YRhsArgs args) {
+  const bool isv = args.first + blockIdx.z == 0;
+  const YRhsEq a = isv ? args.eq[0] : args.eq[1];
+  const int POFF = isv ? 2 : 1;
   constexpr int L = N1 * N2, N = L / 2, TX = YT<double2>::TX, G = ymax(N1, N2);
   constexpr int SB = tile_stride<double2>(N1 * (N2 + 1));
   constexpr int KJ = N / N2 + 1;  // step-B outputs k1 with a point j = k1 N2 + t <= N
@@ -338,8 +345,8 @@ __global__ __launch_bounds__(YT<double2>::TX* ymax(N1, N2)) void k_yrhs(YRhsArgs
   const int t = threadIdx.x / TX, tx = threadIdx.x - t * TX;
   double2* buf = reinterpret_cast<double2*>(smraw) + tx * SB;
   const long col = xcd_order(blockIdx.x, gridDim.x) * TX + tx;
-  const long nc = a.ncol;
-  const double c1 = 1.5 * a.dt, c0 = 0.5 * a.dt;
+  const long nc = args.ncol;
+  const double c1 = 1.5 * args.dt, c0 = 0.5 * args.dt;
   // step A of the type-I DCT of the coefficient column src (threads t < N1)
   auto stepA = [&](const double2* src) {
     if (t < N1) {
@@ -349,7 +356,7 @@ __global__ __launch_bounds__(YT<double2>::TX* ymax(N1, N2)) void k_yrhs(YRhsArgs
         const int m = n2 * N1 + t;
         x[n2] = src[(long)(m <= N ? m : L - m) * nc + col];
       }
-      ystepA<N1, N2, -1>(x, buf, a.twL, t);
+      ystepA<N1, N2, -1>(x, buf, args.twL, t);
     }
   };
   // f_j = (S_j + a_0 + (-1)^j a_N) / 2 at j = k1 N2 + t, after step B
@@ -422,7 +429,7 @@ __global__ __launch_bounds__(YT<double2>::TX* ymax(N1, N2)) void k_yrhs(YRhsArgs
     }
   }
   __syncthreads();
-  const int Me = a.ne - POFF, Mo = a.no - POFF;
+  const int Me = args.ne - POFF, Mo = args.no - POFF;
   for (int r = t; r < Me; r += G) {
     const int p = r + POFF, q = N - p;
     const double2 vp = buf[p];
@@ -516,39 +523,33 @@ hipError_t launch_yanalysis(Ctx& c, const double2* const* in, double2* const* ou
   return run_ydct<double2>(c, 2, in, out, nf);
 }
 template <int N1, int N2>
-static hipError_t run_yrhs(Ctx& c, int which, bool fuse, const YRhsArgs& a) {
+static hipError_t run_yrhs(Ctx& c, int count, bool fuse, const YRhsArgs& a) {
   constexpr int TX = YT<double2>::TX, nt = TX * ymax(N1, N2);
   const size_t shm = sizeof(double2) * (size_t)TX * tile_stride<double2>(N1 * (N2 + 1));
-  if (which == 0)
-    return fuse ? launch_y(c, k_yrhs<N1, N2, 2, true>, TX, nt, shm, a, 1)
-                : launch_y(c, k_yrhs<N1, N2, 2, false>, TX, nt, shm, a, 1);
-  return fuse ? launch_y(c, k_yrhs<N1, N2, 1, true>, TX, nt, shm, a, 1)
-              : launch_y(c, k_yrhs<N1, N2, 1, false>, TX, nt, shm, a, 1);
+  return fuse ? launch_y(c, k_yrhs<N1, N2, true>, TX, nt, shm, a, count)
+              : launch_y(c, k_yrhs<N1, N2, false>, TX, nt, shm, a, count);
 }
 
-hipError_t launch_yrhs(Ctx& c, int which, const double2* g, const double2* hc, double2* hn, const double2* hp,
-                       double2* oE, double2* oO) {
+hipError_t launch_yrhs(Ctx& c, int first, int count) {
+  const int cur = c.hcur, prv = 1 - c.hcur;  // h^n, h^(n-1)
   YRhsArgs a{};
-  a.g = g;
-  a.hc = hc;
-  a.hn = hn;
-  a.hp = hp;
-  a.outE = oE;
-  a.outO = oO;
+  a.eq[0] = {c.gv, c.hvc, c.hv[cur], c.hv[prv], c.rvE, c.rvO};
+  a.eq[1] = {c.go, c.hgc, c.hg[cur], c.hg[prv], c.roE, c.roO};
+  a.first = first;
   a.ncol = c.d.ncol;
   a.ne = c.d.ne;
   a.no = c.d.no;
   a.dt = c.prm.dt;
   a.twL = c.twy;
-  const bool fuse = hc != nullptr;
+  const bool fuse = c.hdefer;
   switch (2 * c.d.N) {
-    case 64: return run_yrhs<8, 8>(c, which, fuse, a);
-    case 96: return run_yrhs<8, 12>(c, which, fuse, a);
-    case 128: return run_yrhs<8, 16>(c, which, fuse, a);
-    case 192: return run_yrhs<12, 16>(c, which, fuse, a);
-    case 256: return run_yrhs<16, 16>(c, which, fuse, a);
-    case 384: return run_yrhs<16, 24>(c, which, fuse, a);
-    case 512: return run_yrhs<16, 32>(c, which, fuse, a);
+    case 64: return run_yrhs<8, 8>(c, count, fuse, a);
+    case 96: return run_yrhs<8, 12>(c, count, fuse, a);
+    case 128: return run_yrhs<8, 16>(c, count, fuse, a);
+    case 192: return run_yrhs<12, 16>(c, count, fuse, a);
+    case 256: return run_yrhs<16, 16>(c, count, fuse, a);
+    case 384: return run_yrhs<16, 24>(c, count, fuse, a);
+    case 512: return run_yrhs<16, 32>(c, count, fuse, a);
     default: return hipErrorNotSupported;
   }
 }
