@@ -628,13 +628,18 @@ constexpr int xpass_buffers() {
   return (sizeof(V) == 16 && W == 64 && L / RA <= 64 && L / RB <= 64) ? 1 : 2;
 }
 
-// Streamwise pass, W threads per (y point, span point) line (one wavefront, or
-// two), for L = RA RB RC with L / RC <= W and Mx = L / 3 spectral points per
+// Streamwise pass, W threads per (y point, span point) line (a wavefront, two,
+// or a half or a quarter of one), for L = RA RB RC with L / RC <= W and Mx = L / 3 spectral points per
 // row.  The threads of a line first read its six input rows into registers (all
 // loads in flight at once), then run the inverse transforms through the line's
-// own LDS buffers; one wavefront needs wave-level ordering only, so the waves of
-// a block never wait for each other, two take the block's barrier (one line per
-// block).  The inverse transforms run the stages RA, RB, RC; the last one leaves
+// own LDS buffers; lines within a wavefront need wave-level ordering only, so the
+// waves of a block never wait for each other, two wavefronts take the block's
+// barrier (one line per block).  A stage keeps L / R of a line's W threads busy,
+// so short lines share a wavefront (us, a wavefront per line or a group of
+// threads with block barriers / lines sharing a wavefront: 192 points FP64
+// 128x129x128 192 / 154, FP32 128x97x128 79 / 56; 288 FP64 192x161x192 476 / 456;
+// 216 FP64 144x97x96 133 / 118; 96 FP32 20.7 / 17.2; 48 13.6 / 9.1).  Slower so,
+// and left as they are: 384 FP32 369 / 450 (registers), 144 and 96 FP64.  The inverse transforms run the stages RA, RB, RC; the last one leaves
 // thread j < L / RC holding the physical points j + r L / RC (r < RC) of every
 // field, so the six products form the Lamb vector in registers, and the forward
 // transforms start with a radix-RC stage on exactly those points (Ns = 1, no
@@ -644,13 +649,13 @@ template <int L, int RA, int RB, int RC, int NL, int W, class V>
 __global__ __launch_bounds__(W* NL) void k_xpass_st(RegX<V> a) {
   constexpr int LC = L / RC;            // threads that hold points
   static_assert(L == RA * RB * RC && LC <= W && L % 3 == 0, "one group of threads per line");
-  static_assert(W == 64 || NL == 1, "the lines of a block share no barrier");
+  static_assert(W <= 64 || NL == 1, "the lines of a block share no barrier");
   using T = decltype(V{}.x);
   constexpr int PL = L + (L >> 3) + 1;  // padded buffer length
   constexpr int MX = L / 3;             // spectral points per row
   constexpr int MP = (MX + W - 1) / W;  // of them per thread
   auto line_sync = [] {
-    if constexpr (W == 64) wave_sync();
+    if constexpr (W <= 64) wave_sync();
     else __syncthreads();
   };
   extern __shared__ __align__(16) unsigned char smraw[];
@@ -819,7 +824,7 @@ __global__ __launch_bounds__(W* NL) void k_xpass_st(RegX<V> a) {
 template <int L, int RA, int RB, int RC, int W = 64, class V>
 static hipError_t run_xpass_st(Ctx& c, const RegX<V>& a) {
   if (a.Mx * 3 != L) return hipErrorInvalidValue;  // the kernel's row length is L / 3
-  constexpr int NL = W > 64 ? 1 : sizeof(V) == 16 ? 2 : 4;  // lines per block
+  constexpr int NL = W > 64 ? 1 : (sizeof(V) == 16 ? 128 : 256) / W;  // lines per block
   constexpr int PL = L + (L >> 3) + 1;
   constexpr int NB = xpass_buffers<L, RA, RB, W, V>();
   const long blocks = (a.nlines + NL - 1) / NL;
@@ -1025,8 +1030,8 @@ static hipError_t xpass_reg(Ctx& c, const RegX<V>& a) {
       case 72: return run_xpass_reg<8, 9>(c, a);
       case 108: return run_xpass_reg<9, 12>(c, a);
       case 162: return run_xpass_reg<9, 18>(c, a);
-      case 216: return run_xpass_st<216, 6, 9, 4>(c, a);
-      case 288: return run_xpass_st<288, 8, 6, 6>(c, a);
+      case 216: return run_xpass_st<216, 6, 4, 9, 32>(c, a);
+      case 288: return run_xpass_st<288, 8, 4, 9, 32>(c, a);
       case 324: return run_xpass_st<324, 9, 6, 6>(c, a);
       case 432: return run_xpass_st<432, 9, 6, 8>(c, a);
       case 576: return run_xpass_st<576, 8, 12, 6, 128>(c, a);
@@ -1037,10 +1042,12 @@ static hipError_t xpass_reg(Ctx& c, const RegX<V>& a) {
   switch (c.d.Lx) {
     case 12: return run_xpass_reg<4, 3>(c, a);
     case 24: return run_xpass_reg<4, 6>(c, a);
-    case 48: return run_xpass_reg<6, 8>(c, a);
-    case 96: return run_xpass_reg<8, 12>(c, a);
+    case 48: return run_xpass_st<48, 4, 4, 3, 16>(c, a);
+    case 96:
+      if constexpr (sizeof(V) == 8) return run_xpass_st<96, 8, 4, 3, 32>(c, a);
+      else return run_xpass_reg<8, 12>(c, a);
     case 144: return run_xpass_reg<12, 12>(c, a);
-    case 192: return run_xpass_st<192, 8, 8, 3>(c, a);
+    case 192: return run_xpass_st<192, 8, 4, 6, 32>(c, a);
     case 384: return run_xpass_st<384, 8, 8, 6>(c, a);
     case 768:
       if constexpr (sizeof(V) == 8) return run_xpass_st<768, 8, 8, 12>(c, a);
