@@ -694,9 +694,9 @@ hipError_t analysis32_fields(Ctx* c, const float2* const* y3, int f0, int nf) {
   return launch_analysis32(*c, y3 + f0, c->Lc + f0, nf);
 }
 
-// defer: with the FFT transforms, leave h^n's point values to the next
-// solve's right-hand-side kernels (the ensemble's graphs form them here).
-int nonlinear(Ctx* c, bool defer = true) {
+// With the FFT transforms h^n's point values are left to the next solve's
+// right-hand-side kernels.
+int nonlinear(Ctx* c) {
   CHF_TRY(form_h_points(c));  // the previous step's, before the h assembly overwrites hvc, hgc
   // six fields in the order the streamwise pass pairs them: (u,v) (w,ox) (oy,oz)
   const double2* in6[6] = {c->u, c->v, c->w, c->ox, c->oy, c->oz};
@@ -744,7 +744,7 @@ int nonlinear(Ctx* c, bool defer = true) {
   }
   CHF_TRY(timed(c, K_HASSEMBLE, [&] { return launch_hassemble(*c); }));
   const int nxt = 1 - c->hcur;
-  if (defer && c->twy) {
+  if (c->twy) {
     c->hdefer = true;
   } else {
     const double2* hc[2] = {c->hvc, c->hgc};
@@ -755,9 +755,10 @@ int nonlinear(Ctx* c, bool defer = true) {
   return 0;
 }
 
-// f32: the kinematics writes u, w, omega_x, omega_z in FP32 only, as the next
-// nonlinear pass of the mixed form with the FFT transforms reads them
-int solve(Ctx* c, bool f32) {
+int solve(Ctx* c) {
+  // the mixed form with the FFT transforms keeps u, w, omega_x, omega_z in
+  // FP32 only, as the next nonlinear pass reads them
+  const bool f32 = c->f32_fields;
   if (!c->diag) {
     CHF_TRY(timed(c, K_RHS_V, [&] { return launch_rhs(*c, 0, 1); }));
     CHF_TRY(timed(c, K_RHS_O, [&] { return launch_rhs(*c, 1, 1); }));
@@ -931,7 +932,7 @@ int chf_nonlinear(void* ctx) {
 int chf_solve(void* ctx) {
   if (!ctx) return -1;
   Ctx* c = static_cast<Ctx*>(ctx);
-  const int rc = solve(c, c->f32_fields);
+  const int rc = solve(c);
   return rc ? rc : check_finite(c, "chf_solve");
 }
 
@@ -940,7 +941,7 @@ int chf_step(void* ctx, int n) {
   Ctx* c = static_cast<Ctx*>(ctx);
   if (n < 0) return fail(c, "chf_step: negative step count");
   for (int i = 0; i < n; ++i) {
-    int rc = solve(c, c->f32_fields);
+    int rc = solve(c);
     if (rc) return rc;
     rc = nonlinear(c);
     if (rc) return rc;
@@ -1135,13 +1136,14 @@ int chf_timing(void* ctx, int id, double* total_ms, int* launches) {
 // advanced together.  One step of all members is one hipGraph launch whose
 // parallel branches are the members' steps (each member on its own stream,
 // forked from and joined to the ensemble stream).  Small members fill the GPU
-// together.  The AB2 history buffers swap every step, so a graph is captured per
-// combination of the members' history phases (normally two) and cached.
+// together.  The AB2 history buffers swap every step, and the first step after a
+// record is loaded finds h^n's point values formed, so a graph is captured per
+// combination of the members' phases (normally two) and cached.
 
 namespace {
 
 struct EnsGraph {
-  std::vector<int> phase;         // members' history phases the graph was captured at
+  std::vector<int> phase;         // members' phases the graph was captured at
   hipGraphExec_t exec = nullptr;
 };
 
@@ -1182,11 +1184,31 @@ void ens_free(Ens* e) {
   if (e->origin) (void)hipStreamDestroy(e->origin);
 }
 
-// Captures one step of every member into g; member host state (history phase)
-// is restored afterwards, the caller advances it per launch.
+// What a captured step depends on: the history buffers in use and whether h^n's
+// point values are pending.
+int step_phase(const Ctx* c) { return c->hcur | (c->hdefer ? 2 : 0); }
+
+// The host state that a launch of a captured step leaves, as solve() and
+// nonlinear() do.
+void step_done(Ctx* c) {
+  c->hcur = 1 - c->hcur;
+  c->hdefer = c->twy != nullptr;
+  c->f32_current = c->f64_stale = c->f32_fields;
+}
+
+// Captures one step of every member into g; member host state is restored
+// afterwards, the caller advances it per launch.
 int ens_capture(Ens* e, EnsGraph* g) {
   const int n = (int)e->m.size();
-  for (Ctx* c : e->m) g->phase.push_back(c->hcur);
+  struct Host {
+    int hcur;
+    bool hdefer, f32_current, f64_stale;
+  };
+  std::vector<Host> host;
+  for (Ctx* c : e->m) {
+    g->phase.push_back(step_phase(c));
+    host.push_back({c->hcur, c->hdefer, c->f32_current, c->f64_stale});
+  }
   ENS_TRY(hipStreamBeginCapture(e->origin, hipStreamCaptureModeRelaxed));
   int rc = 0;
   std::string what;
@@ -1195,8 +1217,8 @@ int ens_capture(Ens* e, EnsGraph* g) {
     Ctx* c = e->m[i];
     he = hipStreamWaitEvent(c->stream, e->fork, 0);
     if (he != hipSuccess) break;
-    rc = solve(c, false);
-    if (rc == 0) rc = nonlinear(c, false);
+    rc = solve(c);
+    if (rc == 0) rc = nonlinear(c);
     if (rc) {
       what = c->err;
       break;
@@ -1206,7 +1228,13 @@ int ens_capture(Ens* e, EnsGraph* g) {
   }
   hipGraph_t graph = nullptr;
   const hipError_t ee = hipStreamEndCapture(e->origin, &graph);
-  for (int i = 0; i < n; ++i) e->m[i]->hcur = g->phase[i];
+  for (int i = 0; i < n; ++i) {
+    Ctx* c = e->m[i];
+    c->hcur = host[i].hcur;
+    c->hdefer = host[i].hdefer;
+    c->f32_current = host[i].f32_current;
+    c->f64_stale = host[i].f64_stale;
+  }
   if (rc) {
     if (graph) (void)hipGraphDestroy(graph);
     return ens_fail(e, "capture of a member step failed: " + what, rc);
@@ -1306,14 +1334,12 @@ int chf_ensemble_step(void* ens, int n) {
   if (n < 0) return ens_fail(e, "chf_ensemble_step: negative step count");
   for (Ctx* c : e->m) {
     if (c->timing) return ens_fail(e, "chf_ensemble_step: turn member timing off first");
-    // the graphs form h^n's point values in nonlinear(): pending ones first
-    ENS_TRY(form_h_points(c));
     // member work queued outside the graph (set_state, init) must finish first
     ENS_TRY(hipStreamSynchronize(c->stream));
   }
   for (int s = 0; s < n; ++s) {
     std::vector<int> phase;
-    for (Ctx* c : e->m) phase.push_back(c->hcur);
+    for (Ctx* c : e->m) phase.push_back(step_phase(c));
     hipGraphExec_t exec = nullptr;
     for (auto& g : e->graphs)
       if (g.phase == phase) exec = g.exec;
@@ -1328,7 +1354,7 @@ int chf_ensemble_step(void* ens, int n) {
       e->graphs.push_back(g);
     }
     ENS_TRY(hipGraphLaunch(exec, e->origin));
-    for (Ctx* c : e->m) c->hcur = 1 - c->hcur;  // what nonlinear() does per step
+    for (Ctx* c : e->m) step_done(c);
   }
   ENS_TRY(hipStreamSynchronize(e->origin));
   for (size_t i = 0; i < e->m.size(); ++i) {
