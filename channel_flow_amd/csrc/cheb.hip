@@ -305,7 +305,6 @@ hipError_t launch_analysis(Ctx& c, const double2* const* in, double2* const* out
 
 // Mixed form: FP32 values on the padded grid -> FP64 coefficients, FP32 matrix cores.
 hipError_t launch_analysis32(Ctx& c, const float2* const* in, double2* const* out, int nf) {
-  if (c.twy) return launch_yanalysis32(c, in, out, nf);
   const float* ri[6];
   for (int i = 0; i < nf; ++i) ri[i] = reinterpret_cast<const float*>(in[i]);
   return analysis_t<float, float>(c, c.costabf, ri, out, nf);

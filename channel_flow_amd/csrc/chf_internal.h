@@ -251,7 +251,6 @@ hipError_t launch_yrhs(Ctx& c, int first, int count);
 hipError_t launch_ysynth32(Ctx& c, const double2* const* in, float2* const* out, int nf);
 hipError_t launch_ysynth32f(Ctx& c, const float2* const* in, float2* const* out, int nf);  // FP32 coefficients in
 hipError_t launch_yanalysis32f(Ctx& c, const float2* const* in, float2* const* out, int nf);  // FP32 coefficients out
-hipError_t launch_yanalysis32(Ctx& c, const float2* const* in, double2* const* out, int nf);
 hipError_t launch_synth_points_h(Ctx& c, const double2* const* in, double2* const* out, int nf);  // FP32 compute in the mixed form
 hipError_t launch_span_inverse_unpadded(Ctx& c, double2* const* inout, int nf);
 hipError_t launch_stream_c2r_lds(Ctx& c, const double2* in, double* out);

@@ -179,15 +179,43 @@ struct Dft<4, S, V> {
   }
 };
 
+template <int S, class V>
+struct Dft<5, S, V> {
+  static __host__ __device__ __forceinline__ void run(V* v) {
+    using T = decltype(v[0].x);
+    const T c1 = (T)0.30901699437494742410, c2 = (T)-0.80901699437494742410;  // cos 72, cos 144 degrees
+    const T s1 = (T)0.95105651629515357212 * (T)S, s2 = (T)0.58778525229247312917 * (T)S;
+    const V a = cadd(v[1], v[4]), b = cadd(v[2], v[3]), c = csub(v[1], v[4]), d = csub(v[2], v[3]);
+    V e, f, g, h;  // X_1, X_4 = e +- i g, X_2, X_3 = f +- i h
+    e.x = v[0].x + c1 * a.x + c2 * b.x;
+    e.y = v[0].y + c1 * a.y + c2 * b.y;
+    f.x = v[0].x + c2 * a.x + c1 * b.x;
+    f.y = v[0].y + c2 * a.y + c1 * b.y;
+    g.x = s1 * c.x + s2 * d.x;
+    g.y = s1 * c.y + s2 * d.y;
+    h.x = s2 * c.x - s1 * d.x;
+    h.y = s2 * c.y - s1 * d.y;
+    v[0] = cadd(v[0], cadd(a, b));
+    v[1].x = e.x - g.y;
+    v[1].y = e.y + g.x;
+    v[4].x = e.x + g.y;
+    v[4].y = e.y - g.x;
+    v[2].x = f.x - h.y;
+    v[2].y = f.y + h.x;
+    v[3].x = f.x + h.y;
+    v[3].y = f.y - h.x;
+  }
+};
+
 template <int R>
 struct Factor {
-  static constexpr int F = (R % 4 == 0) ? 4 : ((R % 2 == 0) ? 2 : 3);
+  static constexpr int F = (R % 4 == 0) ? 4 : ((R % 2 == 0) ? 2 : ((R % 3 == 0) ? 3 : 5));
 };
 
 // R = F * M: x[F m + f] -> DFT_M over m for each f, twiddle W_R^(f k'), DFT_F over f.
 template <int R, int S, class V>
 struct Dft {
-  static_assert(R > 4, "base cases cover R <= 4");
+  static_assert(R > 5, "base cases cover R <= 5");
   static __host__ __device__ __forceinline__ void run(V* v) {
     using T = decltype(v[0].x);
     constexpr int F = Factor<R>::F, M = R / F;

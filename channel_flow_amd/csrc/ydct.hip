@@ -466,30 +466,82 @@ constexpr bool single_load() {
   return sizeof(V) == 8 || ANA;
 }
 
-// mode 0: point values, 1: padded synthesis, 2: analysis; A1 x A2 = 2N
-template <int A1, int A2, class V, class TI, class TO>
-static hipError_t run_y(Ctx& c, int mode, const YArgs& a, int nf) {
-  constexpr int TX = YT<V>::TX, nt = TX * ymax(A1, A2);
-  const size_t shm = sizeof(V) * (size_t)TX * tile_stride<V>(A1 * (A2 + 1));
-  if (mode == 0) {
-    // point values are FP64 arithmetic only (h^n, the statistics profiles)
-    if constexpr (sizeof(V) == sizeof(double2)) return launch_y(c, k_ypoints<A1, A2, V>, TX, nt, shm, a, nf);
-    return hipErrorNotSupported;
-  }
-  if (mode == 1) return launch_y(c, k_ycheb<A1, A2, V, TI, TO, false, single_load<V, false>()>, TX, nt, shm, a, nf);
-  return launch_y(c, k_ycheb<A1, A2, V, TI, TO, true, single_load<V, true>()>, TX, nt, shm, a, nf);
-}
-
-// 1 when 2N has a split below (and so an FFT form of the transforms).
-int ydct_length_supported(int N) {
+// The splits A1 x A2 (A2 even) of the 2N-point transform: every even degree from
+// 32 to 256 whose 2N has factors up to 24 of this form.  Other degrees (and column
+// counts that are no multiple of 16) take the cos-table products.  The FFT was the
+// faster form at each degree, step time in us, FFT / products, FP64 and mixed:
+// 32x32 N = 40 55 / 65, 55 / 58, N = 100 83 / 100, 82 / 91, N = 240 141 / 210,
+// 129 / 172; 128x128 N = 40 190 / 195, 129 / 140, N = 90 393 / 399, 264 / 266,
+// N = 160 636 / 741, 416 / 476, N = 240 986 / 1241, 647 / 794.
+// Calls run.operator()<A1, A2>(); false without a split.
+template <class F>
+static bool with_y_split(int N, F&& run) {
   switch (2 * N) {
-    case 64: case 96: case 128: case 192: case 256: case 384: case 512: return 1;
-    default: return 0;
+    case 64: run.template operator()<8, 8>(); return true;
+    case 80: run.template operator()<8, 10>(); return true;
+    case 96: run.template operator()<8, 12>(); return true;
+    case 100: run.template operator()<10, 10>(); return true;
+    case 120: run.template operator()<10, 12>(); return true;
+    case 128: run.template operator()<8, 16>(); return true;
+    case 144: run.template operator()<12, 12>(); return true;
+    case 160: run.template operator()<10, 16>(); return true;
+    case 180: run.template operator()<10, 18>(); return true;
+    case 192: run.template operator()<12, 16>(); return true;
+    case 200: run.template operator()<10, 20>(); return true;
+    case 240: run.template operator()<12, 20>(); return true;
+    case 256: run.template operator()<16, 16>(); return true;
+    case 288: run.template operator()<16, 18>(); return true;
+    case 300: run.template operator()<15, 20>(); return true;
+    case 320: run.template operator()<16, 20>(); return true;
+    case 360: run.template operator()<18, 20>(); return true;
+    case 384: run.template operator()<16, 24>(); return true;
+    case 400: run.template operator()<20, 20>(); return true;
+    case 432: run.template operator()<18, 24>(); return true;
+    case 480: run.template operator()<20, 24>(); return true;
+    case 512: run.template operator()<16, 32>(); return true;
+    default: return false;
   }
 }
 
-template <class V, class TI, class TO>
-static hipError_t run_ydct(Ctx& c, int mode, const TI* const* in, TO* const* out, int nf) {
+struct HasYSplit {
+  template <int A1, int A2>
+  void operator()() {}
+};
+
+// 1 when 2N has a split (and so an FFT form of the transforms).
+int ydct_length_supported(int N) { return with_y_split(N, HasYSplit{}) ? 1 : 0; }
+
+template <class V, class TI, class TO, bool ANA>
+struct RunYCheb {
+  Ctx& c;
+  const YArgs& a;
+  int nf;
+  hipError_t e = hipErrorNotSupported;
+  template <int A1, int A2>
+  void operator()() {
+    constexpr int TX = YT<V>::TX, nt = TX * ymax(A1, A2);
+    constexpr size_t shm = sizeof(V) * (size_t)TX * tile_stride<V>(A1 * (A2 + 1));
+    e = launch_y(c, k_ycheb<A1, A2, V, TI, TO, ANA, single_load<V, ANA>()>, TX, nt, shm, a, nf);
+  }
+};
+
+// point values are FP64 arithmetic only (h^n, the statistics profiles)
+struct RunYPoints {
+  Ctx& c;
+  const YArgs& a;
+  int nf;
+  hipError_t e = hipErrorNotSupported;
+  template <int A1, int A2>
+  void operator()() {
+    using V = double2;
+    constexpr int TX = YT<V>::TX, nt = TX * ymax(A1, A2);
+    constexpr size_t shm = sizeof(V) * (size_t)TX * tile_stride<V>(A1 * (A2 + 1));
+    e = launch_y(c, k_ypoints<A1, A2, V>, TX, nt, shm, a, nf);
+  }
+};
+
+template <class TI, class TO>
+static YArgs y_args(const Ctx& c, const TI* const* in, TO* const* out, int nf) {
   YArgs a{};
   for (int f = 0; f < nf; ++f) {
     a.in[f] = in[f];
@@ -501,34 +553,53 @@ static hipError_t run_ydct(Ctx& c, int mode, const TI* const* in, TO* const* out
   a.twN = c.twy + 2 * N;
   a.wq = c.twy + 3 * N;
   a.inv2n = 1.0 / (2.0 * N);
-  switch (2 * N) {
-    case 64: return run_y<8, 8, V, TI, TO>(c, mode, a, nf);
-    case 96: return run_y<8, 12, V, TI, TO>(c, mode, a, nf);
-    case 128: return run_y<8, 16, V, TI, TO>(c, mode, a, nf);
-    case 192: return run_y<12, 16, V, TI, TO>(c, mode, a, nf);
-    case 256: return run_y<16, 16, V, TI, TO>(c, mode, a, nf);
-    case 384: return run_y<16, 24, V, TI, TO>(c, mode, a, nf);
-    case 512: return run_y<16, 32, V, TI, TO>(c, mode, a, nf);
-    default: return hipErrorNotSupported;
-  }
+  return a;
+}
+
+template <class V, bool ANA, class TI, class TO>
+static hipError_t run_ycheb(Ctx& c, const TI* const* in, TO* const* out, int nf) {
+  const YArgs a = y_args(c, in, out, nf);
+  RunYCheb<V, TI, TO, ANA> run{c, a, nf};
+  with_y_split(c.d.N, run);
+  return run.e;
 }
 
 hipError_t launch_ypoints(Ctx& c, const double2* const* in, double2* const* out, int nf) {
-  return run_ydct<double2>(c, 0, in, out, nf);
+  const YArgs a = y_args(c, in, out, nf);
+  RunYPoints run{c, a, nf};
+  with_y_split(c.d.N, run);
+  return run.e;
 }
 hipError_t launch_ysynth(Ctx& c, const double2* const* in, double2* const* out, int nf) {
-  return run_ydct<double2>(c, 1, in, out, nf);
+  return run_ycheb<double2, false>(c, in, out, nf);
 }
 hipError_t launch_yanalysis(Ctx& c, const double2* const* in, double2* const* out, int nf) {
-  return run_ydct<double2>(c, 2, in, out, nf);
+  return run_ycheb<double2, true>(c, in, out, nf);
 }
-template <int N1, int N2>
-static hipError_t run_yrhs(Ctx& c, int count, bool fuse, const YRhsArgs& a) {
-  constexpr int TX = YT<double2>::TX, nt = TX * ymax(N1, N2);
-  const size_t shm = sizeof(double2) * (size_t)TX * tile_stride<double2>(N1 * (N2 + 1));
-  return fuse ? launch_y(c, k_yrhs<N1, N2, true>, TX, nt, shm, a, count)
-              : launch_y(c, k_yrhs<N1, N2, false>, TX, nt, shm, a, count);
+hipError_t launch_ysynth32(Ctx& c, const double2* const* in, float2* const* out, int nf) {
+  return run_ycheb<float2, false>(c, in, out, nf);
 }
+hipError_t launch_ysynth32f(Ctx& c, const float2* const* in, float2* const* out, int nf) {
+  return run_ycheb<float2, false>(c, in, out, nf);
+}
+hipError_t launch_yanalysis32f(Ctx& c, const float2* const* in, float2* const* out, int nf) {
+  return run_ycheb<float2, true>(c, in, out, nf);
+}
+
+struct RunYRhs {
+  Ctx& c;
+  const YRhsArgs& a;
+  int count;
+  bool fuse;
+  hipError_t e = hipErrorNotSupported;
+  template <int N1, int N2>
+  void operator()() {
+    constexpr int TX = YT<double2>::TX, nt = TX * ymax(N1, N2);
+    constexpr size_t shm = sizeof(double2) * (size_t)TX * tile_stride<double2>(N1 * (N2 + 1));
+    e = fuse ? launch_y(c, k_yrhs<N1, N2, true>, TX, nt, shm, a, count)
+             : launch_y(c, k_yrhs<N1, N2, false>, TX, nt, shm, a, count);
+  }
+};
 
 hipError_t launch_yrhs(Ctx& c, int first, int count) {
   const int cur = c.hcur, prv = 1 - c.hcur;  // h^n, h^(n-1)
@@ -541,30 +612,9 @@ hipError_t launch_yrhs(Ctx& c, int first, int count) {
   a.no = c.d.no;
   a.dt = c.prm.dt;
   a.twL = c.twy;
-  const bool fuse = c.hdefer;
-  switch (2 * c.d.N) {
-    case 64: return run_yrhs<8, 8>(c, count, fuse, a);
-    case 96: return run_yrhs<8, 12>(c, count, fuse, a);
-    case 128: return run_yrhs<8, 16>(c, count, fuse, a);
-    case 192: return run_yrhs<12, 16>(c, count, fuse, a);
-    case 256: return run_yrhs<16, 16>(c, count, fuse, a);
-    case 384: return run_yrhs<16, 24>(c, count, fuse, a);
-    case 512: return run_yrhs<16, 32>(c, count, fuse, a);
-    default: return hipErrorNotSupported;
-  }
-}
-
-hipError_t launch_ysynth32(Ctx& c, const double2* const* in, float2* const* out, int nf) {
-  return run_ydct<float2>(c, 1, in, out, nf);
-}
-hipError_t launch_ysynth32f(Ctx& c, const float2* const* in, float2* const* out, int nf) {
-  return run_ydct<float2>(c, 1, in, out, nf);
-}
-hipError_t launch_yanalysis32f(Ctx& c, const float2* const* in, float2* const* out, int nf) {
-  return run_ydct<float2>(c, 2, in, out, nf);
-}
-hipError_t launch_yanalysis32(Ctx& c, const float2* const* in, double2* const* out, int nf) {
-  return run_ydct<float2>(c, 2, in, out, nf);
+  RunYRhs run{c, a, count, c.hdefer};
+  with_y_split(c.d.N, run);
+  return run.e;
 }
 
 }  // namespace chf
