@@ -14,6 +14,7 @@
 //              (plan11 and expand(-1), PF:1158-1179)
 #include "chf_internal.h"
 #include "fftreg.h"
+#include <type_traits>
 
 namespace chf {
 
@@ -376,6 +377,8 @@ struct Geo {
   // LDS stride between the exchange tiles of the lines of one span-pass block
   // (paddings of 1, 2 and 8 elements measured: no faster)
   static constexpr int LINE_Z = BUF_A;
+  // the same for half-size (8-byte) values: 4 mod 32
+  static constexpr int HALF_LINE = BUF_A + (4 - BUF_A % 32 + 32) % 32;
   static constexpr int BUF_B = N2 * (N1 + 1);  // transposed-order tile
   static constexpr int BUF = (BUF_A > BUF_B ? BUF_A : BUF_B) > L ? (BUF_A > BUF_B ? BUF_A : BUF_B) : L;
 };
@@ -982,6 +985,108 @@ __global__ __launch_bounds__((TX * Geo<N1, N2>::G)) void k_zfft_pair(RegZ<float2
   }
 }
 
+// Span pass with the exchange in two halves: a lane's 16-byte column (one FP64
+// column or a pair of FP32 ones) goes through the tile as its real, then its
+// imaginary parts (FP32: the first, then the second column), so the tile takes
+// half the LDS.  The long lines need it: at 768 points the whole tile is 101 KB
+// for eight FP64 columns, one block (a wavefront per SIMD) on a CU, whose loads,
+// transforms and stores then follow one another.  HALF_LINE puts the 32 lanes
+// of an 8-byte LDS pass (eight columns, four rows) in distinct banks.
+template <int N1, int N2, int TX, bool INV, class V>
+__global__ __launch_bounds__((TX * Geo<N1, N2>::G)) void k_zfft_half(RegZ<V> a) {
+  constexpr bool F64 = sizeof(V) == 16;
+  using Gm = Geo<N1, N2>;
+  using H = typename std::conditional<F64, double, float2>::type;    // half of a lane's column
+  using Q = typename std::conditional<F64, double2, float4>::type;
+  constexpr int NC = F64 ? 1 : 2, S = INV ? +1 : -1, L = Gm::L;
+  extern __shared__ __align__(16) unsigned char smraw[];
+  V* tw = reinterpret_cast<V*>(smraw);
+  const int t = threadIdx.x / TX, tx = threadIdx.x - t * TX;
+  H* buf = reinterpret_cast<H*>(tw + L) + tx * Gm::HALF_LINE;
+  const int Mz = a.Mz, h = Mz / 2;
+  const int kg = (int)xcd_order(blockIdx.x, gridDim.x);
+  const int Mq = a.Mx / NC, kq = kg * TX + tx;
+  const bool valid = kq < Mq;  // the last group may be partial
+  const int p = blockIdx.y;
+  const Q* in = reinterpret_cast<const Q*>(a.in[blockIdx.z] + (long)p * a.in_plane);
+  Q* out = reinterpret_cast<Q*>(a.out[blockIdx.z] + (long)p * a.out_plane);
+  for (int i = threadIdx.x; i < L; i += TX * Gm::G) tw[i] = a.tw[i];
+  V x[NC][N2], b[NC][N1];
+  if (t < N1 && valid) {
+#pragma unroll
+    for (int n2 = 0; n2 < N2; ++n2) {
+      const int m = n2 * N1 + t;
+      Q q{};
+      if (INV) {
+        int kz = -1;
+        if (m < h) kz = m;                       // Nyquist slot Mz/2 stays zero (expand, PF:730)
+        else if (m > L - h) kz = m - L + Mz;
+        if (kz >= 0) q = in[(long)kz * Mq + kq];
+      } else {
+        q = in[(long)m * Mq + kq];
+      }
+      if constexpr (F64) {
+        x[0][n2] = q;
+      } else {
+        x[0][n2] = make_float2(q.x, q.y);
+        x[1][n2] = make_float2(q.z, q.w);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) Dft<N2, S, V>::run(x[c]);
+  }
+  __syncthreads();  // the twiddles are there
+  if (t < N1 && valid) {
+#pragma unroll
+    for (int k2 = 1; k2 < N2; ++k2) {
+      V w = tw[t * k2];
+      if (S > 0) w.y = -w.y;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) x[c][k2] = cmulv(x[c][k2], w);
+    }
+  }
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    if (half) __syncthreads();  // the first halves are read
+    if (t < N1 && valid) {
+#pragma unroll
+      for (int k2 = 0; k2 < N2; ++k2) {
+        if constexpr (F64) buf[t * (N2 + 1) + k2] = half ? x[0][k2].y : x[0][k2].x;
+        else buf[t * (N2 + 1) + k2] = x[half][k2];
+      }
+    }
+    __syncthreads();
+    if (t < N2 && valid) {
+#pragma unroll
+      for (int n1 = 0; n1 < N1; ++n1) {
+        const H v = buf[n1 * (N2 + 1) + t];
+        if constexpr (!F64) b[half][n1] = v;
+        else if (half) b[0][n1].y = v;
+        else b[0][n1].x = v;
+      }
+    }
+  }
+  if (t < N2 && valid) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) Dft<N1, S, V>::run(b[c]);
+#pragma unroll
+    for (int k1 = 0; k1 < N1; ++k1) {
+      const int m = k1 * N2 + t;
+      Q q;
+      if constexpr (F64) q = b[0][k1];
+      else q = make_float4(b[0][k1].x, b[0][k1].y, b[1][k1].x, b[1][k1].y);
+      if (INV) {
+        out[(long)m * Mq + kq] = q;
+      } else {
+        int kz = -1;                              // expand(-1): keep 0..Mz/2 and the negative band
+        if (m <= h) kz = m;
+        else if (m > L - h) kz = m - L + Mz;
+        if (kz >= 0) out[(long)kz * Mq + kq] = q;
+      }
+    }
+  }
+}
+
 // Lengths of the mixed form's register FFTs.
 bool reg_fft_length32(int L) {
   switch (L) {
@@ -1087,26 +1192,55 @@ static hipError_t run_zfft_pair(Ctx& c, const RegZ<float2>& a, bool inv, int nf)
   return e;
 }
 
+template <int N1, int N2, int TX, class V>
+static hipError_t run_zfft_half(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
+  using Gm = Geo<N1, N2>;
+  constexpr size_t shm = sizeof(V) * Gm::L + 8 * (size_t)TX * Gm::HALF_LINE;
+  constexpr int NC = 16 / sizeof(V);
+  static_assert(shm <= 65536, "the launch takes the default limit");
+  if (c.d.Mx % NC) return hipErrorInvalidValue;
+  for (int f = 0; f < nf; ++f)
+    if (((uintptr_t)a.in[f] | (uintptr_t)a.out[f]) & 15) return hipErrorInvalidValue;
+  const int Mq = c.d.Mx / NC;
+  dim3 grid((Mq + TX - 1) / TX, c.d.Py, nf);
+  if (inv)
+    hipLaunchKernelGGL((k_zfft_half<N1, N2, TX, true, V>), grid, dim3(TX * Gm::G), shm, c.stream, a);
+  else
+    hipLaunchKernelGGL((k_zfft_half<N1, N2, TX, false, V>), grid, dim3(TX * Gm::G), shm, c.stream, a);
+  return hipGetLastError();
+}
+
+// The exchange goes in halves where eight 16-byte columns and the twiddles do not
+// fit in 64 KB (FP64 576 and 768 points, FP32 768), us of whole / half tile, inverse
+// and forward: 512x65x512 FP64 1085 / 747 (5.4 TB/s), 582 / 404, FP32 495 / 369,
+// 291 / 212; 384x65x384 FP64 579 / 404, 316 / 202.  Where they fit a second block
+// hides one's phases already: 288x97x288 344 / 339, 159 / 168; 256x193x256 521 /
+// 585, 299 / 310, FP32 289 / 283, 155 / 149.
 template <int N1, int N2, class V>
 static hipError_t run_zfft_reg(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
   using Gm = Geo<N1, N2>;
-  if constexpr (sizeof(V) == 8) {
-    const hipError_t e = run_zfft_pair<N1, N2>(c, a, inv, nf);
-    if (e != hipErrorNotSupported) return e;
+  if constexpr (sizeof(V) * Gm::L + 8 * 16 * Gm::BUF_A > 65536) {
+    return run_zfft_half<N1, N2, 8>(c, a, inv, nf);
+  } else {
+    if constexpr (sizeof(V) == 8) {
+      const hipError_t e = run_zfft_pair<N1, N2>(c, a, inv, nf);
+      if (e != hipErrorNotSupported) return e;
+    }
+    constexpr int TX = (256 / Gm::G) >= 16 ? 16 : ((256 / Gm::G) >= 8 ? 8 : 4);
+    const size_t shm = sizeof(V) * (Gm::L + (size_t)TX * Gm::LINE_Z);
+    dim3 grid((c.d.Mx + TX - 1) / TX, c.d.Py, nf);
+    const void* fn =
+        inv ? (const void*)k_zfft_reg<N1, N2, TX, true, V> : (const void*)k_zfft_reg<N1, N2, TX, false, V>;
+    if (shm > 65536) {
+      hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+      if (e != hipSuccess) return e;
+    }
+    if (inv)
+      hipLaunchKernelGGL((k_zfft_reg<N1, N2, TX, true, V>), grid, dim3(TX * Gm::G), shm, c.stream, a);
+    else
+      hipLaunchKernelGGL((k_zfft_reg<N1, N2, TX, false, V>), grid, dim3(TX * Gm::G), shm, c.stream, a);
+    return hipGetLastError();
   }
-  constexpr int TX = (256 / Gm::G) >= 16 ? 16 : ((256 / Gm::G) >= 8 ? 8 : 4);
-  const size_t shm = sizeof(V) * (Gm::L + (size_t)TX * Gm::LINE_Z);
-  dim3 grid((c.d.Mx + TX - 1) / TX, c.d.Py, nf);
-  const void* fn = inv ? (const void*)k_zfft_reg<N1, N2, TX, true, V> : (const void*)k_zfft_reg<N1, N2, TX, false, V>;
-  if (shm > 65536) {
-    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    if (e != hipSuccess) return e;
-  }
-  if (inv)
-    hipLaunchKernelGGL((k_zfft_reg<N1, N2, TX, true, V>), grid, dim3(TX * Gm::G), shm, c.stream, a);
-  else
-    hipLaunchKernelGGL((k_zfft_reg<N1, N2, TX, false, V>), grid, dim3(TX * Gm::G), shm, c.stream, a);
-  return hipGetLastError();
 }
 
 // Span pass through the register kernel; hipErrorInvalidValue when the length
