@@ -1,5 +1,6 @@
 // C ABI of libchf: context life cycle, state exchange in the reference
 // layout, and the step sequence of the reference time loop (PF:220-532).
+#include <algorithm>
 #include <array>
 #include <cmath>
 #include <cstdio>
@@ -10,6 +11,8 @@
 #include <mutex>
 #include <system_error>
 #include <thread>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "chf_internal.h"
@@ -327,14 +330,48 @@ int autotune(Ctx* c) {
   return 0;
 }
 
-// Fields from this many values on run their independent launches on the
-// context's two streams: each cross-stream wait costs about 10 us on the
-// device, and the launches' tails that the overlap fills only outweigh that on
-// large grids.  Step times (us) on two streams / one: 24x22x16 143 / 60,
-// 32x33x32 142 / 68, 96x101x96 mixed 266 / 241, 128x129x128 590 / 579 (1.06 M
-// values), 192x161x192 1680 / 1723 (2.97 M), 256x193x256 FP64 2985 / 2965, mixed
-// 1868 / 1873, 512x257x512 FP64 20720 / 21270, mixed 11800 / 12075.
-constexpr size_t kOverlapValues = size_t(2) << 20;
+// Span and streamwise transforms whose six padded fields take more than
+// kSlabsFrom run in slabs of wall-normal planes of about kSlabBytes, on the
+// context's two streams in turn: the two slabs in flight stay in the 256 MB
+// Infinity Cache between the three launches, and the streamwise pass of one
+// (bound by LDS) runs beside the span FFTs of the other (bound by memory).
+// Step times (us), all planes at once on one stream / in slabs: 512x257x512
+// FP64 19466 / 18471 (9.7 GB), mixed 11374 / 11046 (4.8 GB), 256x193x256 FP64
+// 2916 / 2873 (1.8 GB), mixed 1848 / 1857 (0.9 GB), 192x161x192 1434 / 1443
+// (0.85 GB), 128x129x128 500 / 504: each cross-stream wait costs about 10 us.
+// Slabs of half the bytes cost 512x257x512 FP64 0.7%, twice 1.6%; on one stream
+// every slab size is slower than no slabs (each launch's tail is idle).  Field
+// groups of the wall-normal transforms on the two streams (512x257x512 FP64
+// 18520 -> 18670, mixed 11040 -> 11115) gain nothing.
+constexpr size_t kSlabsFrom = size_t(1) << 30;
+constexpr size_t kSlabBytes = size_t(160) << 20;
+
+int slab_planes(const Dims& d, size_t plane) {
+  const int most = (int)std::max<size_t>(1, kSlabBytes / plane);
+  const int pairs = (d.Py + 2 * most - 1) / (2 * most);  // as many on each stream
+  return (d.Py + 2 * pairs - 1) / (2 * pairs);
+}
+
+// Padded-plane work arrays of `planes` wall-normal planes in the place of the
+// present ones, which stay where an allocation fails.
+int alloc_padded(Ctx* c, int planes) {
+  const size_t plane = (size_t)c->d.Lz * c->d.Mx;
+  auto renew = [&](auto& z) -> int {
+    std::remove_reference_t<decltype(z)> fresh = {};
+    hipError_t e = hipSuccess;
+    for (auto& p : fresh)
+      if (e == hipSuccess) e = hipMalloc((void**)&p, planes * plane * sizeof(*p));
+    for (int f = 0; f < 6; ++f) {
+      if (e == hipSuccess) std::swap(z[f], fresh[f]);
+      if (fresh[f]) (void)hipFree(fresh[f]);
+    }
+    CHF_TRY(e);
+    c->bytes += 6ll * (planes - c->zplanes) * (long long)(plane * sizeof(*z[0]));
+    c->zplanes = planes;
+    return 0;
+  };
+  return c->prm.precision == 0 ? renew(c->Z) : renew(c->Zf);
+}
 
 int build(Ctx* c, DegreeCache& cache) {
   Dims& d = c->d;
@@ -373,7 +410,6 @@ int build(Ctx* c, DegreeCache& cache) {
   CHF_TRY(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
 
   const size_t fld = (size_t)d.Ny * d.ncol;
-  c->overlap = c->overlap && fld >= kOverlapValues;
   CHF_TRY(dalloc(c, &c->alpha, d.Mx));
   CHF_TRY(dalloc(c, &c->beta, d.Mz));
   CHF_TRY(dalloc(c, &c->v, fld));
@@ -391,14 +427,15 @@ int build(Ctx* c, DegreeCache& cache) {
   CHF_TRY(dalloc(c, &c->au0, d.Ny));
   CHF_TRY(dalloc(c, &c->w0, d.Ny));
   const size_t ysz = (size_t)d.Py * d.ncol;
-  const size_t zsz = (size_t)d.Py * d.Lz * d.Mx;
   if (p.precision == 0) {
     for (auto& y : c->Y) CHF_TRY(dalloc(c, &y, ysz));
-    for (auto& z : c->Z) CHF_TRY(dalloc(c, &z, zsz));
   } else {
     for (auto& y : c->Yf) CHF_TRY(dalloc(c, &y, ysz));
-    for (auto& z : c->Zf) CHF_TRY(dalloc(c, &z, zsz));
   }
+  const size_t plane = 6 * (p.precision == 0 ? sizeof(double2) : sizeof(float2)) * d.Lz * d.Mx;
+  c->slabs = c->slabs && plane * d.Py > kSlabsFrom;
+  if (c->slabs) c->slab = slab_planes(d, plane);
+  if (const int rc = alloc_padded(c, c->slabs ? 2 * c->slab : d.Py)) return rc;
   for (auto& l : c->Lc) CHF_TRY(dalloc(c, &l, fld));
   CHF_TRY(dalloc(c, &c->hvc, fld));
   CHF_TRY(dalloc(c, &c->hgc, fld));
@@ -642,24 +679,6 @@ hipError_t form_h_points(Ctx* c) {
   return e;
 }
 
-// Runs a() on the context's stream and b() on the side stream, both after the
-// work queued so far, and joins them: two field groups of one transform
-// stage, so that each launch's tail overlaps the other's work.
-template <class A, class B>
-hipError_t on_two_streams(Ctx* c, A&& a, B&& b) {
-  hipError_t e = hipEventRecord(c->ev_fork, c->stream);
-  if (e == hipSuccess) e = hipStreamWaitEvent(c->side, c->ev_fork, 0);
-  if (e == hipSuccess) e = a();
-  if (e != hipSuccess) return e;
-  hipStream_t main = c->stream;
-  c->stream = c->side;  // the launchers use c->stream
-  e = b();
-  if (e == hipSuccess) e = hipEventRecord(c->ev_join, c->side);
-  c->stream = main;
-  if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, c->ev_join, 0);
-  return e;
-}
-
 // Mixed form: the padded FP32 synthesis of fields f0 .. f0 + nf - 1 of
 // (u, v, w, omega_x, omega_y, omega_z) into Yf.  u, w, omega_x, omega_z come
 // from their FP32 copies when those are current: the values the FP64 inputs
@@ -694,52 +713,54 @@ hipError_t analysis32_fields(Ctx* c, const float2* const* y3, int f0, int nf) {
   return launch_analysis32(*c, y3 + f0, c->Lc + f0, nf);
 }
 
+// Y: the six fields at the wall-normal points in, the Lamb vector out in
+// Y[0..2], through the padded planes Z; in slabs on the two streams (build),
+// or all planes at once (with timing on too, so that each launch runs alone
+// and is one of its class per step).
+template <class V>
+hipError_t physical_products(Ctx* c, V* const* Y, V* const* Z) {
+  const Dims& d = c->d;
+  auto planes = [&](int y0, int np, int z0) {
+    V *y[6], *z[6];
+    for (int f = 0; f < 6; ++f) {
+      y[f] = Y[f] + (long)y0 * d.ncol;
+      z[f] = Z[f] + (long)z0 * d.Lz * d.Mx;
+    }
+    hipError_t e = timed(c, K_ZFFT_INV, [&] { return launch_zfft(*c, y, z, 6, true, np); });
+    if (e == hipSuccess) e = timed(c, K_XPASS, [&] { return launch_xpass(*c, z, np); });
+    if (e == hipSuccess) e = timed(c, K_ZFFT_FWD, [&] { return launch_zfft(*c, z, y, 3, false, np); });
+    return e;
+  };
+  if (!c->slabs || c->timing) return planes(0, d.Py, 0);
+  hipError_t e = hipEventRecord(c->ev_fork, c->stream);
+  if (e == hipSuccess) e = hipStreamWaitEvent(c->side, c->ev_fork, 0);
+  hipStream_t main = c->stream;
+  for (int y0 = 0, s = 0; y0 < d.Py && e == hipSuccess; y0 += c->slab, ++s) {
+    c->stream = s & 1 ? c->side : main;  // the launchers use c->stream
+    e = planes(y0, std::min(c->slab, d.Py - y0), s & 1 ? c->slab : 0);
+  }
+  c->stream = main;
+  if (e == hipSuccess) e = hipEventRecord(c->ev_join, c->side);
+  if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, c->ev_join, 0);
+  return e;
+}
+
 // With the FFT transforms h^n's point values are left to the next solve's
 // right-hand-side kernels.
 int nonlinear(Ctx* c) {
   CHF_TRY(form_h_points(c));  // the previous step's, before the h assembly overwrites hvc, hgc
   // six fields in the order the streamwise pass pairs them: (u,v) (w,ox) (oy,oz)
   const double2* in6[6] = {c->u, c->v, c->w, c->ox, c->oy, c->oz};
-  if (!c->timing && c->overlap) {
-    // synthesis and span FFTs of fields 0-2 and 3-5, then of L_x, L_y and
-    // L_z, on the two streams (with timing on every launch runs alone)
-    if (c->prm.precision == 0) {
-      CHF_TRY(on_two_streams(
-          c, [&] { const hipError_t e = launch_synth_padded(*c, in6, c->Y, 3); return e ? e : launch_zfft_inv(*c, c->Y, c->Z, 3); },
-          [&] { const hipError_t e = launch_synth_padded(*c, in6 + 3, c->Y + 3, 3); return e ? e : launch_zfft_inv(*c, c->Y + 3, c->Z + 3, 3); }));
-      CHF_TRY(launch_xpass(*c));
-      const double2* y3[3] = {c->Y[0], c->Y[1], c->Y[2]};
-      CHF_TRY(on_two_streams(
-          c, [&] { const hipError_t e = launch_zfft_fwd(*c, c->Z, c->Y, 2); return e ? e : launch_analysis(*c, y3, c->Lc, 2); },
-          [&] { const hipError_t e = launch_zfft_fwd(*c, c->Z + 2, c->Y + 2, 1); return e ? e : launch_analysis(*c, y3 + 2, c->Lc + 2, 1); }));
-    } else {
-      const float2* y6[6] = {c->Yf[0], c->Yf[1], c->Yf[2], c->Yf[3], c->Yf[4], c->Yf[5]};
-      const float2* z3[3] = {c->Zf[0], c->Zf[1], c->Zf[2]};
-      const float2* y3[3] = {c->Yf[0], c->Yf[1], c->Yf[2]};
-      CHF_TRY(on_two_streams(
-          c, [&] { const hipError_t e = synth32_fields(c, in6, 0, 3); return e ? e : launch_zfft32(*c, y6, c->Zf, 3, true); },
-          [&] { const hipError_t e = synth32_fields(c, in6, 3, 3); return e ? e : launch_zfft32(*c, y6 + 3, c->Zf + 3, 3, true); }));
-      CHF_TRY(launch_xpass32(*c));
-      CHF_TRY(on_two_streams(
-          c, [&] { const hipError_t e = launch_zfft32(*c, z3, c->Yf, 2, false); return e ? e : analysis32_fields(c, y3, 0, 2); },
-          [&] { const hipError_t e = launch_zfft32(*c, z3 + 2, c->Yf + 2, 1, false); return e ? e : analysis32_fields(c, y3, 2, 1); }));
-    }
-  } else if (c->prm.precision == 0) {
+  if (c->prm.precision == 0) {
     CHF_TRY(timed(c, K_SYNTH_PADDED, [&] { return launch_synth_padded(*c, in6, c->Y, 6); }));
-    CHF_TRY(timed(c, K_ZFFT_INV, [&] { return launch_zfft_inv(*c, c->Y, c->Z, 6); }));
-    CHF_TRY(timed(c, K_XPASS, [&] { return launch_xpass(*c); }));
-    CHF_TRY(timed(c, K_ZFFT_FWD, [&] { return launch_zfft_fwd(*c, c->Z, c->Y, 3); }));
+    CHF_TRY(physical_products(c, c->Y, c->Z));
     const double2* y3[3] = {c->Y[0], c->Y[1], c->Y[2]};
     CHF_TRY(timed(c, K_ANALYSIS, [&] { return launch_analysis(*c, y3, c->Lc, 3); }));
   } else {
     // mixed form: FP32 wall-normal values, FP32 FFTs and products, FP64 coefficients out
-    const float2* y6[6] = {c->Yf[0], c->Yf[1], c->Yf[2], c->Yf[3], c->Yf[4], c->Yf[5]};
-    const float2* z3[3] = {c->Zf[0], c->Zf[1], c->Zf[2]};
     const float2* y3[3] = {c->Yf[0], c->Yf[1], c->Yf[2]};
     CHF_TRY(timed(c, K_SYNTH_PADDED, [&] { return synth32_fields(c, in6, 0, 6); }));
-    CHF_TRY(timed(c, K_ZFFT_INV, [&] { return launch_zfft32(*c, y6, c->Zf, 6, true); }));
-    CHF_TRY(timed(c, K_XPASS, [&] { return launch_xpass32(*c); }));
-    CHF_TRY(timed(c, K_ZFFT_FWD, [&] { return launch_zfft32(*c, z3, c->Yf, 3, false); }));
+    CHF_TRY(physical_products(c, c->Yf, c->Zf));
     CHF_TRY(timed(c, K_ANALYSIS, [&] { return analysis32_fields(c, y3, 0, 3); }));
   }
   CHF_TRY(timed(c, K_HASSEMBLE, [&] { return launch_hassemble(*c); }));
@@ -988,6 +1009,8 @@ int chf_set_timing(void* ctx, int on) {
   if (!ctx) return -1;
   Ctx* c = static_cast<Ctx*>(ctx);
   CHF_TRY(hipStreamSynchronize(c->stream));
+  if (on && c->zplanes < c->d.Py)
+    if (const int rc = alloc_padded(c, c->d.Py)) return rc;
   c->timing = on != 0;
   c->marks.clear();
   c->pool_next = 0;
@@ -1275,7 +1298,7 @@ int chf_ensemble_create(const chf_params* members, int n, void** out) {
   for (int i = 0; i < n; ++i) {
     Ctx* c = new Ctx();
     c->prm = members[i];
-    c->overlap = false;
+    c->slabs = false;
     const int rc = build(c, cache);
     if (rc) {
       g_create_err = "member " + std::to_string(i) + ": " + c->err;

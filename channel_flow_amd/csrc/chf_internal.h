@@ -87,15 +87,13 @@ struct Ctx {
   int device = 0;
   bool holds_pool = false;  // counted among the staging pool's users
   hipStream_t stream = nullptr;
-  // second stream of the context (default priority): with the operators
-  // diagonalised, the omega_y right-hand side and solve run on it while the v
-  // path runs on `stream`; the pair of events forks and joins it
+  // second stream of the context (default priority): every other slab of the
+  // padded planes runs on it; the pair of events forks and joins it
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  // off for small grids (kOverlapValues) and for ensemble members, whose steps
-  // already run as parallel graph branches: the extra fork/join nodes cost more
-  // than they overlap
-  bool overlap = true;
+  // padded planes in slabs (kSlabsFrom); off for ensemble members, whose steps
+  // already run as parallel graph branches
+  bool slabs = true;
   // wavenumbers
   double* alpha = nullptr;  // [Mx]
   double* beta = nullptr;   // [Mz]
@@ -124,9 +122,11 @@ struct Ctx {
   bool hdefer = false;
   // nonlinear work
   double2* Y[6] = {};     // [Py][Mz][Mx]   wall-normal points, Fourier modes
-  double2* Z[6] = {};     // [Py][Lz][Mx]   wall-normal + span points, x modes
+  double2* Z[6] = {};     // [zplanes][Lz][Mx]  wall-normal + span points, x modes
   float2* Yf[6] = {};     // mixed form: FP32 copies of Y and Z
   float2* Zf[6] = {};
+  // planes allocated in Z / Zf (two slabs, or all), and planes of a slab
+  int zplanes = 0, slab = 0;
   double2* Lc[3] = {};    // [Ny][Mz][Mx]   Lamb vector coefficients
   double2 *hvc = nullptr, *hgc = nullptr;  // h coefficients
   // solve work
@@ -225,17 +225,18 @@ void hostcopy_release();
 
 // ---- kernel launchers (each returns hipGetLastError()) ----
 bool reg_fft_length32(int L);  // padded lengths that the mixed form takes
-hipError_t launch_zfft32(Ctx& c, const float2* const* in, float2* const* out, int nf, bool inv);
-hipError_t launch_xpass32(Ctx& c);
+// span transforms and streamwise pass of np wall-normal planes; the streamwise
+// pass leaves L_x, L_y, L_z in Z[0..2]
+hipError_t launch_zfft(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv, int np);
+hipError_t launch_zfft(Ctx& c, float2* const* in, float2* const* out, int nf, bool inv, int np);
+hipError_t launch_xpass(Ctx& c, double2* const* Z, int np);
+hipError_t launch_xpass(Ctx& c, float2* const* Z, int np);
 hipError_t launch_synth_padded32(Ctx& c, const double2* const* in, float2* const* out, int nf);
 // FP32 coefficients in (FFT transforms only): the values launch_synth_padded32 rounds its inputs to
 hipError_t launch_synth_padded32f(Ctx& c, const float2* const* in, float2* const* out, int nf);
 // FP32 coefficients out (FFT transforms only): launch_analysis32's values, which are FP32 numbers
 hipError_t launch_analysis32f(Ctx& c, const float2* const* in, float2* const* out, int nf);
 hipError_t launch_analysis32(Ctx& c, const float2* const* in, double2* const* out, int nf);
-hipError_t launch_zfft_inv(Ctx& c, double2* const* in, double2* const* out, int nf);
-hipError_t launch_xpass(Ctx& c);
-hipError_t launch_zfft_fwd(Ctx& c, double2* const* in, double2* const* out, int nf);
 hipError_t launch_synth_padded(Ctx& c, const double2* const* in, double2* const* out, int nf);
 hipError_t launch_analysis(Ctx& c, const double2* const* in, double2* const* out, int nf);
 hipError_t launch_hassemble(Ctx& c);

@@ -186,10 +186,10 @@ static int pick_tx(int Mx, int Lz) {
   return tx;
 }
 
-static hipError_t zfft_reg64(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv);
+static hipError_t zfft_reg64(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv, int np);
 static bool use_zreg(const Ctx& c);
 
-static hipError_t launch_z(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv) {
+static hipError_t launch_z(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv, int np) {
   const Dims& d = c.d;
   ZArgs a{};
   for (int f = 0; f < nf; ++f) {
@@ -204,8 +204,8 @@ static hipError_t launch_z(Ctx& c, double2* const* in, double2* const* out, int 
   a.out_plane = (long)(inv ? d.Lz : d.Mz) * d.Mx;
   a.pl = make_plan(d.Lz);
   a.tw = c.twz;
-  if (use_zreg(c)) return zfft_reg64(c, in, out, nf, inv);
-  dim3 grid(d.Mx / a.TX, d.Py, nf);
+  if (use_zreg(c)) return zfft_reg64(c, in, out, nf, inv, np);
+  dim3 grid(d.Mx / a.TX, np, nf);
   size_t shm = 2ull * a.TX * d.Lz * sizeof(double2);
   if (inv)
     hipLaunchKernelGGL(k_zfft_inv, grid, dim3(256), shm, c.stream, a);
@@ -277,11 +277,8 @@ hipError_t launch_stream_c2r_lds(Ctx& c, const double2* in, double* out) {
   return hipGetLastError();
 }
 
-hipError_t launch_zfft_inv(Ctx& c, double2* const* in, double2* const* out, int nf) {
-  return launch_z(c, in, out, nf, true);
-}
-hipError_t launch_zfft_fwd(Ctx& c, double2* const* in, double2* const* out, int nf) {
-  return launch_z(c, in, out, nf, false);
+hipError_t launch_zfft(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv, int np) {
+  return launch_z(c, in, out, nf, inv, np);
 }
 
 // ------------------------------------------------------------- streamwise
@@ -1166,13 +1163,13 @@ static hipError_t xpass_reg(Ctx& c, const RegX<V>& a) {
 // Returns hipErrorNotSupported when no tile fits (the caller then takes the
 // single-column kernel).
 template <int N1, int N2, int TX>
-static hipError_t launch_zfft_pair(Ctx& c, const RegZ<float2>& a, bool inv, int nf) {
+static hipError_t launch_zfft_pair(Ctx& c, const RegZ<float2>& a, bool inv, int nf, int np) {
   using Gm = Geo<N1, N2>;
   const size_t shm = sizeof(float2) * Gm::L + sizeof(float4) * (size_t)TX * Gm::BUF_A;
   if (shm > 65536 || c.d.Mx % (2 * TX)) return hipErrorNotSupported;
   for (int f = 0; f < nf; ++f)
     if (((uintptr_t)a.in[f] | (uintptr_t)a.out[f]) & 15) return hipErrorNotSupported;
-  dim3 grid(c.d.Mx / (2 * TX), c.d.Py, nf);
+  dim3 grid(c.d.Mx / (2 * TX), np, nf);
   if (inv)
     hipLaunchKernelGGL((k_zfft_pair<N1, N2, TX, true>), grid, dim3(TX * Gm::G), shm, c.stream, a);
   else
@@ -1181,19 +1178,19 @@ static hipError_t launch_zfft_pair(Ctx& c, const RegZ<float2>& a, bool inv, int 
 }
 
 template <int N1, int N2>
-static hipError_t run_zfft_pair(Ctx& c, const RegZ<float2>& a, bool inv, int nf) {
+static hipError_t run_zfft_pair(Ctx& c, const RegZ<float2>& a, bool inv, int nf, int np) {
   using Gm = Geo<N1, N2>;
   constexpr int TX = (256 / Gm::G) >= 8 ? 8 : ((256 / Gm::G) >= 4 ? 4 : 2);
-  hipError_t e = launch_zfft_pair<N1, N2, TX>(c, a, inv, nf);
+  hipError_t e = launch_zfft_pair<N1, N2, TX>(c, a, inv, nf, np);
   if constexpr (TX > 2)
-    if (e == hipErrorNotSupported) e = launch_zfft_pair<N1, N2, TX / 2>(c, a, inv, nf);
+    if (e == hipErrorNotSupported) e = launch_zfft_pair<N1, N2, TX / 2>(c, a, inv, nf, np);
   if constexpr (TX > 4)
-    if (e == hipErrorNotSupported) e = launch_zfft_pair<N1, N2, TX / 4>(c, a, inv, nf);
+    if (e == hipErrorNotSupported) e = launch_zfft_pair<N1, N2, TX / 4>(c, a, inv, nf, np);
   return e;
 }
 
 template <int N1, int N2, int TX, class V>
-static hipError_t run_zfft_half(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
+static hipError_t run_zfft_half(Ctx& c, const RegZ<V>& a, bool inv, int nf, int np) {
   using Gm = Geo<N1, N2>;
   constexpr size_t shm = sizeof(V) * Gm::L + 8 * (size_t)TX * Gm::HALF_LINE;
   constexpr int NC = 16 / sizeof(V);
@@ -1202,7 +1199,7 @@ static hipError_t run_zfft_half(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
   for (int f = 0; f < nf; ++f)
     if (((uintptr_t)a.in[f] | (uintptr_t)a.out[f]) & 15) return hipErrorInvalidValue;
   const int Mq = c.d.Mx / NC;
-  dim3 grid((Mq + TX - 1) / TX, c.d.Py, nf);
+  dim3 grid((Mq + TX - 1) / TX, np, nf);
   if (inv)
     hipLaunchKernelGGL((k_zfft_half<N1, N2, TX, true, V>), grid, dim3(TX * Gm::G), shm, c.stream, a);
   else
@@ -1217,18 +1214,18 @@ static hipError_t run_zfft_half(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
 // hides one's phases already: 288x97x288 344 / 339, 159 / 168; 256x193x256 521 /
 // 585, 299 / 310, FP32 289 / 283, 155 / 149.
 template <int N1, int N2, class V>
-static hipError_t run_zfft_reg(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
+static hipError_t run_zfft_reg(Ctx& c, const RegZ<V>& a, bool inv, int nf, int np) {
   using Gm = Geo<N1, N2>;
   if constexpr (sizeof(V) * Gm::L + 8 * 16 * Gm::BUF_A > 65536) {
-    return run_zfft_half<N1, N2, 8>(c, a, inv, nf);
+    return run_zfft_half<N1, N2, 8>(c, a, inv, nf, np);
   } else {
     if constexpr (sizeof(V) == 8) {
-      const hipError_t e = run_zfft_pair<N1, N2>(c, a, inv, nf);
+      const hipError_t e = run_zfft_pair<N1, N2>(c, a, inv, nf, np);
       if (e != hipErrorNotSupported) return e;
     }
     constexpr int TX = (256 / Gm::G) >= 16 ? 16 : ((256 / Gm::G) >= 8 ? 8 : 4);
     const size_t shm = sizeof(V) * (Gm::L + (size_t)TX * Gm::LINE_Z);
-    dim3 grid((c.d.Mx + TX - 1) / TX, c.d.Py, nf);
+    dim3 grid((c.d.Mx + TX - 1) / TX, np, nf);
     const void* fn =
         inv ? (const void*)k_zfft_reg<N1, N2, TX, true, V> : (const void*)k_zfft_reg<N1, N2, TX, false, V>;
     if (shm > 65536) {
@@ -1246,34 +1243,34 @@ static hipError_t run_zfft_reg(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
 // Span pass through the register kernel; hipErrorInvalidValue when the length
 // has no split.
 template <class V>
-static hipError_t zfft_reg(Ctx& c, const RegZ<V>& a, bool inv, int nf) {
+static hipError_t zfft_reg(Ctx& c, const RegZ<V>& a, bool inv, int nf, int np) {
   // (192x161x192, 288 points: inverse 0.73 -> 0.26 ms, forward 0.33 -> 0.12
   // against the LDS kernels)
   if constexpr (sizeof(V) == 16) {
     switch (c.d.Lz) {
-      case 18: return run_zfft_reg<3, 6>(c, a, inv, nf);
-      case 36: return run_zfft_reg<6, 6>(c, a, inv, nf);
-      case 54: return run_zfft_reg<6, 9>(c, a, inv, nf);
-      case 72: return run_zfft_reg<8, 9>(c, a, inv, nf);
-      case 108: return run_zfft_reg<9, 12>(c, a, inv, nf);
-      case 162: return run_zfft_reg<9, 18>(c, a, inv, nf);
-      case 216: return run_zfft_reg<12, 18>(c, a, inv, nf);
-      case 288: return run_zfft_reg<16, 18>(c, a, inv, nf);
-      case 324: return run_zfft_reg<18, 18>(c, a, inv, nf);
-      case 432: return run_zfft_reg<18, 24>(c, a, inv, nf);
-      case 576: return run_zfft_reg<24, 24>(c, a, inv, nf);
+      case 18: return run_zfft_reg<3, 6>(c, a, inv, nf, np);
+      case 36: return run_zfft_reg<6, 6>(c, a, inv, nf, np);
+      case 54: return run_zfft_reg<6, 9>(c, a, inv, nf, np);
+      case 72: return run_zfft_reg<8, 9>(c, a, inv, nf, np);
+      case 108: return run_zfft_reg<9, 12>(c, a, inv, nf, np);
+      case 162: return run_zfft_reg<9, 18>(c, a, inv, nf, np);
+      case 216: return run_zfft_reg<12, 18>(c, a, inv, nf, np);
+      case 288: return run_zfft_reg<16, 18>(c, a, inv, nf, np);
+      case 324: return run_zfft_reg<18, 18>(c, a, inv, nf, np);
+      case 432: return run_zfft_reg<18, 24>(c, a, inv, nf, np);
+      case 576: return run_zfft_reg<24, 24>(c, a, inv, nf, np);
       default: break;
     }
   }
   switch (c.d.Lz) {
-    case 12: return run_zfft_reg<4, 3>(c, a, inv, nf);
-    case 24: return run_zfft_reg<4, 6>(c, a, inv, nf);
-    case 48: return run_zfft_reg<6, 8>(c, a, inv, nf);
-    case 96: return run_zfft_reg<8, 12>(c, a, inv, nf);
-    case 144: return run_zfft_reg<12, 12>(c, a, inv, nf);
-    case 192: return run_zfft_reg<12, 16>(c, a, inv, nf);
-    case 384: return run_zfft_reg<16, 24>(c, a, inv, nf);
-    case 768: return run_zfft_reg<24, 32>(c, a, inv, nf);
+    case 12: return run_zfft_reg<4, 3>(c, a, inv, nf, np);
+    case 24: return run_zfft_reg<4, 6>(c, a, inv, nf, np);
+    case 48: return run_zfft_reg<6, 8>(c, a, inv, nf, np);
+    case 96: return run_zfft_reg<8, 12>(c, a, inv, nf, np);
+    case 144: return run_zfft_reg<12, 12>(c, a, inv, nf, np);
+    case 192: return run_zfft_reg<12, 16>(c, a, inv, nf, np);
+    case 384: return run_zfft_reg<16, 24>(c, a, inv, nf, np);
+    case 768: return run_zfft_reg<24, 32>(c, a, inv, nf, np);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1295,14 +1292,16 @@ static RegZ<V> regz_args(Ctx& c, const V* const* in, V* const* out, int nf, bool
 
 static bool use_zreg(const Ctx& c) { return reg_fft_length(c.d.Lz); }
 
-static hipError_t zfft_reg64(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv) {
+static hipError_t zfft_reg64(Ctx& c, double2* const* in, double2* const* out, int nf, bool inv, int np) {
   const double2* cin[6];
   for (int f = 0; f < nf; ++f) cin[f] = in[f];
-  return zfft_reg(c, regz_args<double2>(c, cin, out, nf, inv, c.twz), inv, nf);
+  return zfft_reg(c, regz_args<double2>(c, cin, out, nf, inv, c.twz), inv, nf, np);
 }
 
-hipError_t launch_zfft32(Ctx& c, const float2* const* in, float2* const* out, int nf, bool inv) {
-  return zfft_reg(c, regz_args<float2>(c, in, out, nf, inv, c.twzf), inv, nf);
+hipError_t launch_zfft(Ctx& c, float2* const* in, float2* const* out, int nf, bool inv, int np) {
+  const float2* cin[6];
+  for (int f = 0; f < nf; ++f) cin[f] = in[f];
+  return zfft_reg(c, regz_args<float2>(c, cin, out, nf, inv, c.twzf), inv, nf, np);
 }
 
 // One instantiation of the span kernel at the unpadded length Lz = Mz: the same
@@ -1369,39 +1368,39 @@ hipError_t launch_span_inverse_unpadded(Ctx& c, double2* const* inout, int nf) {
   return hipGetLastError();
 }
 
-hipError_t launch_xpass32(Ctx& c) {
+hipError_t launch_xpass(Ctx& c, float2* const* Z, int np) {
   RegX<float2> a{};
-  for (int f = 0; f < 6; ++f) a.in[f] = c.Zf[f];
-  for (int f = 0; f < 3; ++f) a.out[f] = c.Zf[f];
+  for (int f = 0; f < 6; ++f) a.in[f] = Z[f];
+  for (int f = 0; f < 3; ++f) a.out[f] = Z[f];
   a.Mx = c.d.Mx;
-  a.nlines = (long)c.d.Py * c.d.Lz;
+  a.nlines = (long)np * c.d.Lz;
   a.re_p = c.prm.re_p;
   a.scale = 1.0 / ((double)c.d.Lx * (double)c.d.Lz);
   a.tw = c.twxf;
   return xpass_reg(c, a);
 }
 
-hipError_t launch_xpass(Ctx& c) {
+hipError_t launch_xpass(Ctx& c, double2* const* Z, int np) {
   const Dims& d = c.d;
   XArgs a{};
-  for (int f = 0; f < 6; ++f) a.in[f] = c.Z[f];
+  for (int f = 0; f < 6; ++f) a.in[f] = Z[f];
   // outputs overwrite Z[0..2] line by line: each block reads its own lines fully
   // before writing them, and no block touches another block's lines
-  for (int f = 0; f < 3; ++f) a.out[f] = c.Z[f];
+  for (int f = 0; f < 3; ++f) a.out[f] = Z[f];
   a.Mx = d.Mx;
   a.Lx = d.Lx;
   int lpb = 2048 / (3 * d.Lx);
   if (lpb < 1) lpb = 1;
   a.LPB = lpb;
-  a.nlines = (long)d.Py * d.Lz;
+  a.nlines = (long)np * d.Lz;
   a.re_p = c.prm.re_p;
   a.scale = 1.0 / ((double)d.Lx * (double)d.Lz);
   a.pl = make_plan(d.Lx);
   a.tw = c.twx;
   if (reg_fft_length(d.Lx)) {
     RegX<double2> r{};
-    for (int f = 0; f < 6; ++f) r.in[f] = c.Z[f];
-    for (int f = 0; f < 3; ++f) r.out[f] = c.Z[f];
+    for (int f = 0; f < 6; ++f) r.in[f] = Z[f];
+    for (int f = 0; f < 3; ++f) r.out[f] = Z[f];
     r.Mx = d.Mx;
     r.nlines = a.nlines;
     r.re_p = a.re_p;
