@@ -5,15 +5,17 @@
 //   omega_y:  x = Q V diag(1 / sigma) L b
 //   v:        x = Q V s (L b + a l1 - B q),  a, B from the two wall conditions
 // with L, V, the eigenvalues and the wall vectors shared by all modes and by
-// both equations.  A block takes one parity and 64 real columns: the right-hand
+// both equations.  A block takes one parity and 64 or 32 real columns: the right-hand
 // sides are staged in LDS, Y = L B runs on the FP64 matrix cores, Y is scaled
 // per (row, mode) and corrected (v) in registers and written back to LDS as the B
 // operand of X = V Y; the first coefficient is minus the sum of the others (the
 // wall condition x(1) = 0), so it costs adds, not a row block.
 //
 // Bound: the matrix products, 2 m^2 multiply-adds per real column and parity
-// (5 GFLOP per equation at 256x193x256, 38 TFLOP/s for v and 45 for omega_y,
-// against the 72 that a large FP64 library product reaches).  They replace a
+// (5 GFLOP per equation at 256x193x256, 35 TFLOP/s for v and 41 for omega_y,
+// against the 72 that a large FP64 library product reaches); the rest is the
+// blocks' loads, scaling and stores (65 of 138 us, 51 of 119), which overlap the
+// products of other blocks in part only.  They replace a
 // stream of stored v inverses (1.55 GB, one pair per k^2), which HBM bound:
 // v 0.429 -> 0.131 ms and omega_y 0.139 -> 0.110 ms at 256x193x256, v 3.0 ->
 // 0.85 ms at 512x257x512.
@@ -99,19 +101,13 @@ __device__ void mean_mode_block(const HsArgs& a, double* sm) {
   }
 }
 
-constexpr int kHsCols = 64;      // real columns per block
-constexpr int kHsThreads = 256;  // four wavefronts
-
 // IS_V: the v system (right-hand-side rows from p = 2) or omega_y (from p = 1).
-// The four waves split the 16-row blocks into WR groups of up to RB and the
-// columns into 4 / WR groups of CB = WR 16-column blocks.  WR = 2 from four row
-// blocks on (each A fragment feeds two matrix ops, the waves of a SIMD carry
-// equal work); below, one column block per wave and every row block, so no
-// wave idles.
-template <bool IS_V, int WR, int RB>
+// A block takes CT real columns; its WR x WC waves split the 16-row blocks into
+// WR groups of up to RB and the columns into WC groups of CB 16-column blocks.
+template <bool IS_V, int CT, int WR, int WC, int RB>
 __device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
   using MF = Mf<double>;
-  constexpr int CT = kHsCols, CB = WR;
+  constexpr int CB = CT / 16 / WC, NT = 64 * WR * WC;
   const int par = blockIdx.y;
   const int tile = (int)blockIdx.x - 1;
   if (tile < 0) {
@@ -121,30 +117,30 @@ __device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
   const int m = par ? a.m[1] : a.m[0];
   const int MB = (m + 15) / 16, KP = (m + 7) / 8, R = 16 * MB;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int wr = WR == 2 ? wave >> 1 : 0, wc = WR == 2 ? wave & 1 : wave;
+  const int wr = wave / WC, wc = wave % WC;
   const int rb0 = wr * RB;  // this wave's row blocks rb0 .. rb0 + RB - 1 (those < MB)
   const int cl = wc * CB * 16 + (lane & 15);  // its first column in the tile
   const long col0 = (long)tile * (CT / 2);    // first complex column
-  double* red = sB + (16 * ((a.m[0] + 15) / 16)) * CT;  // [2][CT][2]
+  double* red = sB;  // [WR][CT][2], between the products' uses of sB
 
   // stage B: matrix row r holds the right-hand side of point p = r + 1; rows
   // without one (v at p = 1, the padding) and columns past the end are zero
   {
     const double2* ro = IS_V ? (par ? a.rhs[0][1] : a.rhs[0][0]) : (par ? a.rhs[1][1] : a.rhs[1][0]);
-    constexpr int off = IS_V ? 1 : 0, SL = 6;
+    constexpr int off = IS_V ? 1 : 0, SL = (16 * WR * RB * CT / 2 + NT - 1) / NT;  // every load in flight at once
     const int nst = R * (CT / 2), last = m - 1 - off;
-    for (int i0 = threadIdx.x; i0 < nst; i0 += SL * kHsThreads) {
+    for (int i0 = threadIdx.x; i0 < nst; i0 += SL * NT) {
       double2 v[SL];
 #pragma unroll
       for (int u = 0; u < SL; ++u) {
-        const int idx = i0 + u * kHsThreads, r = idx / (CT / 2) - off;
+        const int idx = i0 + u * NT, r = idx / (CT / 2) - off;
         const long cc = col0 + idx % (CT / 2);
         const bool in = idx < nst && r >= 0 && r <= last && cc < a.ncol;
         v[u] = in ? ro[(long)r * a.ncol + cc] : make_double2(0, 0);
       }
 #pragma unroll
       for (int u = 0; u < SL; ++u) {
-        const int idx = i0 + u * kHsThreads;
+        const int idx = i0 + u * NT;
         if (idx < nst) *reinterpret_cast<double2*>(sB + 2 * idx) = v[u];
       }
     }
@@ -239,26 +235,32 @@ __device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
         d1[cb] += __shfl_xor(d1[cb], o);
         d2[cb] += __shfl_xor(d2[cb], o);
       }
-      if (WR == 2 && lane < 16) {
+      if (WR > 1 && lane < 16) {
         red[(wr * CT + cl + 16 * cb) * 2] = d1[cb];
         red[(wr * CT + cl + 16 * cb) * 2 + 1] = d2[cb];
       }
     }
-    if constexpr (WR == 2) __syncthreads();
+    if constexpr (WR > 1) __syncthreads();
     const double* wall = par ? a.wall[1] : a.wall[0];
     double wa[CB], wb[CB];
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
       double e1 = d1[cb], e2 = d2[cb];
-      if constexpr (WR == 2) {
+      if constexpr (WR > 1) {
         const double* r0 = red + (cl + 16 * cb) * 2;
-        e1 = r0[0] + r0[2 * CT];
-        e2 = r0[1] + r0[2 * CT + 1];
+        e1 = r0[0];
+        e2 = r0[1];
+#pragma unroll
+        for (int g = 1; g < WR; ++g) {
+          e1 += r0[2 * CT * g];
+          e2 += r0[2 * CT * g + 1];
+        }
       }
       const double* w = wall + 4 * min(col0 + ((cl + 16 * cb) >> 1), a.ncol - 1);
       wa[cb] = w[0] * e1 + w[1] * e2;
       wb[cb] = w[2] * e1 + w[3] * e2;
     }
+    if constexpr (WR > 1) __syncthreads();
 #pragma unroll
     for (int t = 0; t < RB; ++t)
 #pragma unroll
@@ -274,6 +276,7 @@ __device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
   __syncthreads();
   product(par ? a.V[1] : a.V[0]);
 
+  if constexpr (WR > 1) __syncthreads();
   // x_0 = -sum of x_1 .. x_m (padding rows are zero)
   double sum[CB] = {};
 #pragma unroll
@@ -284,9 +287,9 @@ __device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
       for (int e = 0; e < 4; ++e) sum[cb] += acc[t][cb][e];
 #pragma unroll
     for (int o = 16; o < 64; o <<= 1) sum[cb] += __shfl_xor(sum[cb], o);
-    if (WR == 2 && wr == 1 && lane < 16) red[(2 * CT + cl + 16 * cb)] = sum[cb];
+    if (WR > 1 && lane < 16) red[wr * CT + cl + 16 * cb] = sum[cb];
   }
-  if constexpr (WR == 2) __syncthreads();
+  if constexpr (WR > 1) __syncthreads();
   // the mean mode and the span Nyquist column are not solved here (PF:247)
   const long ncold = 2 * a.ncol;
 #pragma unroll
@@ -295,7 +298,8 @@ __device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
     if (cm >= a.ncol || cm == 0 || (int)((unsigned)cm / (unsigned)a.Mx) == a.Mz / 2) continue;
     double* o = (IS_V ? a.out[0] : a.out[1]) + (long)par * ncold + col;
     if (wr == 0 && lane < 16) {
-      if constexpr (WR == 2) sum[cb] += red[2 * CT + cl + 16 * cb];
+#pragma unroll
+      for (int g = 1; g < WR; ++g) sum[cb] += red[g * CT + cl + 16 * cb];
       o[0] = -sum[cb];
     }
 #pragma unroll
@@ -309,11 +313,11 @@ __device__ __forceinline__ void hsolve_block(const HsArgs& a, double* sB) {
 }
 
 // Both equations in one launch (first = 0, two layers), or one of them.
-template <int WR, int RB>
-__global__ __launch_bounds__(kHsThreads, RB == 4 ? 2 : 3) void k_hsolve(HsArgs a, int first) {
-  extern __shared__ double sB[];  // [16 MB rows][kHsCols], then the wall sums
-  if (first + blockIdx.z == 0) hsolve_block<true, WR, RB>(a, sB);
-  else hsolve_block<false, WR, RB>(a, sB);
+template <int CT, int WR, int WC, int RB, int WPS>
+__global__ __launch_bounds__(64 * WR * WC, WPS) void k_hsolve(HsArgs a, int first) {
+  extern __shared__ double sB[];  // [16 MB rows][CT]
+  if (first + blockIdx.z == 0) hsolve_block<true, CT, WR, WC, RB>(a, sB);
+  else hsolve_block<false, CT, WR, WC, RB>(a, sB);
 }
 
 // The wall matrices of every column and parity (wall_matrix of helmholtz.h).
@@ -374,17 +378,13 @@ hipError_t launch_wall_setup(Ctx& c) {
   return hipGetLastError();
 }
 
-template <int WR, int RB>
+template <int CT, int WR, int WC, int RB, int WPS>
 static hipError_t run_hsolve(Ctx& c, const HsArgs& a, int first, int count) {
-  const size_t shm = sizeof(double) * ((size_t)kHsCols * 16 * ((a.m[0] + 15) / 16) + 5 * kHsCols);
-  const unsigned tiles = (unsigned)((2 * a.ncol + kHsCols - 1) / kHsCols);
+  const size_t shm = sizeof(double) * (size_t)CT * 16 * ((a.m[0] + 15) / 16);
+  const unsigned tiles = (unsigned)((2 * a.ncol + CT - 1) / CT);
   if (sizeof(double) * 8ull * a.Ny > shm) return hipErrorInvalidValue;  // the mean-mode block's arrays
-  if (shm > 65536) {
-    const hipError_t e =
-        hipFuncSetAttribute((const void*)k_hsolve<WR, RB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL((k_hsolve<WR, RB>), dim3(tiles + 1, 2, count), dim3(kHsThreads), shm, c.stream, a, first);
+  hipLaunchKernelGGL((k_hsolve<CT, WR, WC, RB, WPS>), dim3(tiles + 1, 2, count), dim3(64 * WR * WC), shm, c.stream, a,
+                     first);
   return hipGetLastError();
 }
 
@@ -404,13 +404,24 @@ hipError_t launch_hsolve(Ctx& c, int first, int count) {
   a.c3p = c.cl3[1 - c.hcur];
   a.tmean = c.tmean;
   a.inv0 = c.inv0;
-  switch ((a.m[0] + 15) / 16) {  // row blocks of the even half system (the odd one has as many or one less)
-    case 1: return run_hsolve<1, 1>(c, a, first, count);
-    case 2: return run_hsolve<1, 2>(c, a, first, count);
-    case 3: return run_hsolve<1, 3>(c, a, first, count);
-    case 4: return run_hsolve<2, 2>(c, a, first, count);
-    case 5: case 6: return run_hsolve<2, 3>(c, a, first, count);
-    case 7: case 8: return run_hsolve<2, 4>(c, a, first, count);
+  // CT, WR, WC, RB by the row blocks of the even half system (the odd one has as
+  // many or one less).  The resident blocks run in step (they start together and
+  // a launch is a few rounds of them), so loads, products and stores overlap the
+  // less the longer a block is: with 32 columns and a wave's tile of 2 x 2 (7, 8
+  // row blocks) instead of 64 and 4 x 2, 16 waves a CU fit in the place of 8, and
+  // the products reach 49 TFLOP/s in the place of 43 (v / omega_y, us: 256x257x256
+  // 235 / 202 -> 204 / 176, 256x225x256 200 / 175 -> 175 / 150; 96x97x96 21 / 15.3
+  // -> 17.5 / 14.1; 64x65x64 11.4 / 8.9 -> 10.0 / 7.8).  From 4 to 6 row blocks
+  // 64 columns stay: 256x193x256 138 / 117, with 32 columns 148 / 123 to 152 / 132
+  // (one wave per row block 181 / 148: six waves load the four SIMDs unevenly),
+  // 192x161x192 76 / 63 against 76 / 62, 128x129x128 30 / 23 against 34 / 23.
+  switch ((a.m[0] + 15) / 16) {
+    case 1: return run_hsolve<64, 1, 4, 1, 3>(c, a, first, count);
+    case 2: return run_hsolve<32, 2, 2, 1, 4>(c, a, first, count);
+    case 3: return run_hsolve<32, 3, 1, 1, 4>(c, a, first, count);
+    case 4: return run_hsolve<64, 2, 2, 2, 3>(c, a, first, count);
+    case 5: case 6: return run_hsolve<64, 2, 2, 3, 3>(c, a, first, count);
+    case 7: case 8: return run_hsolve<32, 4, 1, 2, 4>(c, a, first, count);
     default: return hipErrorInvalidValue;
   }
 }
