@@ -352,6 +352,24 @@ int slab_planes(const Dims& d, size_t plane) {
   return (d.Py + 2 * pairs - 1) / (2 * pairs);
 }
 
+// Whether the wall-normal transforms run as FFTs.  CHF_Y_TRANSFORMS=matrix in the
+// environment keeps the cos-table products.
+bool ydct_form(const Dims& d) {
+  const char* ytr = std::getenv("CHF_Y_TRANSFORMS");
+  return !(ytr && std::strcmp(ytr, "matrix") == 0) && ydct_length_supported(d.N) && d.ncol % 16 == 0;
+}
+
+// Values from one plane to the next of the fields at the padded wall-normal
+// points.  The wall-normal FFTs read and write a few columns of every plane at a
+// time; planes a multiple of 512 KB apart put those on the same memory channels,
+// so 80 values (640 or 1280 bytes) go between them (us without / with, FP64
+// 512x257x512 synthesis 3008 / 2971, analysis 1440 / 1165, step 18413 / 18000,
+// mixed 10894 / 10736; 512x193x256 6471 / 6394; 256x193x256 2877 / 2856; planes
+// of 128 KB, 128x129x128, 503 / 508).
+long yplane_values(const Dims& d, size_t value_bytes) {
+  return d.ncol + (d.ncol * value_bytes % (size_t(512) << 10) == 0 ? 80 : 0);
+}
+
 // Padded-plane work arrays of `planes` wall-normal planes in the place of the
 // present ones, which stay where an allocation fails.
 int alloc_padded(Ctx* c, int planes) {
@@ -426,7 +444,8 @@ int build(Ctx* c, DegreeCache& cache) {
   }
   CHF_TRY(dalloc(c, &c->au0, d.Ny));
   CHF_TRY(dalloc(c, &c->w0, d.Ny));
-  const size_t ysz = (size_t)d.Py * d.ncol;
+  d.yplane = ydct_form(d) ? yplane_values(d, p.precision == 0 ? sizeof(double2) : sizeof(float2)) : d.ncol;
+  const size_t ysz = (size_t)d.Py * d.yplane;
   if (p.precision == 0) {
     for (auto& y : c->Y) CHF_TRY(dalloc(c, &y, ysz));
   } else {
@@ -595,11 +614,8 @@ int build(Ctx* c, DegreeCache& cache) {
   // tables of the FFT forms of the wall-normal transforms (2N-point and
   // N-point twiddles, the type-III DCT pre-twiddles e^{i pi k/2N} =
   // cos(pi k/2N) + i cos(pi (N-k)/2N)); their blocks take 8 (FP64) or 16
-  // (FP32) adjacent columns.  CHF_Y_TRANSFORMS=matrix in the environment keeps
-  // the cos-table products.
-  const char* ytr = std::getenv("CHF_Y_TRANSFORMS");
-  const bool ymatrix = ytr && std::strcmp(ytr, "matrix") == 0;
-  if (!ymatrix && ydct_length_supported(d.N) && d.ncol % 16 == 0) {
+  // (FP32) adjacent columns.
+  if (ydct_form(d)) {
     const int N = d.N;
     std::vector<double2> ty = twiddles(2 * N), tn = twiddles(N);
     ty.insert(ty.end(), tn.begin(), tn.end());
@@ -723,7 +739,7 @@ hipError_t physical_products(Ctx* c, V* const* Y, V* const* Z) {
   auto planes = [&](int y0, int np, int z0) {
     V *y[6], *z[6];
     for (int f = 0; f < 6; ++f) {
-      y[f] = Y[f] + (long)y0 * d.ncol;
+      y[f] = Y[f] + (long)y0 * d.yplane;
       z[f] = Z[f] + (long)z0 * d.Lz * d.Mx;
     }
     hipError_t e = timed(c, K_ZFFT_INV, [&] { return launch_zfft(*c, y, z, 6, true, np); });

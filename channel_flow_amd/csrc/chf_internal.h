@@ -38,6 +38,7 @@ struct Dims {
   int no;     // odd degrees 1,3,..: (N+1)/2
   int Pn;     // N+1-point grid folded by parity: N/2+1
   long ncol;  // complex columns per plane: Mz*Mx
+  long yplane;  // values from one plane to the next in the arrays Y, Yf
   int ngroups;  // (kx,|kz|) groups: Mx*(Mz/2)
   int nclass;   // stored inverses: operator classes (groups with bitwise-equal k^2 share one); else 1
   int nblocks;  // stored inverses: solve blocks, up to two groups of one class each
@@ -121,7 +122,7 @@ struct Ctx {
   // (FFT transforms only)
   bool hdefer = false;
   // nonlinear work
-  double2* Y[6] = {};     // [Py][Mz][Mx]   wall-normal points, Fourier modes
+  double2* Y[6] = {};     // [Py][yplane: Mz Mx, padding]   wall-normal points, Fourier modes
   double2* Z[6] = {};     // [zplanes][Lz][Mx]  wall-normal + span points, x modes
   float2* Yf[6] = {};     // mixed form: FP32 copies of Y and Z
   float2* Zf[6] = {};

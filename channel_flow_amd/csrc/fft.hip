@@ -200,8 +200,8 @@ static hipError_t launch_z(Ctx& c, double2* const* in, double2* const* out, int 
   a.Mz = d.Mz;
   a.Lz = d.Lz;
   a.TX = pick_tx(d.Mx, d.Lz);
-  a.in_plane = (long)(inv ? d.Mz : d.Lz) * d.Mx;
-  a.out_plane = (long)(inv ? d.Lz : d.Mz) * d.Mx;
+  a.in_plane = inv ? d.yplane : (long)d.Lz * d.Mx;
+  a.out_plane = inv ? (long)d.Lz * d.Mx : d.yplane;
   a.pl = make_plan(d.Lz);
   a.tw = c.twz;
   if (use_zreg(c)) return zfft_reg64(c, in, out, nf, inv, np);
@@ -1284,8 +1284,8 @@ static RegZ<V> regz_args(Ctx& c, const V* const* in, V* const* out, int nf, bool
   }
   a.Mx = c.d.Mx;
   a.Mz = c.d.Mz;
-  a.in_plane = (long)(inv ? c.d.Mz : c.d.Lz) * c.d.Mx;
-  a.out_plane = (long)(inv ? c.d.Lz : c.d.Mz) * c.d.Mx;
+  a.in_plane = inv ? c.d.yplane : (long)c.d.Lz * c.d.Mx;
+  a.out_plane = inv ? (long)c.d.Lz * c.d.Mx : c.d.yplane;
   a.tw = tw;
   return a;
 }

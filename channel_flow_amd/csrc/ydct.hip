@@ -80,7 +80,8 @@ constexpr int ymax(int a, int b) { return a > b ? a : b; }
 struct YArgs {
   const void* in[6];
   void* out[6];
-  long ncol;
+  long ncol;           // row stride of the fields
+  long yplane;         // ... of the padded points
   const double2* twL;  // e^{-2 pi i m / 2N}, m < 2N
   const double2* twN;  // e^{-2 pi i m / N},  m < N
   const double2* wq;   // e^{i pi k / 2N},    k < N
@@ -200,11 +201,11 @@ __global__ __launch_bounds__(YT<V>::TX* ymax(A1, A2)) void k_ycheb(YArgs a) {
   const int t = threadIdx.x / TX, tx = threadIdx.x - t * TX;
   V* buf = reinterpret_cast<V*>(smraw) + tx * SB;
   const long col = xcd_order(blockIdx.x, gridDim.x) * TX + tx;
-  const long nc = a.ncol;
+  const long ni = ANA ? a.yplane : a.ncol, no = ANA ? a.ncol : a.yplane;  // row strides
   const TI* in = static_cast<const TI*>(a.in[blockIdx.z]);
   TO* out = static_cast<TO*>(a.out[blockIdx.z]);
-  auto ld = [&](int r) { return ycvt<V>(in[(long)r * nc + col]); };
-  auto st = [&](int r, V v) { st_nt(out + (long)r * nc + col, ycvt<TO>(v)); };
+  auto ld = [&](int r) { return ycvt<V>(in[(long)r * ni + col]); };
+  auto st = [&](int r, V v) { st_nt(out + (long)r * no + col, ycvt<TO>(v)); };
   // H_q of the analysis from its two points
   auto hodd = [&](int q, V f, V g) { return q == 0 ? ysub(f, g) : yscale(ysub(f, g), (T)2); };
 
@@ -549,6 +550,7 @@ static YArgs y_args(const Ctx& c, const TI* const* in, TO* const* out, int nf) {
   }
   const int N = c.d.N;
   a.ncol = c.d.ncol;
+  a.yplane = c.d.yplane;
   a.twL = c.twy;
   a.twN = c.twy + 2 * N;
   a.wq = c.twy + 3 * N;
