@@ -214,29 +214,34 @@ __device__ __forceinline__ double2 widen(V v) {
 struct MArgs {
   LIn lx, lz;
   double2 *o1, *o3;
-  const double* tpts;  // [Pn][Ny]
-  int N, Ny, Pn;
+  const double* costab;  // cos(pi n / 2N), n < 4N
+  int N, Pn;
   long ncol;
 };
 
+// The cosines come from LDS: read as table rows from the L2, whose latency every
+// few degrees waited for, they made this block the longest of a small grid's launch
+// (us, rows / LDS: 128x97x128 mixed 22.9 / 15.8, 96x101x96 FP64 21.3 / 14.9,
+// 128x129x128 33.2 / 27.5, 64x65x64 9.9 / 8.2; eight or sixteen rows in flight 27 to 54).
 template <bool F32>
 __device__ void mean_points_block(const MArgs& a) {
   __shared__ double2 s1[260], s3[260];
+  __shared__ double ct[512];  // cos(pi m / N), m < 2N
   for (int l = threadIdx.x; l <= a.N; l += blockDim.x) {
     s1[l] = a.lx.at<F32>((long)l * a.ncol);
     s3[l] = a.lz.at<F32>((long)l * a.ncol);
   }
+  for (int m = threadIdx.x; m < 2 * a.N; m += blockDim.x) ct[m] = a.costab[2 * m];
   __syncthreads();
   for (int jj = threadIdx.x; jj < a.Pn; jj += blockDim.x) {
     double2 e1 = make_double2(0, 0), o1 = make_double2(0, 0);
     double2 e3 = make_double2(0, 0), o3 = make_double2(0, 0);
-    // T_l(y_jj) = cos(pi l jj/N): symmetric in l and jj, and (-1)^jj cos(pi (N - l) jj/N),
-    // so the reads run along jj, the lanes' index
-    const double sg = (jj & 1) ? -1.0 : 1.0;
+    int m = 0;  // l jj mod 2N: T_l(y_jj) = cos(pi l jj / N)
 #pragma unroll 4
     for (int l = 0; l <= a.N; ++l) {
-      const int r = 2 * l <= a.N ? l : a.N - l;
-      const double t = (2 * l <= a.N ? 1.0 : sg) * a.tpts[r * a.Ny + jj];
+      const double t = ct[m];
+      m += jj;
+      if (m >= 2 * a.N) m -= 2 * a.N;
       const double2 x1 = s1[l], x3 = s3[l];
       if (l & 1) {
         o1.x += t * x1.x; o1.y += t * x1.y;
@@ -255,7 +260,6 @@ __device__ void mean_points_block(const MArgs& a) {
     }
   }
 }
-
 
 struct HArgs {
   LIn lx, ly, lz;
@@ -539,7 +543,7 @@ __global__ __launch_bounds__(kSegCols* kMaxSegs) void k_hassemble_seg(HArgs a, M
 // Columns up to which the passes run in segments.  Measured (us, serial /
 // segments): kinematics 32x33x32 17 / 10, 96x101x96 mixed 40 / 17, 128x129x128
 // 51 / 30, 192x161x192 (18432 columns) 107 / 93, 256x193x256 (32768) 154 / 214;
-// h assembly 12 / 6.5, 26 / 17, 45 / 37, 66 / 61, 97 / 117.
+// h assembly 12 / 6.5, 26 / 12, 45 / 28, 66 / 54, 97 / 117.
 constexpr long kSegColumns = 24576;
 
 template <int SL>
@@ -628,9 +632,8 @@ hipError_t launch_hassemble(Ctx& c) {
   m.lz = a.lz;
   m.o1 = c.cl1[1 - c.hcur];
   m.o3 = c.cl3[1 - c.hcur];
-  m.tpts = c.tpts;
+  m.costab = c.costab;
   m.N = c.d.N;
-  m.Ny = c.d.Ny;
   m.Pn = c.d.Pn;
   m.ncol = c.d.ncol;
   if (a.ncol <= kSegColumns) {
