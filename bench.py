@@ -47,7 +47,7 @@ def dims(c):
     return d
 
 
-def kernel_work(d, precision="fp64", yfft=False):
+def kernel_work(d, precision="fp64", yfft=False, diag=False):
     """Algorithmic HBM bytes and flops per launch of each kernel class.
 
     Each stage reads its inputs once and writes its outputs once at the
@@ -63,7 +63,8 @@ def kernel_work(d, precision="fp64", yfft=False):
     no separate point-value pass.  In the mixed form with yfft the kinematics
     writes u, w, omega_x, omega_z in FP32 and the padded synthesis reads them
     so (v and omega_y stay FP64), and the analysis writes L^n's coefficients
-    in FP32, which the h assembly reads so.
+    in FP32, which the h assembly reads so.  diag: the v solve by the shared
+    diagonalisation, as omega_y's, in the place of the stored inverses.
     """
     w = 16 if precision == "fp64" else 8
     S = d["Ny"] * d["ncol"] * 16            # spectral field (FP64)
@@ -91,7 +92,7 @@ def kernel_work(d, precision="fp64", yfft=False):
         "rhs_o": ((4 * S if yfft else S + 2 * (Ny - 2) / Ny * S) + ro_rows / Ny * S,
                   yf * 2.0 * ((ne - 1) * ne + (no - 1) * no) * col),
         # v solve (omega_y of the mean group only) and the diagonalised omega_y solve
-        "solve": (inv_v_bytes + rv_rows / Ny * S + S, 0.0),
+        "solve": ((0 if diag else inv_v_bytes) + rv_rows / Ny * S + S, ws_flops if diag else 0.0),
         "wsolve": (ro_rows / Ny * S + S, ws_flops),
         # reads v, omega_y; writes u, w, omega_x, omega_z and the two brackets
         "kinematics": ((2 * S + 4 * S / 2 + 2 * S) if f32f else 8 * S, 0.0),
@@ -117,12 +118,13 @@ def roofline_of(name, avg_ms, work, precision="fp64"):
 
 
 # HIP kernel symbol behind each timed kernel class (the FP32 forms share symbols
-# with the FP64 ones; template arguments differ).
+# with the FP64 ones; template arguments differ; a symbol of two classes tells
+# neither its traffic).
 KERNEL_SYMBOL = {"synth_padded": "k_mfma_cos", "zfft_inv": "k_zfft", "xpass": "k_xpass_st",
                  "zfft_fwd": "k_zfft", "analysis": "k_mfma_cos", "hassemble": "k_hassemble",
                  "synth_points": "k_mfma_cos",
                  "rhs_v": "k_mfma_cos", "rhs_o": "k_mfma_cos",
-                 "solve": "k_solve", "kinematics": "k_kinematics", "wsolve": "k_wsolve"}
+                 "solve": "k_hsolve", "kinematics": "k_kinematics", "wsolve": "k_hsolve"}
 
 
 def measured_traffic(config, form, kernel):
@@ -188,7 +190,7 @@ def run_ensemble(steps, warmup):
     for m in members:
         key = f"{m['nnx']}x{m['nnz'] + 1}x{m['nny']}"
         sizes[key] = sizes.get(key, 0) + 1
-        work = kernel_work(dims(m), m.get("precision", "mixed"))
+        work = kernel_work(dims(m), m.get("precision", "mixed"), yfft=True, diag=True)
         step_bytes += sum(nbytes for nbytes, _ in work.values())
     agg_gbs = step_bytes / (t_graph / steps) / 1e9
     out = {
@@ -300,7 +302,8 @@ def run_form(cfg, ic_arrays, precision, steps, warmup, total, log, y_matrix=Fals
     # the transforms ran as FFTs when they have no tile choice
     yfft = "synth_padded" not in tiles
     return dict(ms_per_step=wall * 1e3 / steps, per_kernel=per_kernel, state=st, fields=fl,
-                setup_s=t_setup, tiles=tiles, yfft=yfft)
+                setup_s=t_setup, tiles=tiles, yfft=yfft,
+                diag="wsolve" in per_kernel)  # the stored inverses solve both in one launch
 
 
 def field_errors(cfg, mixed, ref):
@@ -382,14 +385,14 @@ def main(argv=None):
     head = "mixed" if "mixed" in runs else "fp64"
     r = runs[head]
     finite = all(np.all(np.isfinite(r["state"][k])) for k in ("vnp1", "omegaynp1", "au0"))
-    work = kernel_work(d, head, r["yfft"])
+    work = kernel_work(d, head, r["yfft"], r["diag"])
     pk = r["per_kernel"]
     dom = max(pk, key=lambda k: pk[k]["total_ms"])
     roof = roofline_of(dom, pk[dom]["avg_ms"], work, head)
     roof["traffic"] = measured_traffic(a.config, head, dom)
     for f, rr in runs.items():
         pf = "mixed" if f.startswith("mixed") else "fp64"
-        w = kernel_work(d, pf, rr["yfft"])
+        w = kernel_work(d, pf, rr["yfft"], rr["diag"])
         log(f, json.dumps({k: roofline_of(k, rr["per_kernel"][k]["avg_ms"], w, pf)
                            for k in rr["per_kernel"]}, indent=1))
     cpu = None if a.no_cpu_baseline else cpu_baseline(cfg)

@@ -150,9 +150,10 @@ long long chf_device_bytes(void* ctx);
 /* Instrumentation (no counterpart in the reference, whose only timer is the
  * mpi_wtime bracket of the solve loop, PF:217-229, 481-486).  With timing on,
  * every kernel launch of chf_solve/chf_nonlinear/chf_step is bracketed by HIP
- * events and the launches run one after another (without timing the omega_y
- * solve overlaps the v solve on a second stream), so each kernel class's time
- * is its own; chf_timing sums the elapsed time of kernel class `id`
+ * events and the launches run one after another, over all planes (without timing
+ * both equations share a launch and large grids run in slabs on two streams), so
+ * each kernel class's time is its own.  Turning it on may allocate (the planes
+ * that a large grid's slabs do without); chf_timing sums the elapsed time of kernel class `id`
  * (0 <= id < chf_kernel_count()) since the last chf_set_timing. */
 int chf_set_timing(void* ctx, int on);
 int chf_kernel_count(void);
