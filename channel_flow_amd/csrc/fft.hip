@@ -1106,7 +1106,10 @@ static bool reg_fft_length(int L) {
 template <int N1, int N2, class V>
 static hipError_t run_xpass_reg(Ctx& c, const RegX<V>& a) {
   using Gm = Geo<N1, N2>;
-  constexpr int NG = 256 / Gm::G;
+  // two wavefronts: the block's barriers couple fewer lines, and a small grid has
+  // more blocks (us, 256 / 128 / 64 threads: 36x33x36 15.6 / 14.7 / 14.5, 64x65x64
+  // 27.1 / 25.8 / 26.0, 96x97x96 mixed 41.1 / 40.2 / 39.5, 108x65x96 87 / 86 / 100)
+  constexpr int NG = 128 / Gm::G;
   const long blocks = (a.nlines + NG - 1) / NG;
   const size_t shm = sizeof(V) * (Gm::L + (size_t)NG * Gm::BUF);
   if (shm > 65536) {
