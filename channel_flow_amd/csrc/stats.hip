@@ -207,15 +207,25 @@ __global__ __launch_bounds__(kStatsThreads, 2) void k_line_stats(LineArgs a) {
   }
 }
 
-// The splits' partial sums [Ny][splits][12] to out [12][Ny].
+// The splits' partial results [Ny][splits][12] to out [12][Ny].  A mean, which the
+// lines' kx = 0 modes give, is NaN where a value of its plane is not finite, as a sum
+// over the values is: the squares' sum is NaN where a value is (no term of it is
+// negative), and an infinity is the largest value.
 __global__ __launch_bounds__(256) void k_stats_final(const double* __restrict__ part, int splits, int Ny, double coef,
                                                      double* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= 12 * Ny) return;
   const int q = i / Ny, k = i - q * Ny;
-  const double* p = part + (long)k * splits * 12 + q;
-  double v = p[0];
-  for (int s = 1; s < splits; ++s) v = q < 3 ? v : (q < 9 ? v + p[12 * s] : fmax(v, p[12 * s]));
+  const double* p = part + (long)k * splits * 12;
+  double v = p[q];
+  if (q < 3) {
+    for (int s = 0; s < splits; ++s) {
+      const double sq = p[12 * s + 3 + q], big = p[12 * s + 9 + q];
+      if (sq != sq || isinf(big)) v = __builtin_nan("");
+    }
+  } else {
+    for (int s = 1; s < splits; ++s) v = q < 9 ? v + p[12 * s + q] : fmax(v, p[12 * s + q]);
+  }
   out[i] = (q >= 3 && q < 9) ? v * coef : v;
 }
 
