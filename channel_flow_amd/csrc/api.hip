@@ -684,15 +684,14 @@ hipError_t timed(Ctx* c, int id, F&& launch) {
 }
 
 // Forms h^n's point values that nonlinear() left to the next solve, with the
-// FP64 point-value kernel in both forms: the values the right-hand-side
-// kernels would have formed, bit for bit.
+// FP64 point-value kernel in both forms: the values that the right-hand-side
+// kernels form, bit for bit.  They stay pending: the next solve forms them again
+// from the same coefficients, so reading a record does not change its launches.
 hipError_t form_h_points(Ctx* c) {
   if (!c->hdefer) return hipSuccess;
   const double2* hc[2] = {c->hvc, c->hgc};
   double2* ho[2] = {c->hv[c->hcur], c->hg[c->hcur]};
-  const hipError_t e = launch_ypoints(*c, hc, ho, 2);
-  if (e == hipSuccess) c->hdefer = false;
-  return e;
+  return launch_ypoints(*c, hc, ho, 2);
 }
 
 // Mixed form: the padded FP32 synthesis of fields f0 .. f0 + nf - 1 of
@@ -765,6 +764,7 @@ hipError_t physical_products(Ctx* c, V* const* Y, V* const* Z) {
 // right-hand-side kernels.
 int nonlinear(Ctx* c) {
   CHF_TRY(form_h_points(c));  // the previous step's, before the h assembly overwrites hvc, hgc
+  c->hdefer = false;
   // six fields in the order the streamwise pass pairs them: (u,v) (w,ox) (oy,oz)
   const double2* in6[6] = {c->u, c->v, c->w, c->ox, c->oy, c->oz};
   if (c->prm.precision == 0) {
@@ -1177,7 +1177,10 @@ int chf_timing(void* ctx, int id, double* total_ms, int* launches) {
 // forked from and joined to the ensemble stream).  Small members fill the GPU
 // together.  The AB2 history buffers swap every step, and the first step after a
 // record is loaded finds h^n's point values formed, so a graph is captured per
-// combination of the members' phases (normally two) and cached.
+// combination of the members' phases (normally two) and kept, up to kMaxGraphs:
+// members loaded, or stepped by themselves, between ensemble steps make further
+// combinations.  (24 members, ms: a step 3.1, with its graph's capture 4.5; issued
+// without a graph 4.4.)
 
 namespace {
 
@@ -1191,9 +1194,11 @@ struct Ens {
   hipStream_t origin = nullptr;
   hipEvent_t fork = nullptr;
   std::vector<hipEvent_t> join;
-  std::vector<EnsGraph> graphs;
+  std::vector<EnsGraph> graphs;  // the last used at the end
   std::string err;
 };
+
+constexpr size_t kMaxGraphs = 32;
 
 int ens_fail(Ens* e, const std::string& msg, int rc = -1) {
   e->err = msg;
@@ -1367,6 +1372,11 @@ int chf_ensemble_member(void* ens, int i, void** ctx) {
   return 0;
 }
 
+int chf_ensemble_graphs(void* ens) {
+  if (!ens) return -1;
+  return (int)static_cast<Ens*>(ens)->graphs.size();
+}
+
 int chf_ensemble_step(void* ens, int n) {
   if (!ens) return -1;
   Ens* e = static_cast<Ens*>(ens);
@@ -1379,19 +1389,24 @@ int chf_ensemble_step(void* ens, int n) {
   for (int s = 0; s < n; ++s) {
     std::vector<int> phase;
     for (Ctx* c : e->m) phase.push_back(step_phase(c));
-    hipGraphExec_t exec = nullptr;
-    for (auto& g : e->graphs)
-      if (g.phase == phase) exec = g.exec;
-    if (!exec) {
-      EnsGraph g;
-      const int rc = ens_capture(e, &g);
+    auto g = std::find_if(e->graphs.begin(), e->graphs.end(), [&](const EnsGraph& q) { return q.phase == phase; });
+    if (g != e->graphs.end()) {
+      std::rotate(g, g + 1, e->graphs.end());
+    } else {
+      if (e->graphs.size() >= kMaxGraphs) {  // the one not used for longest goes
+        ENS_TRY(hipStreamSynchronize(e->origin));
+        (void)hipGraphExecDestroy(e->graphs.front().exec);
+        e->graphs.erase(e->graphs.begin());
+      }
+      EnsGraph fresh;
+      const int rc = ens_capture(e, &fresh);
       if (rc) {
-        if (g.exec) (void)hipGraphExecDestroy(g.exec);
+        if (fresh.exec) (void)hipGraphExecDestroy(fresh.exec);
         return rc;
       }
-      exec = g.exec;
-      e->graphs.push_back(g);
+      e->graphs.push_back(fresh);
     }
+    const hipGraphExec_t exec = e->graphs.back().exec;
     ENS_TRY(hipGraphLaunch(exec, e->origin));
     for (Ctx* c : e->m) step_done(c);
   }

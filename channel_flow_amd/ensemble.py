@@ -55,6 +55,10 @@ class Ensemble:
         """n steps of every member; returns when they have completed."""
         self._check(self._lib.chf_ensemble_step(self._ens, int(n)), "chf_ensemble_step")
 
+    def graph_count(self) -> int:
+        """Captured step graphs that the ensemble holds."""
+        return self._lib.chf_ensemble_graphs(self._ens)
+
     def close(self):
         if self._ens:
             for m in self._members:

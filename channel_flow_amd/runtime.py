@@ -19,6 +19,7 @@ EXPORTS = ("chf_create", "chf_destroy", "chf_last_error", "chf_set_state", "chf_
            "chf_get_fields", "chf_dims", "chf_device_bytes", "chf_set_timing", "chf_kernel_count",
            "chf_kernel_name", "chf_timing", "chf_ensemble_create", "chf_ensemble_destroy",
            "chf_ensemble_last_error", "chf_ensemble_size", "chf_ensemble_member", "chf_ensemble_step",
+           "chf_ensemble_graphs",
            "chf_physical", "chf_physical_noalloc", "chf_statistics", "chf_tile_choice",
            "chf_set_tile_choice")
 
@@ -85,6 +86,7 @@ def load():
     lib.chf_ensemble_size.argtypes = [vp]
     lib.chf_ensemble_member.argtypes = [vp, ctypes.c_int, ctypes.POINTER(vp)]
     lib.chf_ensemble_step.argtypes = [vp, ctypes.c_int]
+    lib.chf_ensemble_graphs.argtypes = [vp]
     _lib = lib
     return lib
 

@@ -173,10 +173,8 @@ int chf_set_tile_choice(void* ctx, int id, int cb);
 
 /* Ensemble: n independent channels (any mix of grid sizes, Reynolds numbers
  * and precisions) advanced together, one step of every member being one
- * hipGraph launch: the members' right-hand sides as parallel branches, one
- * solve launch over every member's solve blocks, then the members'
- * kinematics and nonlinear terms as parallel branches (each member's result
- * is bit-identical to the same channel stepped alone).  The
+ * hipGraph launch whose parallel branches are the members' own steps (each
+ * member's result is bit-identical to the same channel stepped alone).  The
  * reference runs one channel per job, so these have no single counterpart;
  * each member is a full context whose state is exchanged with the calls
  * above (chf_set_state, chf_init_fields, chf_get_state, chf_get_fields), and
@@ -189,6 +187,10 @@ const char* chf_ensemble_last_error(void* ens);
 int chf_ensemble_size(void* ens);
 int chf_ensemble_member(void* ens, int i, void** ctx);
 int chf_ensemble_step(void* ens, int nsteps);
+/* Step graphs that the ensemble holds (instrumentation): one per combination of
+ * the members' phases met so far, two unless members were loaded or stepped by
+ * themselves between ensemble steps, and at most 32. */
+int chf_ensemble_graphs(void* ens);
 
 #ifdef __cplusplus
 }
