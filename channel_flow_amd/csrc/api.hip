@@ -213,17 +213,9 @@ int diagonalise(Ctx* c, const std::vector<double>& al, const std::vector<double>
       smax = std::max(smax, s);
       if (s > 0.0 && (smin == 0.0 || s < smin)) smin = s;
     }
-  const bool known = cache.count(d.N) != 0;
   std::array<la::HelmholtzHalf, 2>& h = cache[d.N];
   bool ok[2] = {false, false};
-  auto half = [&](int par) {
-    try {
-      ok[par] = known ? h[par].m > 0 : la::helmholtz_half(d.N, par, h[par]);
-      for (double s : {0.0, smin, smax}) ok[par] = ok[par] && la::helmholtz_verify(par, h[par], cc, s);
-    } catch (...) {
-      ok[par] = false;
-    }
-  };
+  auto half = [&](int par) { ok[par] = la::helmholtz_accept(d.N, par, h[par], cc, {0.0, smin, smax}); };
   std::thread other;
   try {
     other = std::thread(half, 1);

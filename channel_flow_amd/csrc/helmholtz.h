@@ -28,6 +28,7 @@
 // dense double inverses are (N = 32 .. 256: 1e-16 .. 1e-14 against 1e-14 .. 2e-11).
 #pragma once
 #include <cmath>
+#include <initializer_list>
 #include <vector>
 
 #include "eig.h"
@@ -39,6 +40,7 @@ using LD = long double;
 using LMat = std::vector<LD>;
 
 struct HelmholtzHalf {
+  bool ok = false;  // decomposed: set last, so false where that failed or threw on the way
   int m = 0;
   std::vector<double> L, V;               // m x m, row-major
   std::vector<double> lam, w1, w2, l1, q;  // m
@@ -130,6 +132,7 @@ inline bool linverse(const LMat& A, int m, LMat& out) {
 inline bool helmholtz_half(int N, int par, HelmholtzHalf& out) {
   const int n = par ? (N + 1) / 2 : N / 2 + 1, m = n - 1;
   if (m < 1) return false;
+  out.ok = false;
   out.m = m;
   half_points(N, par, out);
   LMat M0((size_t)m * m), M2((size_t)m * m), M0i;
@@ -202,6 +205,7 @@ inline bool helmholtz_half(int N, int par, HelmholtzHalf& out) {
     out.l1[j] = (double)L[(size_t)j * m];
     out.q[j] = (double)(lam[j] * ps);
   }
+  out.ok = true;
   return true;
 }
 
@@ -257,6 +261,7 @@ inline void helmholtz_solve(const HelmholtzHalf& h, bool is_v, double c, double 
 // one k^2 (v for k^2 > 0 only) to 1e-11 of the solution.  The direct solution is
 // the double LU's, refined with residuals in extended precision.
 inline bool helmholtz_verify(int par, const HelmholtzHalf& h, double c, double k2) {
+  if (!h.ok) return false;
   const int m = h.m, n = m + 1;
   for (int is_v = 0; is_v < (k2 > 0.0 ? 2 : 1); ++is_v) {
     const int nbc = is_v ? 2 : 1;  // wall rows, then the points p >= nbc
@@ -301,6 +306,19 @@ inline bool helmholtz_verify(int par, const HelmholtzHalf& h, double c, double k
     if (!(err <= 1e-11L * size)) return false;
   }
   return true;
+}
+
+// Whether a half system is decomposed (here, unless `h` is already) and
+// reproduces direct solves at each k^2; false, not an exception, without memory.
+inline bool helmholtz_accept(int N, int par, HelmholtzHalf& h, double c, std::initializer_list<double> k2s) noexcept {
+  try {
+    if (!h.ok && !helmholtz_half(N, par, h)) return false;
+    for (double k2 : k2s)
+      if (!helmholtz_verify(par, h, c, k2)) return false;
+    return true;
+  } catch (...) {
+    return false;
+  }
 }
 
 }  // namespace la
