@@ -888,7 +888,7 @@ int chf_set_state(void* ctx, const chf_state* st) {
   const Dims& d = c->d;
   const size_t fb = (size_t)d.Ny * d.ncol * sizeof(double2), mb = d.Ny * sizeof(double2);
   const int n = c->hcur, pv = 1 - c->hcur;
-  struct { double2* dst; const double* src; size_t bytes; } m[] = {
+  const HostArray m[] = {
       {c->cl1[n], st->clamb1n, mb}, {c->cl1[pv], st->clamb1nm1, mb},
       {c->cl3[n], st->clamb3n, mb}, {c->cl3[pv], st->clamb3nm1, mb},
       {c->au0, st->au0, mb}, {c->w0, st->w0, mb},
@@ -896,10 +896,8 @@ int chf_set_state(void* ctx, const chf_state* st) {
       {c->hv[n], st->rhsvn, fb}, {c->hg[n], st->rhsomegayn, fb},
       {c->hv[pv], st->unp1, fb}, {c->hg[pv], st->wnp1, fb}};
   for (auto& e : m)
-    if (!e.src) return fail(c, "chf_set_state: null array");
-  std::vector<HostArray> arrays;
-  for (auto& e : m) arrays.push_back({e.dst, const_cast<double*>(e.src), e.bytes});
-  CHF_TRY(copy_arrays(*c, arrays, false));
+    if (!e.host) return fail(c, "chf_set_state: null array");
+  CHF_TRY(copy_arrays(*c, m, 12, false));
   c->hdefer = false;  // h^n's point values are the record's
   // u, w, omega_x, omega_z and the brackets of the loaded v, omega_y, U, W
   CHF_TRY(load_kinematics(c));
@@ -912,7 +910,7 @@ int chf_get_state(void* ctx, const chf_state* st) {
   const Dims& d = c->d;
   const size_t fb = (size_t)d.Ny * d.ncol * sizeof(double2), mb = d.Ny * sizeof(double2);
   const int n = c->hcur, pv = 1 - c->hcur;
-  struct { const double2* src; double* dst; size_t bytes; } m[] = {
+  const HostArray m[] = {
       {c->cl1[n], st->clamb1n, mb}, {c->cl1[pv], st->clamb1nm1, mb},
       {c->cl3[n], st->clamb3n, mb}, {c->cl3[pv], st->clamb3nm1, mb},
       {c->au0, st->au0, mb}, {c->w0, st->w0, mb},
@@ -920,11 +918,9 @@ int chf_get_state(void* ctx, const chf_state* st) {
       {c->hv[n], st->rhsvn, fb}, {c->hg[n], st->rhsomegayn, fb},
       {c->hv[pv], st->unp1, fb}, {c->hg[pv], st->wnp1, fb}};
   for (auto& e : m)
-    if (!e.dst) return fail(c, "chf_get_state: null array");
+    if (!e.host) return fail(c, "chf_get_state: null array");
   CHF_TRY(form_h_points(c));
-  std::vector<HostArray> arrays;
-  for (auto& e : m) arrays.push_back({const_cast<double2*>(e.src), e.dst, e.bytes});
-  CHF_TRY(copy_arrays(*c, arrays, true));
+  CHF_TRY(copy_arrays(*c, m, 12, true));
   return 0;
 }
 
@@ -935,10 +931,9 @@ int chf_init_fields(void* ctx, const double* vnp1, const double* omegaynp1, cons
   if (!vnp1 || !omegaynp1 || !au0 || !w0) return fail(c, "chf_init_fields: null array");
   const Dims& d = c->d;
   const size_t fb = (size_t)d.Ny * d.ncol * sizeof(double2), mb = d.Ny * sizeof(double2);
-  CHF_TRY(copy_arrays(*c,
-                      {{c->v, const_cast<double*>(vnp1), fb}, {c->oy, const_cast<double*>(omegaynp1), fb},
-                       {c->au0, const_cast<double*>(au0), mb}, {c->w0, const_cast<double*>(w0), mb}},
-                      false));
+  const HostArray m[] = {{c->v, const_cast<double*>(vnp1), fb}, {c->oy, const_cast<double*>(omegaynp1), fb},
+                         {c->au0, const_cast<double*>(au0), mb}, {c->w0, const_cast<double*>(w0), mb}};
+  CHF_TRY(copy_arrays(*c, m, 4, false));
   // h^n = 0 and L^n = 0 so that the rotation in getnonlinear leaves h^{-1} = 0 (PF:2316)
   c->hdefer = false;
   for (double2* q : {c->hv[0], c->hv[1], c->hg[0], c->hg[1]})
@@ -990,12 +985,11 @@ int chf_get_fields(void* ctx, double* unp1, double* wnp1, double* omegaxnp1, dou
   Ctx* c = static_cast<Ctx*>(ctx);
   const size_t fb = (size_t)c->d.Ny * c->d.ncol * sizeof(double2);
   CHF_TRY(form_fields64(c));
-  struct { const double2* src; double* dst; } m[] = {
-      {c->u, unp1}, {c->w, wnp1}, {c->ox, omegaxnp1}, {c->oz, omegaznp1}};
-  std::vector<HostArray> arrays;
-  for (auto& e : m)
-    if (e.dst) arrays.push_back({const_cast<double2*>(e.src), e.dst, fb});
-  CHF_TRY(copy_arrays(*c, arrays, true));
+  HostArray m[4];
+  int count = 0;
+  for (const HostArray& a : {HostArray{c->u, unp1, fb}, {c->w, wnp1, fb}, {c->ox, omegaxnp1, fb}, {c->oz, omegaznp1, fb}})
+    if (a.host) m[count++] = a;
+  CHF_TRY(copy_arrays(*c, m, count, true));
   return 0;
 }
 
@@ -1079,7 +1073,8 @@ int chf_physical(void* ctx, int field, double* out) {
   CHF_TRY(form_fields64(c));
   CHF_TRY(launch_physical(*c, f, c->phys_c[0], c->phys_r[0]));
   const size_t n = (size_t)c->d.Ny * c->d.Mz * 2 * c->d.Mx;
-  CHF_TRY(copy_arrays(*c, {{c->phys_r[0], out, n * sizeof(double)}}, true));
+  const HostArray m[] = {{c->phys_r[0], out, n * sizeof(double)}};
+  CHF_TRY(copy_arrays(*c, m, 1, true));
   return 0;
 }
 

@@ -220,7 +220,7 @@ struct HostArray {
   void* host;
   size_t bytes;
 };
-hipError_t copy_arrays(Ctx& c, const std::vector<HostArray>& arrays, bool to_host);
+hipError_t copy_arrays(Ctx& c, const HostArray* arrays, int count, bool to_host);
 void hostcopy_retain();
 void hostcopy_release();
 

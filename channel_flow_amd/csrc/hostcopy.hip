@@ -13,14 +13,15 @@
 //
 // The pinned buffers and streams are kept in a process-wide pool per device, at
 // most kMaxLanes lanes (2 x kChunk bytes each); a lane belongs to one call at a
-// time, and the pool is freed when the last context is destroyed.
+// time, and the pool is freed when the last context is destroyed.  A copy itself
+// allocates nothing but its threads: without memory it has fewer lanes or threads,
+// or goes the plain way, and never throws.
+#include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 #include "chf_internal.h"
 
@@ -55,42 +56,59 @@ hipError_t lane_make(Lane& l) {
   return e;
 }
 
+struct DeviceLanes {
+  Lane idle[kMaxLanes];
+  int nidle = 0, made = 0;
+};
+
 struct Pool {
   std::mutex mu;
-  int users = 0;                          // contexts alive
-  std::map<int, std::vector<Lane>> idle;  // by device
-  std::map<int, int> made;
+  int users = 0;  // contexts alive
+  std::map<int, DeviceLanes> devices;
 } g_pool;
 
-// Up to `want` lanes of the current device (none if all are taken or cannot be made).
-std::vector<Lane> take_lanes(int device, int want) {
-  std::lock_guard<std::mutex> lock(g_pool.mu);
-  std::vector<Lane>& idle = g_pool.idle[device];
-  int& made = g_pool.made[device];
-  std::vector<Lane> got;
-  while ((int)got.size() < want) {
-    if (!idle.empty()) {
-      got.push_back(idle.back());
-      idle.pop_back();
-      continue;
-    }
-    if (made >= kMaxLanes) break;
-    Lane l;
-    if (lane_make(l) != hipSuccess) {
-      lane_free(l);
-      (void)hipGetLastError();
-      break;
-    }
-    ++made;
-    got.push_back(l);
-  }
-  return got;
-}
+// Lanes of the current device for one call, given back at its end.
+struct Lanes {
+  Lane lane[kMaxLanes];
+  int n = 0;
+  const int device;
 
-void give_lanes(int device, const std::vector<Lane>& lanes) {
-  std::lock_guard<std::mutex> lock(g_pool.mu);
-  for (const Lane& l : lanes) g_pool.idle[device].push_back(l);
-}
+  explicit Lanes(int dev) : device(dev) {}
+  Lanes(const Lanes&) = delete;
+
+  // up to `want` (none if all are taken or cannot be made)
+  void take(int want) {
+    std::lock_guard<std::mutex> lock(g_pool.mu);
+    DeviceLanes* d = nullptr;
+    try {
+      d = &g_pool.devices[device];
+    } catch (...) {
+      return;
+    }
+    while (n < want) {
+      if (d->nidle > 0) {
+        lane[n++] = d->idle[--d->nidle];
+        continue;
+      }
+      if (d->made >= kMaxLanes) break;
+      Lane l;
+      if (lane_make(l) != hipSuccess) {
+        lane_free(l);
+        (void)hipGetLastError();
+        break;
+      }
+      ++d->made;
+      lane[n++] = l;
+    }
+  }
+
+  ~Lanes() {
+    if (n == 0) return;
+    std::lock_guard<std::mutex> lock(g_pool.mu);
+    DeviceLanes& d = g_pool.devices.find(device)->second;
+    for (int i = 0; i < n; ++i) d.idle[d.nidle++] = lane[i];
+  }
+};
 
 struct Job {
   char* dev;
@@ -98,24 +116,43 @@ struct Job {
   size_t bytes;
 };
 
-hipError_t run_lane(Lane& l, const std::vector<Job>& jobs, std::atomic<size_t>& next, bool to_host) {
-  const Job* held[2] = {nullptr, nullptr};
+// The chunks of the arrays that go through the lanes, in turn.
+struct Jobs {
+  const HostArray* arrays;
+  int count;
+
+  static size_t chunks(const HostArray& a) { return a.bytes < kChunk ? 0 : (a.bytes + kChunk - 1) / kChunk; }
+  bool get(size_t i, Job& j) const {
+    for (int k = 0; k < count; ++k) {
+      const size_t n = chunks(arrays[k]), o = i * kChunk;
+      if (i < n) {
+        j = {(char*)arrays[k].dev + o, (char*)arrays[k].host + o, std::min(kChunk, arrays[k].bytes - o)};
+        return true;
+      }
+      i -= n;
+    }
+    return false;
+  }
+};
+
+hipError_t run_lane(Lane& l, const Jobs& jobs, std::atomic<size_t>& next, bool to_host) {
+  Job held[2] = {};  // bytes: of the transfer in flight into the buffer, or 0
   bool used[2] = {false, false};
   hipError_t e = hipSuccess;
   auto finish = [&](int b) {
-    if (!held[b]) return;
+    if (!held[b].bytes) return;
     e = hipEventSynchronize(l.done[b]);
-    if (e == hipSuccess) std::memcpy(held[b]->host, l.pin[b], held[b]->bytes);
-    held[b] = nullptr;
+    if (e == hipSuccess) std::memcpy(held[b].host, l.pin[b], held[b].bytes);
+    held[b].bytes = 0;
   };
   int b = 0;
-  for (size_t i = next++; i < jobs.size() && e == hipSuccess; i = next++, b ^= 1) {
-    const Job& j = jobs[i];
+  Job j;
+  for (; e == hipSuccess && jobs.get(next++, j); b ^= 1) {
     if (to_host) {
       e = hipMemcpyAsync(l.pin[b], j.dev, j.bytes, hipMemcpyDeviceToHost, l.stream);
       if (e == hipSuccess) e = hipEventRecord(l.done[b], l.stream);
       if (e != hipSuccess) break;
-      held[b] = &j;
+      held[b] = j;
       finish(b ^ 1);
     } else {
       if (used[b]) e = hipEventSynchronize(l.done[b]);
@@ -141,56 +178,50 @@ void hostcopy_retain() {
 void hostcopy_release() {
   std::lock_guard<std::mutex> lock(g_pool.mu);
   if (--g_pool.users > 0) return;
-  for (auto& d : g_pool.idle) {
-    g_pool.made[d.first] -= (int)d.second.size();
-    for (Lane& l : d.second) lane_free(l);
-    d.second.clear();
+  for (auto& d : g_pool.devices) {
+    for (int i = 0; i < d.second.nidle; ++i) lane_free(d.second.idle[i]);
+    d.second.made -= d.second.nidle;
+    d.second.nidle = 0;
   }
 }
 
-hipError_t copy_arrays(Ctx& c, const std::vector<HostArray>& arrays, bool to_host) {
+hipError_t copy_arrays(Ctx& c, const HostArray* arrays, int count, bool to_host) {
   size_t total = 0;
-  std::vector<Job> jobs;
-  for (const HostArray& a : arrays)
-    if (a.bytes >= kChunk) total += a.bytes;
-  std::vector<Lane> lanes;
-  if (total >= kMinBytes) lanes = take_lanes(c.device, std::min<int>(kMaxLanes, (int)(total / (4 * kChunk)) + 1));
-  for (const HostArray& a : arrays) {
-    if (lanes.empty() || a.bytes < kChunk) {
-      const hipError_t e = to_host ? hipMemcpyAsync(a.host, a.dev, a.bytes, hipMemcpyDeviceToHost, c.stream)
-                                   : hipMemcpyAsync(a.dev, a.host, a.bytes, hipMemcpyHostToDevice, c.stream);
-      if (e != hipSuccess) {
-        give_lanes(c.device, lanes);
-        return e;
-      }
-      continue;
-    }
-    for (size_t o = 0; o < a.bytes; o += kChunk)
-      jobs.push_back({(char*)a.dev + o, (char*)a.host + o, std::min(kChunk, a.bytes - o)});
+  for (int k = 0; k < count; ++k)
+    if (arrays[k].bytes >= kChunk) total += arrays[k].bytes;
+  Lanes lanes(c.device);
+  if (total >= kMinBytes) lanes.take((int)std::min<size_t>(kMaxLanes, total / (4 * kChunk) + 1));
+  for (int k = 0; k < count; ++k) {
+    const HostArray& a = arrays[k];
+    if (lanes.n > 0 && a.bytes >= kChunk) continue;
+    const hipError_t e = to_host ? hipMemcpyAsync(a.host, a.dev, a.bytes, hipMemcpyDeviceToHost, c.stream)
+                                 : hipMemcpyAsync(a.dev, a.host, a.bytes, hipMemcpyHostToDevice, c.stream);
+    if (e != hipSuccess) return e;
   }
   // the lanes' streams start after the work queued on the context's stream, and
   // what is queued there next starts after them
   hipError_t e = hipStreamSynchronize(c.stream);
-  if (e == hipSuccess && !lanes.empty()) {
-    std::atomic<size_t> next{0};
-    std::vector<hipError_t> err(lanes.size(), hipSuccess);
-    auto lane = [&](size_t i) {
-      if (i) err[i] = hipSetDevice(c.device);  // the caller's thread has it current
-      if (err[i] == hipSuccess) err[i] = run_lane(lanes[i], jobs, next, to_host);
-    };
-    std::vector<std::thread> threads;
-    threads.reserve(lanes.size());
+  if (e != hipSuccess || lanes.n == 0) return e;
+  const Jobs jobs{arrays, count};
+  std::atomic<size_t> next{0};
+  hipError_t err[kMaxLanes] = {};
+  auto lane = [&](int i) {
+    if (i) err[i] = hipSetDevice(c.device);  // the caller's thread has it current
+    if (err[i] == hipSuccess) err[i] = run_lane(lanes.lane[i], jobs, next, to_host);
+  };
+  std::thread threads[kMaxLanes];
+  for (int i = 1; i < lanes.n; ++i) {
     try {
-      for (size_t i = 1; i < lanes.size(); ++i) threads.emplace_back(lane, i);
-    } catch (const std::system_error&) {
-      // fewer threads: the others take the remaining chunks
+      threads[i] = std::thread(lane, i);
+    } catch (...) {
+      break;  // fewer threads: the others take the remaining chunks
     }
-    lane(0);
-    for (std::thread& t : threads) t.join();
-    for (hipError_t x : err)
-      if (e == hipSuccess) e = x;
   }
-  give_lanes(c.device, lanes);
+  lane(0);
+  for (std::thread& t : threads)
+    if (t.joinable()) t.join();
+  for (hipError_t x : err)
+    if (e == hipSuccess) e = x;
   return e;
 }
 

@@ -1,0 +1,68 @@
+// Test harness: the host copies (channel_flow_amd/csrc/hostcopy.hip, over
+// tests/native/hipstub) when their n-th allocation fails, a thread's start among
+// them, run by tests/test_hostcopy_host.py.  Every copy has to be whole, and the
+// pool's lanes have to be there again for the next one.
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+#include <vector>
+
+#include "../../channel_flow_amd/csrc/hostcopy.hip"
+
+static std::atomic<long> left{-1};  // allocations until one fails (-1: none does)
+
+static void* take(std::size_t n) {
+  if (left.load() >= 0 && left.fetch_sub(1) == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void* operator new(std::size_t n) { return take(n); }
+void* operator new[](std::size_t n) { return take(n); }
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+void operator delete[](void* p) noexcept { std::free(p); }
+void operator delete[](void* p, std::size_t) noexcept { std::free(p); }
+
+using namespace chf;
+
+// a small array, one of less than a chunk more than a few, and a long one
+static const std::size_t kBytes[3] = {1000, (std::size_t(7) << 20) + 13, std::size_t(45) << 20};
+
+static int copy(Ctx& c, std::vector<char>* dev, std::vector<char>* host, bool to_host) {
+  HostArray a[3];
+  for (int i = 0; i < 3; ++i) a[i] = {dev[i].data(), host[i].data(), kBytes[i]};
+  return (int)copy_arrays(c, a, 3, to_host);
+}
+
+int main() {
+  Ctx c;
+  std::vector<char> from[3], to[3];
+  for (int i = 0; i < 3; ++i) {
+    from[i].resize(kBytes[i]);
+    for (std::size_t k = 0; k < kBytes[i]; ++k) from[i][k] = (char)(k * 31 + (k >> 11) + i);
+  }
+  for (int to_host = 0; to_host < 2; ++to_host)
+    for (long n = 0;; ++n) {
+      hostcopy_retain();  // a fresh pool each time
+      bool hit = false;
+      for (int again = 0; again < 2; ++again) {  // the second copy without a failure
+        for (auto& t : to) t.assign(t.size(), 0);
+        for (int i = 0; i < 3; ++i) to[i].resize(kBytes[i]);
+        left = again ? -1 : n;
+        const int rc = to_host ? copy(c, from, to, true) : copy(c, to, from, false);
+        if (!again) hit = left.load() < 0;
+        left = -1;
+        for (int i = 0; i < 3; ++i)
+          if (rc || to[i] != from[i]) return std::printf("%ld %d array %d: rc %d\n", n, again, i, rc), 1;
+        if (again) {
+          const int lanes = g_pool.devices[0].nidle;
+          std::printf("%d %ld %d\n", to_host, n, lanes);
+          std::fflush(stdout);
+        }
+      }
+      hostcopy_release();
+      if (!hit) break;  // n is past the last allocation
+    }
+  return 0;
+}
