@@ -12,6 +12,7 @@
 // the chip idle for the latency of every batch of loads, in segments.
 #include "chf_internal.h"
 #include "fftreg.h"
+#include "segments.h"
 
 namespace chf {
 
@@ -540,12 +541,6 @@ __global__ __launch_bounds__(kSegCols* kMaxSegs) void k_hassemble_seg(HArgs a, M
     }
 }
 
-// Columns up to which the passes run in segments.  Measured (us, serial /
-// segments): kinematics 32x33x32 17 / 10, 96x101x96 mixed 40 / 17, 128x129x128
-// 51 / 30, 192x161x192 (18432 columns) 107 / 93, 256x193x256 (32768) 154 / 214;
-// h assembly 12 / 6.5, 26 / 12, 45 / 28, 66 / 54, 97 / 117.
-constexpr long kSegColumns = 24576;
-
 template <int SL>
 static hipError_t run_kin_seg(Ctx& c, const KinArgs& a, bool f32) {
   const dim3 grid((unsigned)((a.ncol + kSegCols - 1) / kSegCols) + 1), block(kSegCols * ((a.Ny + SL - 1) / SL));
@@ -589,7 +584,7 @@ hipError_t launch_kinematics(Ctx& c, bool f32) {
   a.Ny = d.Ny;
   a.ncol = d.ncol;
   a.c = c.prm.dt * 0.5 / c.prm.re;
-  if (d.ncol <= kSegColumns) {
+  if (kinematics_in_segments(d.ncol, c.f32_fields)) {
     const int sl = seg_len(d.Ny);
     switch (sl) {
       case 2: return run_kin_seg<2>(c, a, f32);
@@ -636,7 +631,7 @@ hipError_t launch_hassemble(Ctx& c) {
   m.N = c.d.N;
   m.Pn = c.d.Pn;
   m.ncol = c.d.ncol;
-  if (a.ncol <= kSegColumns) {
+  if (hassemble_in_segments(a.ncol, f32)) {
     switch (seg_len(c.d.Ny)) {
       case 2: return run_hasm_seg<2>(c, a, m, f32);
       case 4: return run_hasm_seg<4>(c, a, m, f32);
