@@ -258,8 +258,10 @@ inline void helmholtz_solve(const HelmholtzHalf& h, bool is_v, double c, double 
 }
 
 // Whether the decomposition reproduces direct solves of the half systems at
-// one k^2 (v for k^2 > 0 only) to 1e-11 of the solution.  The direct solution is
-// the double LU's, refined with residuals in extended precision.
+// one k^2 (v for k^2 > 0 only) to 1e-12 of the solution.  The direct solution is
+// the double LU's, refined with residuals in extended precision.  The bar has a
+// factor of ten: every degree from 4 to 256 comes within 1e-13, where the
+// refinement stops, for c from 1e-15 to 1e5 and k^2 to 1e8.
 inline bool helmholtz_verify(int par, const HelmholtzHalf& h, double c, double k2) {
   if (!h.ok) return false;
   const int m = h.m, n = m + 1;
@@ -303,7 +305,7 @@ inline bool helmholtz_verify(int par, const HelmholtzHalf& h, double c, double k
     helmholtz_solve(h, is_v != 0, c, k2, f.data(), x.data());
     LD err = step;  // not refined to the end: no better than the last correction
     for (int i = 0; i < n; ++i) err = std::max(err, std::fabs((LD)x[i] - ref[i]));
-    if (!(err <= 1e-11L * size)) return false;
+    if (!(err <= 1e-12L * size)) return false;
   }
   return true;
 }

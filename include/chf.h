@@ -58,7 +58,7 @@ typedef struct chf_state {
 
 /* Sets up the v and omega_y operators (replaces SCHEB PF:156 and the
  * get_coef_v/get_coef_omegay + zgetrf/zgetri set-up loop, PF:181-204).  Both are
- * diagonalised when the decomposition reproduces direct solves to 1e-11, else
+ * diagonalised when the decomposition reproduces direct solves to 1e-12, else
  * the half-system inverses of every (kx,|kz|) are built on the GPU and stored;
  * CHF_OMEGA_INVERSES=stored in the environment selects the stored inverses.
  * The wall-normal transforms (padded synthesis, analysis, Gauss-Lobatto
