@@ -219,11 +219,15 @@ __global__ __launch_bounds__(256) void k_stats_final(const double* __restrict__ 
   const double* p = part + (long)k * splits * 12;
   double v = p[q];
   if (q < 3) {
+    bool finite = true;  // no branch in the loop: its loads are in flight together
+#pragma unroll 8
     for (int s = 0; s < splits; ++s) {
       const double sq = p[12 * s + 3 + q], big = p[12 * s + 9 + q];
-      if (sq != sq || isinf(big)) v = __builtin_nan("");
+      finite = finite & (sq == sq) & (big < __builtin_inf());
     }
+    if (!finite) v = __builtin_nan("");
   } else {
+#pragma unroll 8
     for (int s = 1; s < splits; ++s) v = q < 9 ? v + p[12 * s + q] : fmax(v, p[12 * s + q]);
   }
   out[i] = (q >= 3 && q < 9) ? v * coef : v;
