@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void k_plane_stats(const double* __restrict__ 
 // Calls run.operator()<N1, N2>() for the split of a line of M complex points
 // (N1 <= N2: a thread keeps N1 values of each field); false without one.
 template <class F>
-static bool with_line_split(int M, F&& run) {
+static bool with_line_split(int M, F& run) {
   switch (M) {
     case 8: run.template operator()<2, 4>(); return true;
     case 12: run.template operator()<3, 4>(); return true;
@@ -320,10 +320,20 @@ static bool with_line_split(int M, F&& run) {
   }
 }
 
-struct HasSplit {
+// Lines that a block of a split transforms at a time; 0 without a split.
+struct LinesPerBlock {
+  int n = 0;
   template <int N1, int N2>
-  void operator()() {}
+  void operator()() {
+    n = LineGeo<N1, N2>::NG;
+  }
 };
+
+static int lines_per_block(int M) {
+  LinesPerBlock lines;
+  with_line_split(M, lines);
+  return lines.n;
+}
 
 struct RunC2r {
   Ctx& c;
@@ -381,12 +391,14 @@ hipError_t launch_physical(Ctx& c, const double2* field, double2* work, double* 
 }
 
 // Blocks per plane of the statistics: enough for six on every CU, each with at
-// least one group of lines.
+// least 16 lines and one group of lines (more of them would sum the plane means
+// for nothing: 16x33x512, 64 lines a group, 76 us with 32 blocks, 63 with 8).
 int stats_splits(const Ctx& c) {
-  return std::max(1, std::min(1536 / c.d.Ny, c.d.Mz / 16));
+  const int ng = lines_per_block(c.d.Mx);
+  return ng ? std::max(1, std::min({1536 / c.d.Ny, c.d.Mz / 16, (c.d.Mz + ng - 1) / ng})) : 1;
 }
 
-bool stats_in_lines(const Ctx& c) { return with_line_split(c.d.Mx, HasSplit{}); }
+bool stats_in_lines(const Ctx& c) { return lines_per_block(c.d.Mx) > 0; }
 
 hipError_t launch_statistics(Ctx& c, const double2* const* fields, double2* const* work, double* const* phys,
                              double* part, double* out) {
