@@ -128,11 +128,11 @@ KERNEL_SYMBOL = {"synth_padded": "k_mfma_cos", "zfft_inv": "k_zfft", "xpass": "k
 
 
 def measured_traffic(config, form, kernel):
-    """HBM bytes per launch of `kernel` from the committed counter summary
-    (FETCH_SIZE + WRITE_SIZE per dispatch, scaled by a device copy of known
-    size), or None when no summary for this workload and form is present or
-    the kernel's symbol is shared by several kernel classes."""
-    path = os.path.join(ROOT, "profiles", f"hbm_traffic_{config}_{form}.json")
+    """HBM bytes per launch of `kernel` from the committed counter summary of
+    --launch-probe (FETCH_SIZE + WRITE_SIZE per dispatch, scaled by a device
+    copy of known size), or None when no summary for this workload and form is
+    present or the kernel's symbol is shared by several kernel classes."""
+    path = os.path.join(ROOT, "profiles", f"hbm_launches_{config}_{form}.json")
     sym = KERNEL_SYMBOL.get(kernel)
     if not os.path.exists(path) or sym is None or list(KERNEL_SYMBOL.values()).count(sym) != 1:
         return None
@@ -155,6 +155,23 @@ def copy_probe(nbytes=1 << 30, reps=5):
         b.copy_(a)
     torch.cuda.synchronize()
     print(json.dumps({"copy_probe_bytes": nbytes, "reps": reps}), flush=True)
+    return 0
+
+
+def launch_probe(cfg, precision, steps):
+    """initial() and `steps` steps with every launch alone and over all planes, run
+    under the FETCH_SIZE and WRITE_SIZE counters: each dispatch is then one
+    launch of its kernel class."""
+    from channel_flow_amd import ic
+    from channel_flow_amd.channel import Channel
+    fields = ic.seeded_ic(cfg["nnx"], cfg["nny"], cfg["nnz"], cfg["aphi"], cfg["beta"], cfg["u_c"],
+                          cfg["rms"], cfg["kmax"], cfg["slope"], cfg["seed"])
+    with Channel(cfg["nnx"], cfg["nny"], cfg["nnz"], cfg["aphi"], cfg["beta"], cfg["dt"], cfg["re"],
+                 cfg["re_p"], precision=precision) as ch:
+        ch.set_timing(True)
+        ch.initial(*fields)
+        ch.step(steps)
+    print(json.dumps({"launch_probe_steps": steps, "precision": precision}), flush=True)
     return 0
 
 
@@ -353,6 +370,8 @@ def main(argv=None):
                     help="run the 24-channel batched-ensemble workload instead (its own JSON line)")
     ap.add_argument("--copy-probe", action="store_true",
                     help="run only a 1 GiB device copy (counter calibration)")
+    ap.add_argument("--launch-probe", action="store_true",
+                    help="run only --steps steps of one --precision, every launch alone (counters per launch)")
     ap.add_argument("--verbose", action="store_true")
     a = ap.parse_args(argv)
     if a.copy_probe:
@@ -367,6 +386,8 @@ def main(argv=None):
     from channel_flow_amd import ic
 
     cfg = dict(ic.CONFIGS[a.config])
+    if a.launch_probe:
+        return launch_probe(cfg, "mixed" if a.precision == "both" else a.precision, a.steps)
     d = dims(cfg)
     log = (lambda *x: print(*x, file=sys.stderr, flush=True)) if a.verbose else (lambda *x: None)
     t0 = time.perf_counter()
