@@ -3,8 +3,8 @@
 // A plain hipMemcpy of pageable memory moves about 10 GB/s here: one thread
 // copies through the runtime's staging buffer, and a freshly allocated
 // destination takes its page faults in that copy.  Here several threads move
-// chunks, each through two pinned buffers of its own and on a stream of its own:
-// while one buffer's transfer is in flight the other is copied to or from the
+// chunks, each through two pinned buffers of its own and on a stream of its own
+// (the first two on the context's, which are idle then): while one buffer's transfer is in flight the other is copied to or from the
 // caller's array, so the copies and page faults run in parallel with the link.
 // Bound: the link (and, for a new destination, the page faults).  A state record
 // at 256x193x256 (0.81 GB): read 61 -> 12.7 ms, loaded 23 -> 11.2 ms; one physical
@@ -13,7 +13,10 @@
 //
 // The pinned buffers and streams are kept in a process-wide pool per device, at
 // most kMaxLanes lanes (2 x kChunk bytes each); a lane belongs to one call at a
-// time, and the pool is freed when the last context is destroyed.  A copy itself
+// time, and the pool is freed when the last context is destroyed.  A stream costs
+// 0.5 ms to make and 0.6 to destroy, the buffers 0.2 and 0.1: with a stream in every
+// lane a program that makes a context, loads, reads and destroys it paid up to 2 ms
+// at the first copy and 4 at the end.  A copy itself
 // allocates nothing but its threads: without memory it has fewer lanes or threads,
 // or goes the plain way, and never throws.
 #include <algorithm>
@@ -31,10 +34,14 @@ namespace {
 
 constexpr size_t kChunk = size_t(2) << 20;
 constexpr int kMaxLanes = 6;
-constexpr size_t kMinBytes = size_t(4) << 20;  // smaller transfers go the plain way
+// Smaller transfers go the plain way.  Loading, which meets no page faults, is as
+// fast so up to about 40 MB: records of 13 MB 0.6 ms, through lanes 1.0; 43 MB 1.6 / 1.1;
+// two fields into a new context, which makes its lanes then, 14 MB 0.7 / 1.3, 34 MB
+// 1.6 / 2.8, 95 MB 6.4 / 5.1.
+constexpr size_t kMinRead = size_t(4) << 20, kMinLoad = size_t(40) << 20;
 
 struct Lane {
-  hipStream_t stream = nullptr;
+  hipStream_t stream = nullptr;  // made for a call's third lane on
   void* pin[2] = {nullptr, nullptr};
   hipEvent_t done[2] = {nullptr, nullptr};
 };
@@ -48,7 +55,7 @@ void lane_free(Lane& l) {
 }
 
 hipError_t lane_make(Lane& l) {
-  hipError_t e = hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking);
+  hipError_t e = hipSuccess;
   for (int b = 0; b < 2 && e == hipSuccess; ++b) {
     e = hipHostMalloc(&l.pin[b], kChunk, hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&l.done[b], hipEventDisableTiming);
@@ -76,7 +83,16 @@ struct Lanes {
   explicit Lanes(int dev) : device(dev) {}
   Lanes(const Lanes&) = delete;
 
-  // up to `want` (none if all are taken or cannot be made)
+  // An idle lane, with or without a stream of its own as wanted where there is one.
+  static Lane pick(DeviceLanes& d, bool stream) {
+    int k = d.nidle - 1;
+    while (k > 0 && (d.idle[k].stream != nullptr) != stream) --k;
+    std::swap(d.idle[k], d.idle[--d.nidle]);
+    return d.idle[d.nidle];
+  }
+
+  // up to `want` (none if all are taken or cannot be made), from the third on with
+  // streams of their own
   void take(int want) {
     std::lock_guard<std::mutex> lock(g_pool.mu);
     DeviceLanes* d = nullptr;
@@ -86,18 +102,25 @@ struct Lanes {
       return;
     }
     while (n < want) {
-      if (d->nidle > 0) {
-        lane[n++] = d->idle[--d->nidle];
-        continue;
-      }
-      if (d->made >= kMaxLanes) break;
+      const bool own = n >= 2;
       Lane l;
-      if (lane_make(l) != hipSuccess) {
-        lane_free(l);
+      if (d->nidle > 0) {
+        l = pick(*d, own);
+      } else {
+        if (d->made >= kMaxLanes) break;
+        if (lane_make(l) != hipSuccess) {
+          lane_free(l);
+          (void)hipGetLastError();
+          break;
+        }
+        ++d->made;
+      }
+      if (own && !l.stream && hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking) != hipSuccess) {
+        l.stream = nullptr;
         (void)hipGetLastError();
+        d->idle[d->nidle++] = l;
         break;
       }
-      ++d->made;
       lane[n++] = l;
     }
   }
@@ -135,7 +158,7 @@ struct Jobs {
   }
 };
 
-hipError_t run_lane(Lane& l, const Jobs& jobs, std::atomic<size_t>& next, bool to_host) {
+hipError_t run_lane(Lane& l, hipStream_t stream, const Jobs& jobs, std::atomic<size_t>& next, bool to_host) {
   Job held[2] = {};  // bytes: of the transfer in flight into the buffer, or 0
   bool used[2] = {false, false};
   hipError_t e = hipSuccess;
@@ -149,8 +172,8 @@ hipError_t run_lane(Lane& l, const Jobs& jobs, std::atomic<size_t>& next, bool t
   Job j;
   for (; e == hipSuccess && jobs.get(next++, j); b ^= 1) {
     if (to_host) {
-      e = hipMemcpyAsync(l.pin[b], j.dev, j.bytes, hipMemcpyDeviceToHost, l.stream);
-      if (e == hipSuccess) e = hipEventRecord(l.done[b], l.stream);
+      e = hipMemcpyAsync(l.pin[b], j.dev, j.bytes, hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipEventRecord(l.done[b], stream);
       if (e != hipSuccess) break;
       held[b] = j;
       finish(b ^ 1);
@@ -158,13 +181,13 @@ hipError_t run_lane(Lane& l, const Jobs& jobs, std::atomic<size_t>& next, bool t
       if (used[b]) e = hipEventSynchronize(l.done[b]);
       if (e != hipSuccess) break;
       std::memcpy(l.pin[b], j.host, j.bytes);
-      e = hipMemcpyAsync(j.dev, l.pin[b], j.bytes, hipMemcpyHostToDevice, l.stream);
-      if (e == hipSuccess) e = hipEventRecord(l.done[b], l.stream);
+      e = hipMemcpyAsync(j.dev, l.pin[b], j.bytes, hipMemcpyHostToDevice, stream);
+      if (e == hipSuccess) e = hipEventRecord(l.done[b], stream);
       used[b] = true;
     }
   }
   if (e == hipSuccess) finish(b ^ 1);
-  const hipError_t s = hipStreamSynchronize(l.stream);  // the buffers are free again
+  const hipError_t s = hipStreamSynchronize(stream);  // the buffers are free again
   return e != hipSuccess ? e : s;
 }
 
@@ -190,7 +213,7 @@ hipError_t copy_arrays(Ctx& c, const HostArray* arrays, int count, bool to_host)
   for (int k = 0; k < count; ++k)
     if (arrays[k].bytes >= kChunk) total += arrays[k].bytes;
   Lanes lanes(c.device);
-  if (total >= kMinBytes) lanes.take((int)std::min<size_t>(kMaxLanes, total / (4 * kChunk) + 1));
+  if (total >= (to_host ? kMinRead : kMinLoad)) lanes.take((int)std::min<size_t>(kMaxLanes, total / (4 * kChunk) + 1));
   for (int k = 0; k < count; ++k) {
     const HostArray& a = arrays[k];
     if (lanes.n > 0 && a.bytes >= kChunk) continue;
@@ -198,8 +221,9 @@ hipError_t copy_arrays(Ctx& c, const HostArray* arrays, int count, bool to_host)
                                  : hipMemcpyAsync(a.dev, a.host, a.bytes, hipMemcpyHostToDevice, c.stream);
     if (e != hipSuccess) return e;
   }
-  // the lanes' streams start after the work queued on the context's stream, and
-  // what is queued there next starts after them
+  // the lanes' streams start after the work queued on the context's streams (the
+  // side stream's is joined to the first's), and what is queued there next starts
+  // after them
   hipError_t e = hipStreamSynchronize(c.stream);
   if (e != hipSuccess || lanes.n == 0) return e;
   const Jobs jobs{arrays, count};
@@ -207,7 +231,8 @@ hipError_t copy_arrays(Ctx& c, const HostArray* arrays, int count, bool to_host)
   hipError_t err[kMaxLanes] = {};
   auto lane = [&](int i) {
     if (i) err[i] = hipSetDevice(c.device);  // the caller's thread has it current
-    if (err[i] == hipSuccess) err[i] = run_lane(lanes.lane[i], jobs, next, to_host);
+    hipStream_t stream = i == 0 ? c.stream : i == 1 ? c.side : lanes.lane[i].stream;
+    if (err[i] == hipSuccess) err[i] = run_lane(lanes.lane[i], stream, jobs, next, to_host);
   };
   std::thread threads[kMaxLanes];
   for (int i = 1; i < lanes.n; ++i) {

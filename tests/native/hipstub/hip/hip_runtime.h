@@ -20,7 +20,8 @@ constexpr unsigned hipStreamNonBlocking = 1, hipEventDisableTiming = 2, hipHostM
 
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
-inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = std::malloc(1), hipSuccess; }
+inline int streams_made = 0;
+inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return ++streams_made, *s = std::malloc(1), hipSuccess; }
 inline hipError_t hipStreamDestroy(hipStream_t s) { return std::free(s), hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = std::malloc(1), hipSuccess; }

@@ -35,8 +35,21 @@ static int copy(Ctx& c, std::vector<char>* dev, std::vector<char>* host, bool to
   return (int)copy_arrays(c, a, 3, to_host);
 }
 
+// One array of a few chunks through a pool of its own: the streams made for it.
+static int streams_for(Ctx& c, std::size_t bytes) {
+  std::vector<char> from(bytes, 5), to(bytes);
+  const HostArray a[] = {{from.data(), to.data(), bytes}};
+  const int before = streams_made;
+  hostcopy_retain();
+  const bool ok = copy_arrays(c, a, 1, true) == hipSuccess && copy_arrays(c, a, 1, true) == hipSuccess && to == from;
+  hostcopy_release();
+  return ok ? streams_made - before : -1;
+}
+
 int main() {
   Ctx c;
+  std::printf("streams %d %d %d\n", streams_for(c, std::size_t(5) << 20), streams_for(c, std::size_t(12) << 20),
+              streams_for(c, std::size_t(100) << 20));
   std::vector<char> from[3], to[3];
   for (int i = 0; i < 3; ++i) {
     from[i].resize(kBytes[i]);

@@ -1,7 +1,7 @@
 """Copies between device and host arrays (csrc/hostcopy.hip, compiled with g++ over
-host stand-ins for the HIP calls) without memory: whichever allocation fails, the
+host stand-ins for the HIP calls): without memory, whichever allocation fails, the
 start of a helper thread among them, the copy is whole, nothing is thrown, and the
-pool's lanes serve the next copy."""
+pool's lanes serve the next copy; copies of one or two lanes make no streams."""
 import os
 import shutil
 import subprocess
@@ -11,7 +11,7 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def test_failed_allocations(tmp_path):
+def test_copies(tmp_path):
     cxx = shutil.which("g++")
     if cxx is None:
         pytest.skip("no g++")
@@ -21,6 +21,9 @@ def test_failed_allocations(tmp_path):
                     os.path.join(native, "hostcopy_harness.cpp"), "-o", exe], check=True, capture_output=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.returncode, r.stdout[-500:], r.stderr[-500:])
-    rows = [tuple(map(int, line.split())) for line in r.stdout.splitlines()]
+    head, *lines = r.stdout.splitlines()
+    # 5 MB: one lane; 12 MB: two, on the context's own streams; 100 MB: all six
+    assert head == "streams 0 0 4", head
+    rows = [tuple(map(int, line.split())) for line in lines]
     assert {d for d, _, _ in rows} == {0, 1} and max(n for _, n, _ in rows) >= 5, rows
     assert all(lanes == 6 for _, _, lanes in rows), rows
