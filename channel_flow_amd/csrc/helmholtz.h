@@ -29,6 +29,7 @@
 #pragma once
 #include <cmath>
 #include <initializer_list>
+#include <thread>
 #include <vector>
 
 #include "eig.h"
@@ -77,33 +78,52 @@ inline void half_points(int N, int par, HelmholtzHalf& h) {
 }
 
 // a b (m x m) in extended precision: dot products, four columns at a time (the
-// accumulators stay in registers; x87 stores are what the row form waits for).
+// accumulators stay in registers; x87 stores are what the row form waits for), the
+// rows of large ones by several threads (m = 96, the decomposition's products are
+// 7 of its 13 ms in one).
 inline LMat lmul(const LMat& a, const LMat& b, int m) {
   LMat bt((size_t)m * m), c((size_t)m * m);
   for (int i = 0; i < m; ++i)
     for (int j = 0; j < m; ++j) bt[(size_t)j * m + i] = b[(size_t)i * m + j];
-  for (int i = 0; i < m; ++i) {
-    const LD* x = &a[(size_t)i * m];
-    int j = 0;
-    for (; j + 4 <= m; j += 4) {
-      const LD *y0 = &bt[(size_t)j * m], *y1 = y0 + m, *y2 = y1 + m, *y3 = y2 + m;
-      LD s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-      for (int k = 0; k < m; ++k) {
-        const LD f = x[k];
-        s0 += f * y0[k];
-        s1 += f * y1[k];
-        s2 += f * y2[k];
-        s3 += f * y3[k];
+  auto rows = [&](int i0, int i1) {
+    for (int i = i0; i < i1; ++i) {
+      const LD* x = &a[(size_t)i * m];
+      int j = 0;
+      for (; j + 4 <= m; j += 4) {
+        const LD *y0 = &bt[(size_t)j * m], *y1 = y0 + m, *y2 = y1 + m, *y3 = y2 + m;
+        LD s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+        for (int k = 0; k < m; ++k) {
+          const LD f = x[k];
+          s0 += f * y0[k];
+          s1 += f * y1[k];
+          s2 += f * y2[k];
+          s3 += f * y3[k];
+        }
+        LD* o = &c[(size_t)i * m + j];
+        o[0] = s0; o[1] = s1; o[2] = s2; o[3] = s3;
       }
-      LD* o = &c[(size_t)i * m + j];
-      o[0] = s0; o[1] = s1; o[2] = s2; o[3] = s3;
+      for (; j < m; ++j) {
+        LD s0 = 0;
+        for (int k = 0; k < m; ++k) s0 += x[k] * bt[(size_t)j * m + k];
+        c[(size_t)i * m + j] = s0;
+      }
     }
-    for (; j < m; ++j) {
-      LD s0 = 0;
-      for (int k = 0; k < m; ++k) s0 += x[k] * bt[(size_t)j * m + k];
-      c[(size_t)i * m + j] = s0;
+  };
+  constexpr int kThreads = 4;
+  std::thread others[kThreads - 1];
+  int done = 0;  // rows handed out
+  if (m >= 48)
+    for (std::thread& t : others) {
+      try {
+        t = std::thread(rows, done, done + m / kThreads);
+      } catch (...) {
+        break;  // the rest of the rows is done here
+      }
+      done += m / kThreads;
     }
-  }
+  rows(done, m);
+  for (std::thread& t : others)
+    if (t.joinable()) t.join();
   return c;
 }
 
