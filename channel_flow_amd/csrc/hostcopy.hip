@@ -74,7 +74,7 @@ struct Pool {
   std::map<int, DeviceLanes> devices;
 } g_pool;
 
-// Lanes of the current device for one call, given back at its end.
+// Lanes of a context's device for one call, given back at its end.
 struct Lanes {
   Lane lane[kMaxLanes];
   int n = 0;
@@ -92,8 +92,18 @@ struct Lanes {
   }
 
   // up to `want` (none if all are taken or cannot be made), from the third on with
-  // streams of their own
+  // streams of their own; made on the context's device, whichever is current
   void take(int want) {
+    int current = device;
+    if (hipGetDevice(&current) != hipSuccess || (current != device && hipSetDevice(device) != hipSuccess)) {
+      (void)hipGetLastError();
+      return;
+    }
+    take_here(want);
+    if (current != device) (void)hipSetDevice(current);
+  }
+
+  void take_here(int want) {
     std::lock_guard<std::mutex> lock(g_pool.mu);
     DeviceLanes* d = nullptr;
     try {
@@ -230,7 +240,7 @@ hipError_t copy_arrays(Ctx& c, const HostArray* arrays, int count, bool to_host)
   std::atomic<size_t> next{0};
   hipError_t err[kMaxLanes] = {};
   auto lane = [&](int i) {
-    if (i) err[i] = hipSetDevice(c.device);  // the caller's thread has it current
+    if (i) err[i] = hipSetDevice(c.device);  // a helper thread of this call
     hipStream_t stream = i == 0 ? c.stream : i == 1 ? c.side : lanes.lane[i].stream;
     if (err[i] == hipSuccess) err[i] = run_lane(lanes.lane[i], stream, jobs, next, to_host);
   };

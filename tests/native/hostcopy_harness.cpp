@@ -48,6 +48,12 @@ static int streams_for(Ctx& c, std::size_t bytes) {
 
 int main() {
   Ctx c;
+  // a context of device 1, called with device 0 current
+  (void)hipSetDevice(1);
+  c.device = 1;
+  (void)hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
+  (void)hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking);
+  (void)hipSetDevice(0);
   std::printf("streams %d %d %d\n", streams_for(c, std::size_t(5) << 20), streams_for(c, std::size_t(12) << 20),
               streams_for(c, std::size_t(100) << 20));
   std::vector<char> from[3], to[3];
@@ -67,9 +73,9 @@ int main() {
         if (!again) hit = left.load() < 0;
         left = -1;
         for (int i = 0; i < 3; ++i)
-          if (rc || to[i] != from[i]) return std::printf("%ld %d array %d: rc %d\n", n, again, i, rc), 1;
+          if (rc || to[i] != from[i] || current_device) return std::printf("%ld %d array %d: rc %d\n", n, again, i, rc), 1;
         if (again) {
-          const int lanes = g_pool.devices[0].nidle;
+          const int lanes = g_pool.devices[1].nidle;
           std::printf("%d %ld %d\n", to_host, n, lanes);
           std::fflush(stdout);
         }

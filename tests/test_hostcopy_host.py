@@ -1,7 +1,8 @@
 """Copies between device and host arrays (csrc/hostcopy.hip, compiled with g++ over
 host stand-ins for the HIP calls): without memory, whichever allocation fails, the
 start of a helper thread among them, the copy is whole, nothing is thrown, and the
-pool's lanes serve the next copy; copies of one or two lanes make no streams."""
+pool's lanes serve the next copy; copies of one or two lanes make no streams; and a
+context of another device than the caller's current one copies as well."""
 import os
 import shutil
 import subprocess
