@@ -1011,8 +1011,11 @@ int chf_set_timing(void* ctx, int on) {
   if (!ctx) return -1;
   Ctx* c = static_cast<Ctx*>(ctx);
   CHF_TRY(hipStreamSynchronize(c->stream));
-  if (on && c->zplanes < c->d.Py)
+  if (on && c->zplanes < c->d.Py) {
+    const DeviceScope here(c->device);
+    if (!here.ok()) return fail(c, "chf_set_timing: the context's device cannot be made current");
     if (const int rc = alloc_padded(c, c->d.Py)) return rc;
+  }
   c->timing = on != 0;
   c->marks.clear();
   c->pool_next = 0;
@@ -1027,6 +1030,8 @@ namespace {
 // on first use (they are not part of the timestep).
 int ensure_physical(Ctx* c) {
   const Dims& d = c->d;
+  const DeviceScope here(c->device);
+  if (!here.ok()) return fail(c, "chf_physical: the context's device cannot be made current");
   if (!c->phys_c[0]) CHF_TRY(dalloc(c, &c->phys_c[0], (size_t)d.Ny * d.ncol));
   if (!c->phys_r[0]) CHF_TRY(dalloc(c, &c->phys_r[0], (size_t)d.Ny * d.Mz * 2 * d.Mx));
   return 0;
@@ -1034,6 +1039,8 @@ int ensure_physical(Ctx* c) {
 
 int ensure_statistics(Ctx* c) {
   const Dims& d = c->d;
+  const DeviceScope here(c->device);
+  if (!here.ok()) return fail(c, "chf_statistics: the context's device cannot be made current");
   for (auto& p : c->phys_c)
     if (!p) CHF_TRY(dalloc(c, &p, (size_t)d.Ny * d.ncol));
   if (stats_in_lines(*c)) {

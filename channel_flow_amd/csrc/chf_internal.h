@@ -213,6 +213,25 @@ bool fft_length_ok(int L);
 
 extern const char* const kKernelNames[K_COUNT];
 
+// Makes a device current for a scope, for what is allocated or made in it.
+class DeviceScope {
+ public:
+  explicit DeviceScope(int device) {
+    ok_ = hipGetDevice(&before_) == hipSuccess && (before_ == device || hipSetDevice(device) == hipSuccess);
+    back_ = ok_ && before_ != device;
+    if (!ok_) (void)hipGetLastError();
+  }
+  ~DeviceScope() {
+    if (back_) (void)hipSetDevice(before_);
+  }
+  DeviceScope(const DeviceScope&) = delete;
+  bool ok() const { return ok_; }
+
+ private:
+  int before_ = 0;
+  bool ok_ = false, back_ = false;
+};
+
 // hostcopy.hip: device arrays to or from the caller's pageable arrays; returns
 // when the copies are done.  The contexts alive hold the staging pool.
 struct HostArray {

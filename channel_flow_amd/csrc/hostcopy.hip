@@ -94,16 +94,8 @@ struct Lanes {
   // up to `want` (none if all are taken or cannot be made), from the third on with
   // streams of their own; made on the context's device, whichever is current
   void take(int want) {
-    int current = device;
-    if (hipGetDevice(&current) != hipSuccess || (current != device && hipSetDevice(device) != hipSuccess)) {
-      (void)hipGetLastError();
-      return;
-    }
-    take_here(want);
-    if (current != device) (void)hipSetDevice(current);
-  }
-
-  void take_here(int want) {
+    const DeviceScope here(device);
+    if (!here.ok()) return;
     std::lock_guard<std::mutex> lock(g_pool.mu);
     DeviceLanes* d = nullptr;
     try {
