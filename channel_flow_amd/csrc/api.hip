@@ -794,7 +794,8 @@ int solve(Ctx* c) {
     CHF_TRY(timed(c, K_SOLVE, [&] { return launch_solve(*c); }));
   } else if (!c->timing) {
     // both equations in each launch (32x33x32 step 60 -> 51 us, 128x129x128 552 ->
-    // 540, 256x193x256 mixed 1866 -> 1844 against one launch each, on two streams there)
+    // 540, 256x193x256 mixed 1866 -> 1844 against one launch each, on two streams
+    // there); the right-hand sides as cos-table products are a launch each
     CHF_TRY(launch_rhs(*c, 0, 2));
     CHF_TRY(launch_hsolve(*c, 0, 2));
   } else {  // every launch alone, so that each time is its own

@@ -89,7 +89,8 @@ struct Ctx {
   bool holds_pool = false;  // counted among the staging pool's users
   hipStream_t stream = nullptr;
   // second stream of the context (default priority): every other slab of the
-  // padded planes runs on it; the pair of events forks and joins it
+  // padded planes runs on it, and a lane of the host copies; the pair of events
+  // forks and joins it
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   // padded planes in slabs (kSlabsFrom); off for ensemble members, whose steps
@@ -117,9 +118,9 @@ struct Ctx {
   double2* cl3[2] = {nullptr, nullptr};  // mean L_z(0,0) point values [Ny]
   double2 *au0 = nullptr, *w0 = nullptr;  // mean U, W coefficients [Ny]
   int hcur = 0;
-  // h^n's point values hv[hcur], hg[hcur] are not yet formed: hvc, hgc hold
-  // h^n's coefficients and the next solve's right-hand-side kernels form them
-  // (FFT transforms only)
+  // h^n's point values hv[hcur], hg[hcur] are pending: hvc, hgc hold h^n's
+  // coefficients and the next solve's right-hand-side kernels form them (FFT
+  // transforms only; chf_get_state forms them too and leaves them pending)
   bool hdefer = false;
   // nonlinear work
   double2* Y[6] = {};     // [Py][yplane: Mz Mx, padding]   wall-normal points, Fourier modes

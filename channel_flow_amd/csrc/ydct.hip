@@ -467,9 +467,10 @@ constexpr bool single_load() {
   return sizeof(V) == 8 || ANA;
 }
 
-// The splits A1 x A2 (A2 even) of the 2N-point transform: every even degree from
-// 32 to 256 whose 2N has factors up to 24 of this form.  Other degrees (and column
-// counts that are no multiple of 16) take the cos-table products.  The FFT was the
+// The splits A1 x A2 (A2 even) of the 2N-point transform, for even degrees from 32
+// to 256.  Other degrees (N = 36, 54, 108 and 162 among them, whose splits would be
+// 8 x 9, 9 x 12, 12 x 18 and 18 x 18) and column counts that are no multiple of 16
+// take the cos-table products.  The FFT was the
 // faster form at each degree, step time in us, FFT / products, FP64 and mixed:
 // 32x32 N = 40 55 / 65, 55 / 58, N = 100 83 / 100, 82 / 91, N = 240 141 / 210,
 // 129 / 172; 128x128 N = 40 190 / 195, 129 / 140, N = 90 393 / 399, 264 / 266,

@@ -80,8 +80,10 @@ const char* chf_last_error(void* ctx);
 int chf_set_state(void* ctx, const chf_state* st);
 /* Device -> host copy of the pre-solve state (replaces output, PF:2460-2504).
  * With the FFT transforms, first forms h^n's point values when the last
- * chf_nonlinear left them to the next solve (the values that solve would
- * form, bit for bit). */
+ * chf_nonlinear left them to the next solve (the values that solve forms, bit
+ * for bit).  Like every call here that moves arrays to or from the host, it may
+ * copy through up to five helper threads and a pool of pinned memory, at most
+ * 24 MB per GPU, which is freed with the last context. */
 int chf_get_state(void* ctx, const chf_state* st);
 
 /* Cold start (replaces initial(isign=-1) after input, PF:1932-1946): from v,
