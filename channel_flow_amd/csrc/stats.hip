@@ -135,7 +135,10 @@ constexpr int kStatsThreads = 256;
 // Plane statistics without storing the physical fields: a block transforms
 // some of a plane's lines of u, v, w, keeps them in registers and sums the
 // products about the plane means and the extrema.  The mean of a field over the
-// plane is the mean over the span of its lines' (real) kx = 0 modes.
+// plane is the mean over the span of its lines' (real) kx = 0 modes, and NaN where a
+// value of the plane is not finite, as a sum over the values is: the squares' sum is
+// NaN where a value is (no term of it is negative), and an infinity is the largest
+// value (a test of every value costs 2%).
 template <int N1, int N2>
 __global__ __launch_bounds__(kStatsThreads, 2) void k_line_stats(LineArgs a) {
   using Ge = LineGeo<N1, N2>;
@@ -190,6 +193,7 @@ __global__ __launch_bounds__(kStatsThreads, 2) void k_line_stats(LineArgs a) {
   for (int i = 0; i < 6; ++i) {
     const double v = block_sum(acc[i], red);
     if (threadIdx.x == 0) p[3 + i] = v;
+    if (i < 3 && v != v) mean[i] = v;
   }
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
@@ -202,33 +206,24 @@ __global__ __launch_bounds__(kStatsThreads, 2) void k_line_stats(LineArgs a) {
     if (threadIdx.x == 0) {
       for (int w = 1; w < (int)(blockDim.x >> 6); ++w) v = fmax(v, red[w]);
       p[9 + i] = v;
-      p[i] = mean[i];
+      p[i] = isinf(v) ? v - v : mean[i];
     }
   }
 }
 
-// The splits' partial results [Ny][splits][12] to out [12][Ny].  A mean, which the
-// lines' kx = 0 modes give, is NaN where a value of its plane is not finite, as a sum
-// over the values is: the squares' sum is NaN where a value is (no term of it is
-// negative), and an infinity is the largest value.
+// The splits' partial results [Ny][splits][12] to out [12][Ny]; no branch in a loop,
+// so that its loads are in flight together.
 __global__ __launch_bounds__(256) void k_stats_final(const double* __restrict__ part, int splits, int Ny, double coef,
                                                      double* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= 12 * Ny) return;
   const int q = i / Ny, k = i - q * Ny;
-  const double* p = part + (long)k * splits * 12;
-  double v = p[q];
-  if (q < 3) {
-    bool finite = true;  // no branch in the loop: its loads are in flight together
+  const double* p = part + (long)k * splits * 12 + q;
+  double v = p[0];
 #pragma unroll 8
-    for (int s = 0; s < splits; ++s) {
-      const double sq = p[12 * s + 3 + q], big = p[12 * s + 9 + q];
-      finite = finite & (sq == sq) & (big < __builtin_inf());
-    }
-    if (!finite) v = __builtin_nan("");
-  } else {
-#pragma unroll 8
-    for (int s = 1; s < splits; ++s) v = q < 9 ? v + p[12 * s + q] : fmax(v, p[12 * s + q]);
+  for (int s = 1; s < splits; ++s) {
+    const double x = p[12 * s];
+    v = q < 3 ? (x == x ? v : x) : q < 9 ? v + x : fmax(v, x);  // the same mean in every split, but for NaN
   }
   out[i] = (q >= 3 && q < 9) ? v * coef : v;
 }
