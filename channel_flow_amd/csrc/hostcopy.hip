@@ -35,10 +35,12 @@ namespace {
 constexpr size_t kChunk = size_t(2) << 20;
 constexpr int kMaxLanes = 6;
 // Smaller transfers go the plain way.  Loading, which meets no page faults, is as
-// fast so up to about 40 MB: records of 13 MB 0.6 ms, through lanes 1.0; 43 MB 1.6 / 1.1;
-// two fields into a new context, which makes its lanes then, 14 MB 0.7 / 1.3, 34 MB
-// 1.6 / 2.8, 95 MB 6.4 / 5.1.
-constexpr size_t kMinRead = size_t(4) << 20, kMinLoad = size_t(40) << 20;
+// fast so up to about 40 MB while one context is alive: records of 13 MB 0.6 ms, through
+// lanes 1.0; 43 MB 1.6 / 1.1; two fields into a new context, which makes its lanes
+// then, 14 MB 0.7 / 1.3, 34 MB 1.6 / 2.8, 95 MB 6.4 / 5.1.  With several contexts the
+// runtime's copy is slower: 14 MB into each of two 0.75, of three 2.2, of sixteen 4.6 ms,
+// through lanes 1.2, 1.1, 0.7 (an ensemble of 24 loaded 93 / 19).
+constexpr size_t kMinBytes = size_t(4) << 20, kMinLoadAlone = size_t(40) << 20;
 
 struct Lane {
   hipStream_t stream = nullptr;  // made for a call's third lane on
@@ -210,12 +212,18 @@ void hostcopy_release() {
   }
 }
 
+// Bytes from which a copy goes through lanes.
+static size_t lanes_from(bool to_host) {
+  std::lock_guard<std::mutex> lock(g_pool.mu);
+  return to_host || g_pool.users > 1 ? kMinBytes : kMinLoadAlone;
+}
+
 hipError_t copy_arrays(Ctx& c, const HostArray* arrays, int count, bool to_host) {
   size_t total = 0;
   for (int k = 0; k < count; ++k)
     if (arrays[k].bytes >= kChunk) total += arrays[k].bytes;
   Lanes lanes(c.device);
-  if (total >= (to_host ? kMinRead : kMinLoad)) lanes.take((int)std::min<size_t>(kMaxLanes, total / (4 * kChunk) + 1));
+  if (total >= lanes_from(to_host)) lanes.take((int)std::min<size_t>(kMaxLanes, total / (4 * kChunk) + 1));
   for (int k = 0; k < count; ++k) {
     const HostArray& a = arrays[k];
     if (lanes.n > 0 && a.bytes >= kChunk) continue;

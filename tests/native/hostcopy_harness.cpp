@@ -35,6 +35,17 @@ static int copy(Ctx& c, std::vector<char>* dev, std::vector<char>* host, bool to
   return (int)copy_arrays(c, a, 3, to_host);
 }
 
+// Lanes made for loading an array with one context alive, and with two.
+static int lanes_for_load(Ctx& c, std::size_t bytes, int contexts) {
+  std::vector<char> from(bytes, 7), to(bytes);
+  const HostArray a[] = {{to.data(), from.data(), bytes}};
+  for (int i = 0; i < contexts; ++i) hostcopy_retain();
+  const bool ok = copy_arrays(c, a, 1, false) == hipSuccess && to == from;
+  const int made = g_pool.devices[c.device].made;
+  for (int i = 0; i < contexts; ++i) hostcopy_release();
+  return ok ? made : -1;
+}
+
 // One array of a few chunks through a pool of its own: the streams made for it.
 static int streams_for(Ctx& c, std::size_t bytes) {
   std::vector<char> from(bytes, 5), to(bytes);
@@ -61,6 +72,8 @@ int main() {
     from[i].resize(kBytes[i]);
     for (std::size_t k = 0; k < kBytes[i]; ++k) from[i][k] = (char)(k * 31 + (k >> 11) + i);
   }
+  std::printf("lanes %d %d %d %d\n", lanes_for_load(c, std::size_t(3) << 20, 2), lanes_for_load(c, std::size_t(14) << 20, 1),
+              lanes_for_load(c, std::size_t(14) << 20, 2), lanes_for_load(c, std::size_t(50) << 20, 1));
   for (int to_host = 0; to_host < 2; ++to_host)
     for (long n = 0;; ++n) {
       hostcopy_retain();  // a fresh pool each time

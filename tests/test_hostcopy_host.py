@@ -22,9 +22,11 @@ def test_copies(tmp_path):
                     os.path.join(native, "hostcopy_harness.cpp"), "-o", exe], check=True, capture_output=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.returncode, r.stdout[-500:], r.stderr[-500:])
-    head, *lines = r.stdout.splitlines()
+    head, loads, *lines = r.stdout.splitlines()
     # 5 MB: one lane; 12 MB: two, on the context's own streams; 100 MB: all six
     assert head == "streams 0 0 4", head
+    # loads of 3 MB with two contexts alive, 14 MB with one and with two, 50 MB with one
+    assert loads == "lanes 0 0 2 6", loads
     rows = [tuple(map(int, line.split())) for line in lines]
     assert {d for d, _, _ in rows} == {0, 1} and max(n for _, n, _ in rows) >= 5, rows
     assert all(lanes == 6 for _, _, lanes in rows), rows
