@@ -80,7 +80,7 @@ inline void half_points(int N, int par, HelmholtzHalf& h) {
 // a b (m x m) in extended precision: dot products, four columns at a time (the
 // accumulators stay in registers; x87 stores are what the row form waits for), the
 // rows of large ones by several threads (m = 96, the decomposition's products are
-// 7 of its 13 ms in one).
+// 7 of its 13 ms in one; below 80 the threads cost what they save).
 inline LMat lmul(const LMat& a, const LMat& b, int m) {
   LMat bt((size_t)m * m), c((size_t)m * m);
   for (int i = 0; i < m; ++i)
@@ -112,7 +112,7 @@ inline LMat lmul(const LMat& a, const LMat& b, int m) {
   constexpr int kThreads = 4;
   std::thread others[kThreads - 1];
   int done = 0;  // rows handed out
-  if (m >= 48)
+  if (m >= 80)
     for (std::thread& t : others) {
       try {
         t = std::thread(rows, done, done + m / kThreads);
