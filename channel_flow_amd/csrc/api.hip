@@ -747,9 +747,10 @@ hipError_t physical_products(Ctx* c, V* const* Y, V* const* Z) {
     e = planes(y0, std::min(c->slab, d.Py - y0), s & 1 ? c->slab : 0);
   }
   c->stream = main;
-  if (e == hipSuccess) e = hipEventRecord(c->ev_join, c->side);
-  if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, c->ev_join, 0);
-  return e;
+  // joined after a failure too: slabs queued before it still run on the side stream
+  hipError_t j = hipEventRecord(c->ev_join, c->side);
+  if (j == hipSuccess) j = hipStreamWaitEvent(c->stream, c->ev_join, 0);
+  return e != hipSuccess ? e : j;
 }
 
 // With the FFT transforms h^n's point values are left to the next solve's
