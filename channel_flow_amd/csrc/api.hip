@@ -9,7 +9,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
 #include <type_traits>
 #include <utility>
@@ -219,7 +219,7 @@ int diagonalise(Ctx* c, const std::vector<double>& al, const std::vector<double>
   std::thread other;
   try {
     other = std::thread(half, 1);
-  } catch (const std::system_error&) {
+  } catch (...) {  // no thread to be had
     half(1);
   }
   half(0);
@@ -650,6 +650,17 @@ int build(Ctx* c, DegreeCache& cache) {
   return autotune(c);
 }
 
+// build() for the C entries: out of host memory (the operators' and the
+// decomposition's tables) is an error code there, not an exception.
+int build_context(Ctx* c, DegreeCache& cache) {
+  try {
+    return build(c, cache);
+  } catch (const std::bad_alloc&) {
+    c->err = "no memory";  // fits the string without an allocation
+    return (int)hipErrorOutOfMemory;
+  }
+}
+
 hipEvent_t next_event(Ctx* c) {
   if (c->pool_next == c->event_pool.size()) {
     hipEvent_t e;
@@ -859,7 +870,7 @@ int chf_create(const chf_params* prm, void** out) {
   Ctx* c = new Ctx();
   c->prm = *prm;
   DegreeCache cache;
-  int rc = build(c, cache);
+  int rc = build_context(c, cache);
   if (rc) {
     g_create_err = c->err;
     free_all(c);
@@ -1316,7 +1327,7 @@ int chf_ensemble_create(const chf_params* members, int n, void** out) {
     Ctx* c = new Ctx();
     c->prm = members[i];
     c->slabs = false;
-    const int rc = build(c, cache);
+    const int rc = build_context(c, cache);
     if (rc) {
       g_create_err = "member " + std::to_string(i) + ": " + c->err;
       free_all(c);
